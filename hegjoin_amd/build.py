@@ -24,7 +24,7 @@ CLI = os.path.join(PKG, "main")
 ARCH = os.environ.get("HEGJ_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["hegj_prims.hip", "hegj_index.hip", "hegj_join.hip", "hegj_util.hip",
-           "hegj_mfma.hip", "hegj_query.hip", "hegj_serve.cpp", "hegj_dataset.cpp", "hegj_ego.cpp",
+           "hegj_mfma.hip", "hegj_gram16.hip", "hegj_query.hip", "hegj_serve.cpp", "hegj_dataset.cpp", "hegj_ego.cpp",
            "hegj_scratch.hip", "hegj_api.cpp"]
 
 # -packed-fp32-ops: keep the compiler from emitting packed FP32 instructions.
@@ -34,7 +34,8 @@ HIPFLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Wall",
 # VGPRs (gfx950 MFMAs read and write either file): in the AGPR form every
 # reject test first copied each accumulator out with v_accvgpr_read (128 of
 # them per two chunks at 18-D; 501 -> 486 ms per launch without them).
-FILE_FLAGS = {"hegj_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+FILE_FLAGS = {"hegj_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "hegj_gram16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd):

@@ -206,10 +206,8 @@ struct hegj_index {
     uint64_t total_candidates = 0;
     double workload_ms = 0;
     bool have_workload = false;
-    // split-BF16 operands of the MFMA refine (lazily computed)
-    uint16_t *gb_A = nullptr, *gb_B = nullptr;
-    float *gb_w = nullptr;
-    uint32_t gb_kp = 0;
+    // operands of the MFMA refine (lazily computed)
+    hegj::GbOperands gb;
     double gb_ms = 0;
     // FP64 join plan + captured batch graph, reused while the options match
     hegj::GraphPlan *gplan = nullptr;
@@ -1081,12 +1079,10 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
 }
 
 hegj_status ensure_gb(hegj_index *h) {
-    if (h->gb_A) return HEGJ_OK;
-    const uint32_t kb = gb_kblocks(h->g.dim);
-    if (kb == 0) return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA refine for this dimensionality");
+    if (h->gb.A) return HEGJ_OK;
+    if (gb_kblocks(h->g.dim) == 0) return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA refine for this dimensionality");
     EventTimer t(h->stream);
-    HEGJ_TRY(gb_prepare(h->g, h->ix, kb * 32, &h->gb_A, &h->gb_B, &h->gb_w, h->stream));
-    h->gb_kp = kb * 32;
+    HEGJ_TRY(gb_prepare(h->g, h->ix, &h->gb, h->stream));
     h->gb_ms = t.stop();
     return HEGJ_OK;
 }
@@ -1101,16 +1097,22 @@ hegj_status selfjoin_mfma(hegj_index *h, const uint32_t *order, uint64_t result_
     HEGJ_TRY(ensure_gb(h));
     Scratch sc;
     uint2 *units = nullptr;
+    uint4 *units16 = nullptr;
     uint32_t U = 0;
     struct UnitsGuard {
         hipStream_t s;
         uint2 *&p;
+        uint4 *&q;
         ~UnitsGuard() {
             (void)hipStreamSynchronize(s);
             dev_free(p);
+            dev_free(q);
         }
-    } units_guard{s, units};
-    HEGJ_TRY(build_units(h->g, h->ix, gb_unit_queries(h->gb_kp / 32), order, &units, &U, s));
+    } units_guard{s, units, units16};
+    if (h->gb.f16)
+        HEGJ_TRY(g16_units(h->ix, order, h->d_work, h->total_candidates, &units16, &U, s));
+    else
+        HEGJ_TRY(build_units(h->g, h->ix, gb_unit_queries(h->gb.kp / 32), order, &units, &U, s));
     r->info.n_units = U;
     HIP_TRY(dev_malloc_n(&r->d_row_off, n));
     HIP_TRY(dev_malloc_n(&r->d_row_cnt, n));
@@ -1123,8 +1125,11 @@ hegj_status selfjoin_mfma(hegj_index *h, const uint32_t *order, uint64_t result_
     o.row_off = r->d_row_off;
     o.row_cnt = r->d_row_cnt;
     o.hash = d_hash;
-    HEGJ_TRY(gb_join(h->g, h->ix, units, U, h->gb_A, h->gb_B, h->gb_w, h->gb_kp, h->device, s, &o,
-                     result_capacity, parts));
+    // points that the cell-0 wrap silences are candidates only: then a pair's
+    // two directions are not both results
+    const bool mirror = h->gb.f16 && h->n_dead == 0;
+    HEGJ_TRY(gb_join(h->g, h->ix, h->gb.f16 ? (const void *)units16 : (const void *)units, U, h->gb, mirror,
+                     h->device, s, &o, result_capacity, parts));
     r->batches.push_back(o.buf);
     r->bases.push_back(0);
     unsigned long long hash = 0;
@@ -1247,9 +1252,9 @@ hegj_status hegj_index_free(hegj_index *h) {
     if (h->d_work) (void)hipFree(h->d_work);
     if (h->d_order) (void)hipFree(h->d_order);
     if (h->d_morton) (void)hipFree(h->d_morton);
-    if (h->gb_A) (void)hipFree(h->gb_A);
-    if (h->gb_B) (void)hipFree(h->gb_B);
-    if (h->gb_w) (void)hipFree(h->gb_w);
+    if (h->gb.A) (void)hipFree(h->gb.A);
+    if (h->gb.B) (void)hipFree(h->gb.B);
+    if (h->gb.w) (void)hipFree(h->gb.w);
     if (h->gplan) free_graph_plan(h->gplan);
     if (h->soa32) (void)hipFree(h->soa32);
     if (h->aos32) (void)hipFree(h->aos32);

@@ -224,19 +224,39 @@ struct GbOutput {
     uint64_t pairs = 0, band = 0, evals = 0;
     float kernel_ms = 0;
 };
-uint32_t gb_kblocks(uint32_t dim);        // K blocks of 32 for dim, 0 if unsupported
-uint32_t gb_unit_queries(uint32_t kb);    // queries per work unit of the MFMA kernel
+// Operands of one of the two MFMA joins (device arrays owned by the index).
+struct GbOperands {
+    uint16_t *A = nullptr, *B = nullptr;  // rows of kp 16-bit values
+    float *w = nullptr;                   // accept guards
+    uint32_t kp = 0;
+    bool f16 = false;                     // hegj_gram16.hip's, else split BF16
+    float trej = 0;                       // f16: reject above
+    double tacc = 0;                      // f16: accept at or below
+};
+uint32_t gb_kblocks(uint32_t dim);        // split BF16: K blocks of 32 for dim, 0 if unsupported
+uint32_t gb_unit_queries(uint32_t kb);    // queries per work unit of the split-BF16 kernel
 double gb_coefficient(uint32_t dim, uint32_t kp);
-hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, uint32_t kp, uint16_t **Av,
-                       uint16_t **Bv, float **w, hipStream_t s);
+// FP16 operands when they serve the data, else the split-BF16 ones.
+hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, GbOperands *ops, hipStream_t s);
+uint32_t g16_kblocks(uint32_t dim);
+hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mean, GbOperands *ops,
+                        hipStream_t s);
+hegj_status g16_units(const DevIndex &ix, const uint32_t *order, const uint32_t *work, uint64_t candidates,
+                      uint4 **units, uint32_t *n_units, hipStream_t s);
+hegj_status g16_occupancy(uint32_t kp, int device, uint32_t *blocks);
+struct GbArgs;
+hegj_status g16_launch(const GbArgs &a, uint32_t blocks, hipStream_t s);
+// Survivors of the launch -> pair list (guards, FP64 chain for the band).
+hegj_status g16_decide(const GbArgs &a, uint32_t blocks, hipStream_t s);
+// units: build_units' (uint2) for split BF16, g16_units' (uint4) for FP16.
+// mirror (FP16): evaluate each unordered pair once (every point is a query).
 // pair_cap: size (8-byte keys) of the first attempt's pair list, 0 for the
 // default of 48 per point; an attempt that overflows is repeated once with a
 // list sized from the count it reached.  parts: the units split into that
 // many contiguous ranges (1..kMaxParts), one queue per XCD.
-hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const uint2 *units, uint32_t n_units,
-                    const uint16_t *Av, const uint16_t *Bv, const float *w, uint32_t kp,
-                    int device, hipStream_t s, GbOutput *out, uint64_t pair_cap = 0,
-                    uint32_t parts = 1);
+hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, uint32_t n_units,
+                    const GbOperands &ops, bool mirror, int device, hipStream_t s, GbOutput *out,
+                    uint64_t pair_cap = 0, uint32_t parts = 1);
 
 // ---- query join against a resident index (hegj_query.hip) ----------------
 struct QueryGeom {

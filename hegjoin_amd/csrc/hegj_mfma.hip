@@ -1,5 +1,5 @@
 // hegj_mfma.hip -- split-BF16 MFMA distance tiles with a proven guard band
-// and an exact FP64 recheck: the refine of the join at high dimensionality.
+// and an exact FP64 recheck: a refine of the join at high dimensionality.
 //
 // At 18-D and 90-D the k = 6 grid leaves each query a large share of the
 // data as candidates (the reference evaluates ~1e12-3e12 FP64 distances,
@@ -26,10 +26,15 @@
 // FP64 chain.  The guard is twice the error bound (safety factor 2).  The
 // pair set is therefore identical to the FP64 one; the band count is
 // reported.
+//
+// This join serves the data that hegj_gram16.hip (one FP16 product per
+// dimension) cannot: a scale so wide that FP16 loses the bulk of the points,
+// or more than 124 dimensions.  Elsewhere it is 7 to 10 times slower (18-D 2M
+// 488 against 67.7 ms, 90-D 1M 701 against 67.6 ms).
 #include <algorithm>
 #include <cmath>
 
-#include "hegj_internal.h"
+#include "hegj_gb.h"
 
 namespace hegj {
 
@@ -46,39 +51,12 @@ constexpr int gb_waves(int kb) { return kb >= 6 ? 8 : 4; }
 constexpr int kGbChunk = 64;         // candidates per LDS chunk (4 col tiles)
 // 16-query row tiles per wave: 4 while the A fragments are small, 2 above
 constexpr int gb_rt(int kb) { return kb <= 4 ? 4 : 2; }
-constexpr int kGbBlk = 256;          // pair-list slots reserved per wave at a time
-constexpr uint64_t kSentinel = ~0ull;
-
-// Bit moves between float and uint32 that compile for host and device.
-__host__ __device__ __forceinline__ uint32_t f2u(float f) {
-    uint32_t u;
-    __builtin_memcpy(&u, &f, 4);
-    return u;
-}
-__host__ __device__ __forceinline__ float u2f(uint32_t u) {
-    float f;
-    __builtin_memcpy(&f, &u, 4);
-    return f;
-}
-
 __host__ __device__ __forceinline__ uint16_t bf16_bits_rne(float f) {
     uint32_t u = f2u(f);
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
 __host__ __device__ __forceinline__ float bf16_to_f(uint16_t b) { return u2f((uint32_t)b << 16); }
-
-// Neighbouring FP32 values (finite inputs), by bit arithmetic.
-__host__ __device__ __forceinline__ float f32_next_up(float f) {
-    uint32_t u = f2u(f);
-    if (f == 0.0f) return u2f(1u);
-    return u2f((u >> 31) ? u - 1 : u + 1);
-}
-__host__ __device__ __forceinline__ float f32_next_down(float f) {
-    uint32_t u = f2u(f);
-    if (f == 0.0f) return u2f(0x80000001u);
-    return u2f((u >> 31) ? u + 1 : u - 1);
-}
 
 // FP64 -> FP32 rounded toward -inf.
 __host__ __device__ __forceinline__ float f32_down(double v) {
@@ -174,8 +152,10 @@ __global__ __launch_bounds__(256) void k_dim_sums(const double *__restrict__ soa
     __shared__ double sh[256];
     for (uint32_t l = 0; l < dim; l++) {
         double s = 0;
-        for (uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (uint64_t)gridDim.x * 256)
-            s += soa[(uint64_t)l * n + p];
+        for (uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (uint64_t)gridDim.x * 256) {
+            const double v = soa[(uint64_t)l * n + p];
+            s += __builtin_isfinite(v) ? v : 0.0;  // the centre stays finite
+        }
         sh[threadIdx.x] = s;
         __syncthreads();
         for (int o = 128; o > 0; o >>= 1) {
@@ -187,76 +167,10 @@ __global__ __launch_bounds__(256) void k_dim_sums(const double *__restrict__ soa
     }
 }
 
-struct GbArgs {
-    GridGeom g;
-    DevIndex ix;
-    const uint2 *units;
-    uint32_t n_units;
-    uint32_t *queue_heads;        // [kMaxParts] units taken per range
-    uint32_t n_parts;             // unit ranges: range p is [part_end[p - 1], part_end[p])
-    uint32_t part_end[kMaxParts];
-    const uint16_t *Av;
-    const uint16_t *Bv;
-    const float *w;
-    uint32_t kp;
-    uint64_t *pairs;              // accepted keys (qpos << 32 | cpos)
-    uint64_t pair_cap;
-    unsigned long long *pair_cursor;
-    uint64_t *band;               // band keys
-    uint64_t band_cap;
-    unsigned long long *band_cursor;
-    unsigned long long *n_accept;
-    unsigned long long *n_band;
-    unsigned long long *evals;
-    uint32_t *overflow;
-};
-
-// Stencil-row list shared by the workgroup.
-struct GbRows {
-    uint32_t start[kMaxRows];
-    uint32_t off[kMaxRows + 1];
-};
-
 __device__ __forceinline__ uint32_t gb_cand_pos(const GbRows &rl, uint32_t nslots, uint32_t t,
                                                 uint32_t &slot) {
     while (slot + 1 < nslots && rl.off[slot + 1] <= t) slot++;
     return rl.start[slot] + (t - rl.off[slot]);
-}
-
-// Per-wave append buffer into a global key list (blocks of kGbBlk slots;
-// unused tails are filled with the sentinel, which sorts last).
-struct Appender {
-    uint64_t cur, end;
-};
-
-__device__ __forceinline__ void append_keys(uint64_t key, bool pred, Appender &ap,
-                                            uint64_t *list, uint64_t cap,
-                                            unsigned long long *cursor, uint32_t *overflow) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return;
-    const uint32_t k = (uint32_t)__popcll(m);
-    if (ap.cur + k > ap.end) {
-        // pad the rest of the block, then take a new one
-        for (uint64_t i = ap.cur + lane; i < ap.end; i += 64) list[i] = kSentinel;
-        uint64_t b = 0;
-        if (lane == 0) b = atomicAdd(cursor, (unsigned long long)kGbBlk);
-        b = wave_bcast_u64(b);
-        if (b + kGbBlk > cap) {
-            if (lane == 0) atomicOr(overflow, 1u);
-            ap.cur = ap.end = 0;
-            return;
-        }
-        ap.cur = b;
-        ap.end = b + kGbBlk;
-    }
-    if (pred) list[ap.cur + lanes_below(m)] = key;
-    ap.cur += k;
-}
-
-__device__ __forceinline__ void close_appender(Appender &ap, uint64_t *list) {
-    const int lane = threadIdx.x & 63;
-    for (uint64_t i = ap.cur + lane; i < ap.end; i += 64) list[i] = kSentinel;
 }
 
 template <int KB>
@@ -281,24 +195,10 @@ __global__ __launch_bounds__(64 * gb_waves(KB)) void k_gb_join(GbArgs a) {
     Appender apA{0, 0}, apB{0, 0};
     uint64_t my_acc = 0, my_band = 0, my_evals = 0;
 
-    // A workgroup takes units from its XCD's range first (neighbouring cells
-    // share candidates in that XCD's L2), then from the other ranges.
     const uint32_t part0 = xcc_id() % a.n_parts;
     uint32_t tried = 0;  // ranges found empty (thread 0's)
     while (true) {
-        if (tid == 0) {
-            uint32_t got = ~0u;
-            while (tried < a.n_parts) {
-                const uint32_t p = (part0 + tried) % a.n_parts;
-                const uint32_t k = (p ? a.part_end[p - 1] : 0u) + atomicAdd(&a.queue_heads[p], 1u);
-                if (k < a.part_end[p]) {
-                    got = k;
-                    break;
-                }
-                tried++;
-            }
-            sh_unit[0] = got;
-        }
+        if (tid == 0) sh_unit[0] = gb_next_unit(a.queue_heads, a.n_parts, a.part_end, part0, tried);
         __syncthreads();
         const uint32_t ui = sh_unit[0];
         if (ui >= a.n_units) break;
@@ -311,42 +211,9 @@ __global__ __launch_bounds__(64 * gb_waves(KB)) void k_gb_join(GbArgs a) {
 
         // stencil rows of the cell (wave 0), shared through LDS
         if (wid == 0) {
-            uint32_t c[kMaxK], lo[kMaxK], hi[kMaxK];
-            decode_cell(a.ix.cell_key[cell], a.g, c);
-            bool ok = true;
-            for (uint32_t j = 0; j < a.g.k; j++)
-                ok &= stencil_dim(c[j], a.g.nCells[j], a.g.emulate_cell0, &lo[j], &hi[j]);
-            uint32_t slots = 0, total = 0;
-            if (ok) {
-                const uint32_t nrows = pow3(a.g.k - 1);
-                for (uint32_t r0 = 0; r0 < nrows; r0 += 64) {
-                    const uint32_t r = r0 + lane;
-                    uint32_t pstart = 0, plen = 0;
-                    if (r < nrows) {
-                        uint32_t cf, cl;
-                        stencil_row(c, lo, hi, r, a.g, a.ix, &cf, &cl);
-                        if (cl > cf) {
-                            pstart = a.ix.cell_start[cf];
-                            plen = a.ix.cell_start[cl] - pstart;
-                        }
-                    }
-                    const uint64_t nz = __ballot(plen > 0);
-                    uint32_t x = plen;
-                    for (int o = 1; o < 64; o <<= 1) {
-                        uint32_t y = __shfl_up(x, o, 64);
-                        if (lane >= o) x += y;
-                    }
-                    if (plen > 0) {
-                        const uint32_t s = slots + lanes_below(nz);
-                        rl.start[s] = pstart;
-                        rl.off[s] = total + x - plen;
-                    }
-                    slots += (uint32_t)__popcll(nz);
-                    total += __shfl(x, 63, 64);
-                }
-            }
+            uint32_t slots, total, below;
+            gb_build_rows(a.g, a.ix, cell, 0, rl, &slots, &total, &below);
             if (lane == 0) {
-                rl.off[slots] = total;
                 sh_unit[1] = total;
                 sh_unit[2] = slots;
             }
@@ -651,8 +518,7 @@ double gb_coefficient(uint32_t dim, uint32_t kp) {
     return 1.01 * (2.05 * gamma + cll + 4.04 * eta + 2.0 * eta * eta + 4.04 * (dim + 2) * u64);
 }
 
-hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, uint32_t kp, uint16_t **Av,
-                       uint16_t **Bv, float **w, hipStream_t s) {
+hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, GbOperands *ops, hipStream_t s) {
     const uint32_t n = g.n, dim = g.dim;
     // centre = per-dim mean
     uint32_t blocks = std::min<uint32_t>(ceil_div(n, 256), 1024);
@@ -669,38 +535,63 @@ hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, uint32_t kp, uint1
         for (uint32_t l = 0; l < dim; l++) hm[l] += hp[(size_t)b * dim + l];
     for (uint32_t l = 0; l < dim; l++) hm[l] /= n;
     HIP_TRY(hipMemcpyAsync(mean, hm.data(), sizeof(double) * dim, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMalloc(Av, sizeof(uint16_t) * (size_t)n * kp));
-    HIP_TRY(hipMalloc(Bv, sizeof(uint16_t) * (size_t)n * kp));
-    HIP_TRY(hipMalloc(w, sizeof(float) * n));
+    HEGJ_TRY(g16_prepare(g, ix, mean, ops, s));
+    if (ops->A) return HEGJ_OK;
+    const uint32_t kb = gb_kblocks(dim), kp = kb * 32;
+    if (kb == 0) return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA refine for this dimensionality");
+    HIP_TRY(hipMalloc(&ops->A, sizeof(uint16_t) * (size_t)n * kp));
+    HIP_TRY(hipMalloc(&ops->B, sizeof(uint16_t) * (size_t)n * kp));
+    HIP_TRY(hipMalloc(&ops->w, sizeof(float) * n));
+    ops->kp = kp;
     k_gb_prepare<<<ceil_div(n, 256), 256, 0, s>>>(ix.soa, n, dim, kp, mean, gb_coefficient(dim, kp),
-                                                 *Av, *Bv, *w);
+                                                 ops->A, ops->B, ops->w);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
     return HEGJ_OK;
 }
 
-hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const uint2 *units, uint32_t n_units,
-                    const uint16_t *Av, const uint16_t *Bv, const float *w, uint32_t kp,
-                    int device, hipStream_t s, GbOutput *out, uint64_t pair_cap_first, uint32_t parts) {
-    const uint32_t kb = kp / 32;
-    uint32_t max_blocks = 0;
-    switch (kb) {
-        case 2: HEGJ_TRY(occ_gb<2>(device, &max_blocks)); break;
-        case 3: HEGJ_TRY(occ_gb<3>(device, &max_blocks)); break;
-        case 4: HEGJ_TRY(occ_gb<4>(device, &max_blocks)); break;
-        case 6: HEGJ_TRY(occ_gb<6>(device, &max_blocks)); break;
-        case 8: HEGJ_TRY(occ_gb<8>(device, &max_blocks)); break;
-        case 9: HEGJ_TRY(occ_gb<9>(device, &max_blocks)); break;
-        case 12: HEGJ_TRY(occ_gb<12>(device, &max_blocks)); break;
-        default: return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA kernel for this dimensionality");
+static hegj_status gb_occupancy(const GbOperands &ops, int device, uint32_t *blocks) {
+    if (ops.f16) return g16_occupancy(ops.kp, device, blocks);
+    switch (ops.kp / 32) {
+        case 2: return occ_gb<2>(device, blocks);
+        case 3: return occ_gb<3>(device, blocks);
+        case 4: return occ_gb<4>(device, blocks);
+        case 6: return occ_gb<6>(device, blocks);
+        case 8: return occ_gb<8>(device, blocks);
+        case 9: return occ_gb<9>(device, blocks);
+        case 12: return occ_gb<12>(device, blocks);
     }
+    return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA kernel for this dimensionality");
+}
+
+static hegj_status gb_launch(const GbOperands &ops, const GbArgs &a, uint32_t blocks, hipStream_t s) {
+    if (ops.f16) return g16_launch(a, blocks, s);
+    switch (ops.kp / 32) {
+        case 2: return launch_gb<2>(a, blocks, s);
+        case 3: return launch_gb<3>(a, blocks, s);
+        case 4: return launch_gb<4>(a, blocks, s);
+        case 6: return launch_gb<6>(a, blocks, s);
+        case 8: return launch_gb<8>(a, blocks, s);
+        case 9: return launch_gb<9>(a, blocks, s);
+        case 12: return launch_gb<12>(a, blocks, s);
+    }
+    return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA kernel for this dimensionality");
+}
+
+hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, uint32_t n_units,
+                    const GbOperands &ops, bool mirror, int device, hipStream_t s, GbOutput *out,
+                    uint64_t pair_cap_first, uint32_t parts) {
+    uint32_t max_blocks = 0;
+    HEGJ_TRY(gb_occupancy(ops, device, &max_blocks));
     const uint32_t n = g.n;
     uint64_t pair_cap = pair_cap_first ? std::max<uint64_t>(pair_cap_first, 4096)
                                        : std::max<uint64_t>((uint64_t)n * 48, 1u << 22);
     uint64_t band_cap = std::max<uint64_t>((uint64_t)n * 8, 1u << 22);
+    // FP16: one survivor stands for up to two pairs
+    uint64_t raw_cap = pair_cap_first ? pair_cap : std::max<uint64_t>((uint64_t)n * 32, 1u << 22);
     struct Ctr {
         uint32_t queue_heads[kMaxParts], overflow, pad;
-        unsigned long long pair_cursor, band_cursor, n_accept, n_band, evals;
+        unsigned long long pair_cursor, band_cursor, n_accept, n_band, evals, raw_cursor, raw_lost;
     };
     parts = std::max<uint32_t>(1, std::min<uint32_t>(parts, (uint32_t)kMaxParts));
     if (n_units < parts * 64) parts = 1;
@@ -712,21 +603,33 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const uint2 *units, u
         uint64_t *pairs = nullptr, *band = nullptr;
         Scratch it;
         HIP_TRY(it.get(&pairs, pair_cap));
-        HIP_TRY(it.get(&band, band_cap));
+        uint64_t *raw = nullptr;
+        float *raw_s = nullptr;
+        if (ops.f16) {
+            raw_cap = std::min<uint64_t>((raw_cap + kGbBlk - 1) / kGbBlk, 0xFFFFFFu) * kGbBlk;
+            HIP_TRY(it.get(&raw, raw_cap));
+            HIP_TRY(it.get(&raw_s, raw_cap));
+        } else {
+            HIP_TRY(it.get(&band, band_cap));
+        }
         HIP_TRY(hipMemsetAsync(d, 0, sizeof(Ctr), s));
         GbArgs a{};
         a.g = g;
         a.ix = ix;
-        a.units = units;
+        a.units = static_cast<const uint2 *>(units);
+        a.units16 = static_cast<const uint4 *>(units);
         a.n_units = n_units;
+        a.mirror = mirror ? 1u : 0u;
+        a.trej = ops.trej;
+        a.tacc = ops.tacc;
         a.queue_heads = d->queue_heads;
         a.n_parts = parts;
         for (uint32_t p = 0; p < parts; p++)
             a.part_end[p] = (uint32_t)((uint64_t)n_units * (p + 1) / parts);
-        a.Av = Av;
-        a.Bv = Bv;
-        a.w = w;
-        a.kp = kp;
+        a.Av = ops.A;
+        a.Bv = ops.B;
+        a.w = ops.w;
+        a.kp = ops.kp;
         a.pairs = pairs;
         a.pair_cap = pair_cap;
         a.pair_cursor = &d->pair_cursor;
@@ -737,34 +640,39 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const uint2 *units, u
         a.n_band = &d->n_band;
         a.evals = &d->evals;
         a.overflow = &d->overflow;
+        a.raw = raw;
+        a.raw_s = raw_s;
+        a.raw_cap = raw_cap;
+        a.raw_cursor = &d->raw_cursor;
+        a.raw_lost = &d->raw_lost;
         const uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>(max_blocks, n_units));
         hipEvent_t e0, e1;
         HIP_TRY(hipEventCreate(&e0));
         HIP_TRY(hipEventCreate(&e1));
         HIP_TRY(hipEventRecord(e0, s));
-        switch (kb) {
-            case 2: HEGJ_TRY(launch_gb<2>(a, blocks, s)); break;
-            case 3: HEGJ_TRY(launch_gb<3>(a, blocks, s)); break;
-            case 4: HEGJ_TRY(launch_gb<4>(a, blocks, s)); break;
-            case 6: HEGJ_TRY(launch_gb<6>(a, blocks, s)); break;
-            case 8: HEGJ_TRY(launch_gb<8>(a, blocks, s)); break;
-            case 9: HEGJ_TRY(launch_gb<9>(a, blocks, s)); break;
-            case 12: HEGJ_TRY(launch_gb<12>(a, blocks, s)); break;
-        }
+        HEGJ_TRY(gb_launch(ops, a, blocks, s));
         HIP_TRY(hipEventRecord(e1, s));
+        if (ops.f16) HEGJ_TRY(g16_decide(a, 2048, s));
         HIP_TRY(hipMemcpyAsync(&c, d, sizeof(Ctr), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         float kms = 0;
         HIP_TRY(hipEventElapsedTime(&kms, e0, e1));
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
+        if (c.raw_lost) {
+            const uint64_t need = (uint64_t)((raw_cap + c.raw_lost) * 1.125) + (1u << 22);
+            if (need > 0xFFFFFF00ull) return fail(HEGJ_ERR_UNSUPPORTED, "more than 2^32 pair slots");
+            raw_cap = need;
+            pair_cap = std::max(pair_cap, need * (mirror ? 2 : 1));
+            continue;
+        }
         if (c.overflow) {
-            pair_cap = std::max(pair_cap * 2, (uint64_t)((c.n_accept + c.n_band) * 1.25) + (1u << 22));
+            pair_cap = std::max(pair_cap * 2, (uint64_t)((c.n_accept + (ops.f16 ? 0 : c.n_band)) * 1.25) + (1u << 22));
             band_cap = std::max(band_cap * 2, (uint64_t)(c.n_band * 1.25) + (1u << 22));
             continue;
         }
         // exact FP64 recheck of the band
-        uint64_t nb = c.band_cursor;
+        const uint64_t nb = ops.f16 ? 0 : c.band_cursor;
         if (nb) {
             k_gb_recheck<<<ceil_div(nb, 256), 256, 0, s>>>(band, nb, ix.soa, n, g.dim, g.thresh, pairs,
                                                           pair_cap, &d->pair_cursor, &d->n_accept,
