@@ -1786,18 +1786,9 @@ hegj_status hegj_result_copy_csr(const hegj_result *r, uint64_t *offsets, uint32
     if (!nbrs || total == 0) return HEGJ_OK;
     uint32_t *d_nb;
     HIP_TRY(sc.get(&d_nb, total));
-    HEGJ_TRY(gather_rows(r->batches, r->bases, r->d_row_off, r->d_row_cnt, d_off, n, d_nb, s));
+    HEGJ_TRY(gather_rows(r->batches, r->bases, r->d_row_off, r->d_row_cnt, d_off, n, d_nb, sort_rows != 0, s));
     HIP_TRY(hipMemcpyAsync(nbrs, d_nb, sizeof(uint32_t) * total, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (sort_rows) {
-        unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-        std::vector<std::thread> th;
-        for (unsigned t = 0; t < nt; t++)
-            th.emplace_back([&, t]() {
-                for (uint64_t q = t; q < n; q += nt) std::sort(nbrs + offsets[q], nbrs + offsets[q + 1]);
-            });
-        for (auto &x : th) x.join();
-    }
     return HEGJ_OK;
 }
 

@@ -335,9 +335,10 @@ hegj_status split_units(const DevIndex &ix, const uint2 *units, uint32_t n_units
 hegj_status gather_units(const uint2 *in, const uint32_t *idx, uint32_t n, uint2 *out,
                          hipStream_t s);
 hegj_status csr_offsets(const uint32_t *row_cnt, uint32_t n, uint64_t *csr_off, hipStream_t s);
+// Rows into CSR order; sorted: each ascending.
 hegj_status gather_rows(const std::vector<uint32_t *> &batches, const std::vector<uint64_t> &bases,
                         const uint64_t *row_off, const uint32_t *row_cnt, const uint64_t *csr_off,
-                        uint32_t n, uint32_t *out, hipStream_t s);
+                        uint32_t n, uint32_t *out, bool sorted, hipStream_t s);
 
 hegj_status stream_copy(uint64_t bytes, int reps, double *ms_per_copy);
 // row_off[qid[i]] = base + off[i], row_cnt[qid[i]] = cnt[i] (rows answered

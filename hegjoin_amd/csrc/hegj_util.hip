@@ -100,6 +100,204 @@ __global__ __launch_bounds__(kT) void k_gather_rows(BatchTable bt,
     for (uint32_t i = lane; i < cnt; i += 64) dst[i] = src[i];
 }
 
+// ---- rows sorted ascending on their way into CSR ---------------------------
+// Sorting on the host (16 threads of std::sort) cost more than the join: join
+// and table of 500k 3-D points, 25 neighbours each, took 24.9 ms and take
+// 8.7; of 60k 6-D points, 64 each, 6.2 and 2.5; of 20k 2-D points 2.1 and
+// 0.82.  Here a row is sorted in a wave's registers between its load and its
+// store, so the pass moves what the plain gather moves.  Networks are bitonic with ascending
+// comparators only (the first step of a stage pairs mirrored elements), so
+// absent elements are ~0 and stay at the end.
+//   rows of up to 16 / 32: four / two of them per wave (most rows are short;
+//   one 64-wide network each would idle half the lanes or more);
+//   up to 1024: 1 to 16 elements per lane;
+//   longer: listed, one workgroup each in LDS (k_sort_long).
+
+// One comparator step for the lane's own element: its partner is lane ^ x,
+// and the lane with a zero in `bit` keeps the smaller.
+__device__ __forceinline__ uint32_t cx_lane(uint32_t v, int x, int bit) {
+    const uint32_t o = (uint32_t)__shfl_xor((int)v, x, 64);
+    return ((threadIdx.x & bit) == 0) == (o < v) ? o : v;
+}
+
+// Ascending within each group of G lanes.
+template <int G>
+__device__ __forceinline__ uint32_t sort_lanes(uint32_t v) {
+#pragma unroll
+    for (int k = 2; k <= G; k <<= 1) {
+        v = cx_lane(v, k - 1, k >> 1);
+#pragma unroll
+        for (int j = k >> 2; j > 0; j >>= 1) v = cx_lane(v, j, j);
+    }
+    return v;
+}
+
+// Ascending over 64 E elements, element e * 64 + lane in v[e].
+template <int E>
+__device__ __forceinline__ void sort_wave(uint32_t (&v)[E]) {
+#pragma unroll
+    for (int e = 0; e < E; e++) v[e] = sort_lanes<64>(v[e]);
+#pragma unroll
+    for (int m = 2; m <= E; m <<= 1) {  // stage of 64 m elements
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int f = e ^ (m - 1);
+            if (f < e) continue;
+            // mirrored partner: lane ^ 63 of register f
+            const uint32_t a = (uint32_t)__shfl_xor((int)v[e], 63, 64), b = (uint32_t)__shfl_xor((int)v[f], 63, 64);
+            v[e] = min(v[e], b);
+            v[f] = max(v[f], a);
+        }
+#pragma unroll
+        for (int j = m >> 2; j > 0; j >>= 1)
+#pragma unroll
+            for (int e = 0; e < E; e++)
+                if ((e & j) == 0) {
+                    const uint32_t lo = min(v[e], v[e | j]), hi = max(v[e], v[e | j]);
+                    v[e] = lo;
+                    v[e | j] = hi;
+                }
+#pragma unroll
+        for (int e = 0; e < E; e++)
+#pragma unroll
+            for (int j = 32; j > 0; j >>= 1) v[e] = cx_lane(v[e], j, j);
+    }
+}
+
+template <int E>
+__device__ __forceinline__ void sort_row(const uint32_t *src, uint32_t *dst, uint32_t cnt) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) v[e] = e * 64 + lane < cnt ? src[e * 64 + lane] : ~0u;
+    sort_wave<E>(v);
+#pragma unroll
+    for (int e = 0; e < E; e++)
+        if (e * 64 + lane < cnt) dst[e * 64 + lane] = v[e];
+}
+
+__device__ __forceinline__ const uint32_t *row_src(const BatchTable &bt, uint64_t go) {
+    uint32_t b = 0;
+    while (b + 1 < bt.nb && bt.base[b + 1] <= go) b++;
+    return bt.ptr[b] + (go - bt.base[b]);
+}
+
+// Four consecutive rows per wave and step.
+__global__ __launch_bounds__(kT) void k_gather_sorted(BatchTable bt, const uint64_t *__restrict__ row_off,
+                                                      const uint32_t *__restrict__ row_cnt,
+                                                      const uint64_t *__restrict__ csr_off, uint32_t n,
+                                                      uint32_t *__restrict__ out, uint32_t *__restrict__ longs,
+                                                      uint32_t *__restrict__ n_long) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = blockIdx.x * (kT / 64) + (threadIdx.x >> 6), waves = gridDim.x * (kT / 64);
+    for (uint64_t r0 = (uint64_t)wave * 4; r0 < n; r0 += (uint64_t)waves * 4) {
+        const uint32_t seg = (uint32_t)r0 + (lane >> 4);  // 16 lanes per row
+        const uint32_t c = seg < n ? row_cnt[seg] : 0u;
+        uint32_t c4[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) c4[i] = (uint32_t)__builtin_amdgcn_readlane((int)c, i * 16);
+        if (max(max(c4[0], c4[1]), max(c4[2], c4[3])) <= 16) {
+            const uint32_t i = lane & 15;
+            const uint32_t v = sort_lanes<16>(i < c ? row_src(bt, row_off[seg])[i] : ~0u);
+            if (i < c) out[csr_off[seg] + i] = v;
+            continue;
+        }
+#pragma unroll
+        for (int p = 0; p < 4; p += 2) {
+            if (max(c4[p], c4[p + 1]) <= 32) {
+                const uint32_t q = (uint32_t)r0 + p + (lane >> 5), i = lane & 31;
+                const uint32_t cq = lane < 32 ? c4[p] : c4[p + 1];
+                const uint32_t v = sort_lanes<32>(i < cq ? row_src(bt, row_off[q])[i] : ~0u);
+                if (i < cq) out[csr_off[q] + i] = v;
+                continue;
+            }
+#pragma unroll 1
+            for (int h = 0; h < 2; h++) {
+                const uint32_t q = (uint32_t)r0 + p + h, cq = h ? c4[p + 1] : c4[p];
+                if (cq == 0) continue;
+                const uint32_t *src = row_src(bt, row_off[q]);
+                uint32_t *dst = out + csr_off[q];
+                if (cq <= 64) {
+                    sort_row<1>(src, dst, cq);
+                } else if (cq <= 128) {
+                    sort_row<2>(src, dst, cq);
+                } else if (cq <= 256) {
+                    sort_row<4>(src, dst, cq);
+                } else if (cq <= 512) {
+                    sort_row<8>(src, dst, cq);
+                } else if (cq <= 1024) {
+                    sort_row<16>(src, dst, cq);
+                } else {
+                    for (uint32_t i = lane; i < cq; i += 64) dst[i] = src[i];
+                    if (lane == 0) longs[atomicAdd(n_long, 1u)] = q;
+                }
+            }
+        }
+    }
+}
+
+// Listed rows, one workgroup each, in place: LDS blocks of kLdsRow elements;
+// rows longer than that also take the network's far steps in global memory
+// (one workgroup's accesses, ordered by its barriers).
+constexpr uint32_t kLdsRow = 16384;
+constexpr uint32_t kLongT = 1024;
+
+// Comparator step on n elements at p: pairs (lo, lo + j), or mirrored within
+// blocks of 2 j.  Elements at and past `c` are absent (above all others).
+template <bool MIRROR>
+__device__ __forceinline__ void cx_step(uint32_t *p, uint32_t half, uint32_t j, uint32_t c) {
+    for (uint32_t i = threadIdx.x; i < half; i += kLongT) {
+        const uint32_t o = i & (j - 1), b = (i - o) * 2;
+        const uint32_t lo = b + o, hi = MIRROR ? b + 2 * j - 1 - o : lo + j;
+        if (hi < c) {
+            const uint32_t x = p[lo], y = p[hi];
+            if (y < x) {
+                p[lo] = y;
+                p[hi] = x;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(kLongT) void k_sort_long(const uint32_t *__restrict__ row_cnt,
+                                                      const uint64_t *__restrict__ csr_off, uint32_t *out,
+                                                      const uint32_t *__restrict__ longs,
+                                                      const uint32_t *__restrict__ n_long) {
+    __shared__ uint32_t sh[kLdsRow];
+    const uint32_t rows = *n_long;
+    for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const uint32_t q = longs[r], c = row_cnt[q];
+        uint32_t *row = out + csr_off[q];
+        uint32_t pow2 = 2048;
+        while (pow2 < c) pow2 <<= 1;
+        for (uint32_t k = 0; k <= pow2;) {
+            // k = 0: sort the blocks; else stage k of the far network, then its near steps
+            if (k) {
+                cx_step<true>(row, pow2 / 2, k / 2, c);
+                for (uint32_t j = k / 4; j >= kLdsRow; j >>= 1) cx_step<false>(row, pow2 / 2, j, c);
+            }
+            for (uint32_t b = 0; b < c; b += kLdsRow) {
+                const uint32_t m = min(kLdsRow, c - b);
+                for (uint32_t i = threadIdx.x; i < m; i += kLongT) sh[i] = row[b + i];
+                __syncthreads();
+                const uint32_t half = min(pow2, kLdsRow) / 2;
+                if (k == 0) {
+                    for (uint32_t s = 2; s <= half * 2; s <<= 1) {
+                        cx_step<true>(sh, half, s / 2, m);
+                        for (uint32_t j = s / 4; j > 0; j >>= 1) cx_step<false>(sh, half, j, m);
+                    }
+                } else {
+                    for (uint32_t j = half; j > 0; j >>= 1) cx_step<false>(sh, half, j, m);
+                }
+                for (uint32_t i = threadIdx.x; i < m; i += kLongT) row[b + i] = sh[i];
+                __syncthreads();
+            }
+            k = k ? k * 2 : kLdsRow * 2;
+        }
+    }
+}
+
 __global__ __launch_bounds__(kT) void k_u32_to_u64(const uint32_t *__restrict__ in, uint32_t n,
                                                    uint64_t *__restrict__ out) {
     uint32_t i = blockIdx.x * kT + threadIdx.x;
@@ -174,7 +372,7 @@ hegj_status csr_offsets(const uint32_t *row_cnt, uint32_t n, uint64_t *csr_off, 
 
 hegj_status gather_rows(const std::vector<uint32_t *> &batches, const std::vector<uint64_t> &bases,
                         const uint64_t *row_off, const uint32_t *row_cnt, const uint64_t *csr_off,
-                        uint32_t n, uint32_t *out, hipStream_t s) {
+                        uint32_t n, uint32_t *out, bool sorted, hipStream_t s) {
     if (batches.size() > (size_t)kMaxBatches) return fail(HEGJ_ERR_UNSUPPORTED, "too many result batches");
     BatchTable bt{};
     bt.nb = (uint32_t)batches.size();
@@ -183,6 +381,19 @@ hegj_status gather_rows(const std::vector<uint32_t *> &batches, const std::vecto
         bt.base[i] = bases[i];
     }
     bt.base[batches.size()] = ~0ull;
+    if (sorted) {
+        Scratch sc;
+        uint32_t *longs;  // row ids, then their number
+        HIP_TRY(sc.get(&longs, (size_t)n + 1));
+        HEGJ_TRY(zero_words(longs + n, sizeof(uint32_t), s));
+        k_gather_sorted<<<std::min<uint32_t>(ceil_div((uint64_t)n, 4 * (kT / 64)), 8192), kT, 0, s>>>(
+            bt, row_off, row_cnt, csr_off, n, out, longs, longs + n);
+        HIP_TRY(hipGetLastError());
+        k_sort_long<<<512, kLongT, 0, s>>>(row_cnt, csr_off, out, longs, longs + n);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(s));
+        return HEGJ_OK;
+    }
     k_gather_rows<<<ceil_div((uint64_t)n * 64, kT), kT, 0, s>>>(bt, row_off, row_cnt, csr_off, n, out);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
