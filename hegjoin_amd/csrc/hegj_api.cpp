@@ -323,16 +323,17 @@ uint32_t default_qb(uint32_t dim) {
     return 8;
 }
 
+// Device counters of a join; what many waves update has a line of its own.
 struct Counters {
-    uint32_t queue_heads[kMaxParts];
-    uint32_t n_deferred;
-    uint32_t pad;
-    unsigned long long cursor;
-    unsigned long long hash;
-    unsigned long long evals;
-    unsigned long long pairs;
-    unsigned long long band;  // FP32 filter: pairs rechecked in FP64
-    unsigned long long mismatch;  // units whose write pass disagreed with their count
+    uint32_t queue_heads[kMaxParts * kLineWords];
+    uint32_t n_deferred, pad0[kLineWords - 1];
+    unsigned long long cursor, pad1[kLineWords / 2 - 1];
+    unsigned long long stats[kStatSlots][kLineWords / 2];
+    uint64_t sum(JoinStat k) const {
+        uint64_t t = 0;
+        for (const auto &line : stats) t += line[k];
+        return t;
+    }
 };
 
 hegj_status ensure_morton(hegj_index *h) {
@@ -402,6 +403,7 @@ struct JoinPlan {
     uint32_t parts = 1;
     uint32_t part_end[kMaxParts] = {};
     uint64_t capacity = 0;
+    uint32_t chunk = 0;  // output entries a wave reserves at a time in the first batch
     double estimate_ms = 0;
     uint64_t estimated_pairs = 0;  // the estimator's extrapolated pair count
     bool f32 = false;  // FP32 filter with FP64 band recheck
@@ -458,17 +460,13 @@ JoinArgs base_args(const hegj_index *h, const hegj_join_opts &opts, const JoinPl
     a.queue_heads = P.d_ctr->queue_heads;
     a.n_deferred = &P.d_ctr->n_deferred;
     a.cursor = &P.d_ctr->cursor;
-    a.hash = &P.d_ctr->hash;
-    a.evals = &P.d_ctr->evals;
-    a.pairs = &P.d_ctr->pairs;
+    a.stats = P.d_ctr->stats[0];
     a.deferred = P.deferred;
     a.gmask = P.gmask;
     a.gmask_slots = P.gmask_slots;
     a.block_waves = P.waves;
     a.part_by_xcc = opts.part_by_block ? 0u : 1u;
     a.prune = opts.no_prune ? 0u : 1u;
-    a.band = &P.d_ctr->band;
-    a.mismatch = &P.d_ctr->mismatch;
     if (P.f32) {
         a.f32 = 1;
         a.soa32 = h->soa32;
@@ -539,10 +537,22 @@ hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, co
         Counters c;
         HIP_TRY(hipMemcpyAsync(&c, P.d_ctr, sizeof(c), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
-        const double est = (double)c.pairs * ((double)U / (double)ns);
+        const double est = (double)c.sum(kStatPairs) * ((double)U / (double)ns);
         P.estimated_pairs = (uint64_t)est;
         const uint32_t nb = opts.batches ? opts.batches : 1u;
         P.capacity = (uint64_t)(est * 1.10 / nb) + (1u << 20);
+        if (nb == 1) {
+            // Waves reserve output in chunks of 16 average units (less when
+            // the waves' last chunks would exceed an eighth of the result).
+            // Up to a quarter of a chunk stays unused when the next one is
+            // taken, and each wave's last one: room for both is added.
+            const double avg = est / U, waves = (double)P.max_blocks * P.waves;
+            const double chunk = std::min(16.0 * avg + 64.0, (est / 8 + (1 << 20)) / waves);
+            if (chunk >= 4.0 * avg && chunk < 1e9) {
+                P.chunk = (uint32_t)chunk;
+                P.capacity += (uint64_t)(est * 0.15 + waves * chunk);
+            }
+        }
         size_t free_b = 0, total_b = 0;
         HIP_TRY(hipMemGetInfo(&free_b, &total_b));
         P.capacity = std::min<uint64_t>(P.capacity, (uint64_t)(free_b * 0.6) / sizeof(uint32_t));
@@ -638,6 +648,9 @@ struct BatchRunner {
                 set_parts(a, 1, &one_end);
             }
             a.count_only = 0;
+            // later batches are sized exactly, and launches that share a
+            // batch would each leave the ends of their chunks in it
+            a.chunk = last && cur == units ? P.chunk : 0u;
             {
                 EventTimer t(s);
                 HEGJ_TRY(launch_join(a, qb, blocks_for(P, cur_n, a.units_per_grab), s));
@@ -647,8 +660,8 @@ struct BatchRunner {
             if (last) HEGJ_TRY(launch_pair_hash(a, capacity, s));
             HIP_TRY(hipMemcpyAsync(&c, P.d_ctr, sizeof(c), hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
-            if (c.mismatch)
-                return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.mismatch) +
+            if (c.sum(kStatMismatch))
+                return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.sum(kStatMismatch)) +
                                               " work units disagreed with their counts");
             used = c.cursor;
             if (c.n_deferred == 0) {
@@ -688,16 +701,14 @@ struct BatchRunner {
             e.queue_heads = P.d_ctr2->queue_heads;
             e.n_deferred = &P.d_ctr2->n_deferred;
             e.cursor = &P.d_ctr2->cursor;
-            e.hash = &P.d_ctr2->hash;
-            e.evals = &P.d_ctr2->evals;
-            e.pairs = &P.d_ctr2->pairs;
+            e.stats = P.d_ctr2->stats[0];
             HIP_TRY(hipMemsetAsync(P.d_ctr2, 0, sizeof(Counters), s));
             HEGJ_TRY(launch_join(e, qb, blocks_for(P, e.n_units, e.units_per_grab), s));
             Counters c2;
             HIP_TRY(hipMemcpyAsync(&c2, P.d_ctr2, sizeof(c2), hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
             if (!opts.result_capacity) {
-                capacity = std::max<uint64_t>(c2.pairs, 1);
+                capacity = std::max<uint64_t>(c2.sum(kStatPairs), 1);
                 // a requested batch count keeps every batch at the first one's size
                 if (opts.batches > 1) capacity = std::min<uint64_t>(capacity, P.capacity);
             }
@@ -713,10 +724,10 @@ struct BatchRunner {
             HIP_TRY(hipMemcpyAsync(&c, P.d_ctr, sizeof(c), hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
         }
-        r->info.total_neighbors = c.pairs;
-        r->info.pair_hash = c.hash;
-        r->info.evals_executed = c.evals;
-        r->info.band_rechecks = c.band;
+        r->info.total_neighbors = c.sum(kStatPairs);
+        r->info.pair_hash = c.sum(kStatHash);
+        r->info.evals_executed = c.sum(kStatEvals);
+        r->info.band_rechecks = c.sum(kStatBand);
         r->info.refine_used = P.f32 ? HEGJ_REFINE_F32 : HEGJ_REFINE_FP64;
         r->info.n_batches = (uint32_t)r->batches.size();
         r->info.join_ms = join_ms;
@@ -1047,6 +1058,7 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
     a.out = buf;
     a.out_base = 0;
     a.capacity = G.P.capacity;
+    a.chunk = G.P.chunk;
     a.count_only = 0;
     HIP_TRY(hipStreamSynchronize(s));  // the previous replay has read the block
     *G.h_args = a;
@@ -1056,8 +1068,8 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
         r->info.join_ms = t.stop();  // synchronises the stream
     }
     const Counters c = *G.h_ctr;
-    if (c.mismatch)
-        return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.mismatch) +
+    if (c.sum(kStatMismatch))
+        return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.sum(kStatMismatch)) +
                                       " work units disagreed with their counts");
     if (c.n_deferred) {
         // grow the cached capacity for later replays; this call runs eagerly
@@ -1066,10 +1078,10 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
         return HEGJ_OK;
     }
     *fits = true;
-    r->info.total_neighbors = c.pairs;
-    r->info.pair_hash = c.hash;
-    r->info.evals_executed = c.evals;
-    r->info.band_rechecks = c.band;
+    r->info.total_neighbors = c.sum(kStatPairs);
+    r->info.pair_hash = c.sum(kStatHash);
+    r->info.evals_executed = c.sum(kStatEvals);
+    r->info.band_rechecks = c.sum(kStatBand);
     r->info.refine_used = G.P.f32 ? HEGJ_REFINE_F32 : HEGJ_REFINE_FP64;
     r->info.n_batches = 1;
     r->info.join_launches = 1;
@@ -1634,8 +1646,8 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
     info->join_kernel_avg_ms = join_ms;
     info->workload_ms = h->workload_ms;
     info->refine_used = P.f32 ? HEGJ_REFINE_F32 : HEGJ_REFINE_FP64;
-    if (c.mismatch)
-        return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.mismatch) +
+    if (c.sum(kStatMismatch))
+        return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.sum(kStatMismatch)) +
                                       " work units disagreed with their counts");
     if (c.n_deferred) {
         // the rows do not fit: count them all (count-only pass) for the caller
@@ -1644,23 +1656,21 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
         e.queue_heads = P.d_ctr2->queue_heads;
         e.n_deferred = &P.d_ctr2->n_deferred;
         e.cursor = &P.d_ctr2->cursor;
-        e.hash = &P.d_ctr2->hash;
-        e.evals = &P.d_ctr2->evals;
-        e.pairs = &P.d_ctr2->pairs;
+        e.stats = P.d_ctr2->stats[0];
         HEGJ_TRY(zero_words(P.d_ctr2, sizeof(Counters), s));
         HEGJ_TRY(launch_join(e, qb, blocks_for(P, U, e.units_per_grab), s));
         Counters c2;
         HIP_TRY(hipMemcpyAsync(&c2, P.d_ctr2, sizeof(c2), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
-        info->total_neighbors = c2.pairs;
-        return fail(HEGJ_ERR_CAPACITY, "hegj_selfjoin_noalloc: the result has " + std::to_string(c2.pairs) +
+        info->total_neighbors = c2.sum(kStatPairs);
+        return fail(HEGJ_ERR_CAPACITY, "hegj_selfjoin_noalloc: the result has " + std::to_string(c2.sum(kStatPairs)) +
                                            " neighbours, the buffer holds " + std::to_string(capacity) +
                                            " (info->total_neighbors has the count)");
     }
-    info->total_neighbors = c.pairs;
-    info->pair_hash = c.hash;
-    info->evals_executed = c.evals;
-    info->band_rechecks = c.band;
+    info->total_neighbors = c.sum(kStatPairs);
+    info->pair_hash = c.sum(kStatHash);
+    info->evals_executed = c.sum(kStatEvals);
+    info->band_rechecks = c.sum(kStatBand);
     info->n_batches = 1;
     info->estimated_pairs = 0;
     info->total_ms =

@@ -137,6 +137,12 @@ hegj_status radix_sort_u32(uint32_t *keys, uint32_t *vals, uint32_t *keys_alt,
 
 // Arguments of the join kernel (hegj_join.hip).
 constexpr int kMaxParts = 8;   // one unit range (queue) per XCD
+// Atomics on one address are served one after the other, ~12 ns each (a pair
+// hash pass of 16384 of them took 190 us), so counters that many waves update
+// have lines of their own and waves add to them as rarely as they can.
+constexpr int kLineWords = 32;              // uint32 per line
+constexpr int kStatSlots = 8;               // sums, one line per XCD
+enum JoinStat { kStatEvals, kStatPairs, kStatBand, kStatHash, kStatMismatch };
 struct JoinArgs {
     GridGeom g;
     DevIndex ix;
@@ -148,20 +154,22 @@ struct JoinArgs {
     uint32_t part_by_xcc;         // 1: range = hardware XCC id, 0: blockIdx % n_parts
     uint32_t part_begin[kMaxParts];
     uint32_t part_end[kMaxParts];
-    uint32_t *queue_heads;        // [kMaxParts] units taken per range
+    uint32_t *queue_heads;        // [kMaxParts] lines: units taken per range past the static grabs
     uint64_t *gmask;              // per-wave hit-mask scratch (global)
     uint32_t gmask_slots;         // masks per wave in gmask
     uint32_t *out;                // this batch's neighbour buffer
     uint64_t out_base;            // global offset of out[0]
     uint64_t capacity;            // entries in out
     unsigned long long *cursor;   // entries reserved in out
+    uint32_t chunk;               // entries a wave reserves at a time (0: exactly its unit's)
     uint64_t *row_off;            // [n] global offset per query id
     uint32_t *row_cnt;            // [n]
     uint32_t *deferred;           // units that did not fit
     uint32_t *n_deferred;
-    unsigned long long *hash;     // multiset hash of written pairs
-    unsigned long long *evals;    // distance evaluations performed
-    unsigned long long *pairs;    // pairs found (count-only) or written
+    // [kStatSlots] lines of sums, by JoinStat: distance evaluations performed,
+    // pairs found (count-only) or written, pairs rechecked in FP64, multiset
+    // hash of the written pairs, units whose write pass disagreed with their count
+    unsigned long long *stats;
     uint32_t count_only;
     uint32_t prune;               // 1: cell-box pruning of stencil cells
     // FP32 filter (f32 != 0): centred float coordinates and the two
@@ -170,8 +178,6 @@ struct JoinArgs {
     const float *soa32;           // [dim][n], cell order
     const float *aos32;           // [n][dim], cell order (dim <= kAosMaxDim)
     float tacc32, trej32;
-    unsigned long long *band;     // pairs rechecked in FP64
-    unsigned long long *mismatch; // units whose write pass disagreed with their count
 };
 
 // ---- index (hegj_index.hip) ----------------------------------------------
@@ -190,7 +196,7 @@ hegj_status build_units(const GridGeom &g, const DevIndex &ix, uint32_t qb, cons
 hegj_status launch_join(const JoinArgs &a, uint32_t qb, uint32_t blocks, hipStream_t s,
                         const JoinArgs *dev_args = nullptr);
 // Adds the pair hash of the batch's finished rows (a.out, a.row_off,
-// a.row_cnt, a.out_base, a.capacity) to *a.hash; pairs_hint (expected pairs)
+// a.row_cnt, a.out_base, a.capacity) to a.stats; pairs_hint (expected pairs)
 // picks the lanes per row.
 hegj_status launch_pair_hash(const JoinArgs &a, uint64_t pairs_hint, hipStream_t s,
                              const JoinArgs *dev_args = nullptr);

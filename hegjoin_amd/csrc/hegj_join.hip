@@ -470,24 +470,120 @@ struct HitStore {
 
 constexpr int kRegDims = 32;  // dims kept in registers (with prefetch)
 
-// Takes the next grab of units: from the workgroup's own range first (its
-// XCD's share of the space, for L2 locality), then from the others.
-__device__ __forceinline__ bool next_grab(const JoinArgs &a, uint32_t &part, uint32_t &tries,
-                                          uint32_t &grab, uint32_t &gend) {
+// The kernel arguments, to be read again from here on.  They are ~100 scalar
+// registers' worth; kept live through a unit's loops they were spilled to
+// vector lanes (300 scalar spills, and vector spills in turn, in the
+// 128-register kernels: k_join_f32<6, 4> 39 vector spills, 4 with the reload;
+// k_join<0, 4> 161 registers, 128 with it, one more wave per SIMD).  Reloading
+// them costs scalar-cache hits.
+typedef __attribute__((address_space(4))) const JoinArgs *ArgsPtr;
+__device__ __forceinline__ const JoinArgs &reload(ArgsPtr p) {
+    __asm__ volatile("" : "+s"(p));
+    return *(const JoinArgs *)p;
+}
+template <bool IND>
+__device__ __forceinline__ ArgsPtr args_ptr(const JoinArgs *ap) {
+    if constexpr (IND)
+        return (ArgsPtr)ap;
+    else
+        return (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// Takes the next grab of units.  The first one is static (a wave's share of
+// the range of its workgroup's turn, blockIdx % n_parts: workgroups go to the
+// XCDs in turn), so a join with a grab per wave or less touches no queue;
+// then from the range of the wave's own XCD (for L2 locality), then from the
+// others, whose heads are read before they are added to.  With the chunked
+// output (reserve) this took the 3-D 500k kernel from 4.05 to 0.82 ms, 6-D 60k
+// from 0.99 to 0.6, 6-D 5M from 41.7 to 37.3: their waves queued for one line.
+struct Grabs {
+    uint32_t part = 0, tries = 0;
+    bool first = true;
+};
+
+__device__ __forceinline__ bool next_grab(const JoinArgs &a, Grabs &q, uint32_t &grab, uint32_t &gend) {
     const int lane = threadIdx.x & 63;
-    while (tries < a.n_parts) {
-        uint32_t g = 0;
-        if (lane == 0) g = atomicAdd(&a.queue_heads[part], a.units_per_grab);
-        g = wave_bcast_u32(g) + a.part_begin[part];
-        if (g < a.part_end[part]) {
-            grab = g;
-            gend = min(g + a.units_per_grab, a.part_end[part]);
+    const uint32_t wpb = blockDim.x >> 6;
+    if (q.first) {
+        q.first = false;
+        const uint32_t p = blockIdx.x % a.n_parts;
+        const uint64_t g = a.part_begin[p] + ((uint64_t)(blockIdx.x / a.n_parts) * wpb + wave_bcast_u32(threadIdx.x >> 6)) * a.units_per_grab;
+        if (g < a.part_end[p]) {
+            grab = (uint32_t)g;
+            gend = min(grab + a.units_per_grab, a.part_end[p]);
             return true;
         }
-        part = part + 1 == a.n_parts ? 0 : part + 1;
-        tries++;
+    }
+    while (q.tries < a.n_parts) {
+        const uint32_t p = q.part;
+        // units past the static grabs of the range
+        const uint64_t base = a.part_begin[p] + (uint64_t)((gridDim.x - p + a.n_parts - 1) / a.n_parts) * wpb * a.units_per_grab;
+        uint64_t g = base;
+        if (g < a.part_end[p]) {
+            uint32_t *const head = a.queue_heads + p * kLineWords;
+            uint32_t h = 0;
+            if (lane == 0) {
+                if (q.tries) h = __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (base + h < a.part_end[p]) h = atomicAdd(head, a.units_per_grab);
+            }
+            g = base + wave_bcast_u32(h);
+            if (g < a.part_end[p]) {
+                grab = (uint32_t)g;
+                gend = min(grab + a.units_per_grab, a.part_end[p]);
+                return true;
+            }
+        }
+        q.part = p + 1 == a.n_parts ? 0 : p + 1;
+        q.tries++;
     }
     return false;
+}
+
+// Output space: a wave reserves a.chunk entries at a time and gives its units
+// consecutive segments of it (one atomic per unit, all on one address, held
+// the 6-D join up); a unit of a quarter chunk or more, and any unit where the
+// chunk is 0, reserves exactly its entries, so at most a quarter of a chunk
+// is left behind when the next one is taken.  False: the unit does not fit in
+// the batch.  The wave's open chunk [cur, end) lives in LDS: it is used once
+// per unit, and the loops between have no registers to spare.
+struct Segment {
+    uint64_t cur, end;
+};
+
+__device__ __forceinline__ bool reserve(const JoinArgs &a, Segment &sg, uint32_t total, uint64_t &base) {
+    const bool lane0 = (threadIdx.x & 63) == 0;
+    if (total >= (a.chunk >> 2)) {
+        uint64_t b = 0;
+        if (lane0) b = atomicAdd(a.cursor, (unsigned long long)total);
+        base = wave_bcast_u64(b);
+        return base + total <= a.capacity;
+    }
+    uint64_t b = sg.cur, e = sg.end;
+    if (wave_bcast_u32(b + total > e ? 1u : 0u)) {
+        if (lane0) b = atomicAdd(a.cursor, (unsigned long long)a.chunk);
+        e = min(b + a.chunk, a.capacity);
+    }
+    base = wave_bcast_u64(b);
+    const bool fits = base + total <= a.capacity;
+    if (lane0) {
+        sg.cur = fits ? base + total : 0;
+        sg.end = fits ? e : 0;
+    }
+    return fits;
+}
+
+// The workgroup's sums, added to its XCD's line by one thread (every wave of
+// the workgroup calls this once, at its end).
+__device__ __forceinline__ void add_stats(const JoinArgs &a, unsigned long long *sh, uint64_t evals, uint64_t pairs,
+                                          uint64_t band) {
+    if ((threadIdx.x & 63) == 0) {
+        if (evals) atomicAdd(&sh[kStatEvals], (unsigned long long)evals);
+        if (pairs) atomicAdd(&sh[kStatPairs], (unsigned long long)pairs);
+        if (band) atomicAdd(&sh[kStatBand], (unsigned long long)band);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 && sh[threadIdx.x])
+        atomicAdd(a.stats + (xcc_id() % kStatSlots) * (kLineWords / 2) + threadIdx.x, sh[threadIdx.x]);
 }
 
 // IND: the arguments are read from device memory (ap) instead of the kernel
@@ -510,7 +606,8 @@ constexpr int join_min_waves() {
 template <int D, int QB, bool IND = false, bool FLT = false>
 __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) void k_join(
     JoinArgs av, const JoinArgs *__restrict__ ap) {
-    const JoinArgs &a = IND ? *ap : av;
+    const ArgsPtr args = args_ptr<IND>(ap);
+    const JoinArgs &a0 = reload(args);
     static_assert(!FLT || D == 0, "DTYPE=float: generic instance only");
     __shared__ RowList rls[kWavesPerBlock];
     __shared__ HitStore hs_all[kWavesPerBlock];
@@ -518,20 +615,28 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     RowList &rl = rls[wid];
     uint64_t *const hs_lds = hs_all[wid].w;
-    uint64_t *const hs_glb = a.gmask + (uint64_t)(blockIdx.x * (blockDim.x >> 6) + wid) * a.gmask_slots;
-    const double T = a.g.thresh;
+    uint64_t *const hs_glb = a0.gmask + (uint64_t)(blockIdx.x * (blockDim.x >> 6) + wid) * a0.gmask_slots;
+    const double T = a0.g.thresh;
     constexpr bool kRegs = (D > 0 && D <= kRegDims);
     constexpr int DR = kRegs ? D : 1;
     uint64_t my_evals = 0, my_pairs = 0;
     constexpr bool kQS = q_in_sgprs<D, QB>();
-    const uint32_t dimq = D > 0 ? (uint32_t)D : a.g.dim;
+    const uint32_t dimq = D > 0 ? (uint32_t)D : a0.g.dim;
     double *const qs = q_dyn + (size_t)wid * QB * dimq;
     double qreg[kQS ? QB : 1][kQS ? DR : 1];
-    uint32_t part = (a.part_by_xcc ? xcc_id() : blockIdx.x) % a.n_parts;
-    uint32_t tries = 0, grab = 0, gend = 0;
+    __shared__ unsigned long long sh_stats[3];
+    __shared__ Segment segs[kWavesPerBlock];
+    if (threadIdx.x < 3) sh_stats[threadIdx.x] = 0;
+    if (threadIdx.x < kWavesPerBlock) segs[threadIdx.x] = Segment{0, 0};
+    __syncthreads();
+    Grabs queue;
+    queue.part = (a0.part_by_xcc ? xcc_id() : blockIdx.x) % a0.n_parts;
+    uint32_t grab = 0, gend = 0;
+    Segment &seg = segs[wid];
 
-    while (next_grab(a, part, tries, grab, gend)) {
+    while (next_grab(reload(args), queue, grab, gend)) {
         for (uint32_t ui = grab; ui < gend; ui++) {
+            const JoinArgs &a = reload(args);
             const uint2 unit = a.units[ui];
             const uint32_t cell = wave_bcast_u32(unit.x), qoff = wave_bcast_u32(unit.y);
             const uint32_t cstart = a.ix.cell_start[cell];
@@ -687,16 +792,14 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
                 if (lane >= o) incl_l += y;
             }
             const uint32_t excl_l = incl_l - cnt_l;
-            const uint32_t total = __shfl(incl_l, QB - 1, 64);
+            const uint32_t total = wave_bcast_u32(__shfl(incl_l, QB - 1, 64));
             if (a.count_only) {
                 my_pairs += total;
                 continue;
             }
             uint64_t base = 0;
             if (total > 0) {
-                if (lane == 0) base = atomicAdd(a.cursor, (unsigned long long)total);
-                base = wave_bcast_u64(base);
-                if (base + total > a.capacity) {
+                if (!reserve(a, seg, total, base)) {
                     if (lane == 0) a.deferred[atomicAdd(a.n_deferred, 1u)] = ui;
                     continue;
                 }
@@ -767,7 +870,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
                 // masks did not fit anywhere (very large units): evaluate
                 // each chunk again, one query at a time.  The writes stay
                 // inside each query's reserved row [oq, oend); a count that
-                // differs from the first pass is reported (a.mismatch), never
+                // differs from the first pass is reported (kStatMismatch), never
                 // written past the row.
                 uint64_t oend[QB];
                 {
@@ -812,15 +915,11 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
                 }
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++) bad |= (uint32_t)qi < nq && oq[qi] != oend[qi];
-                if (bad && lane == 0) atomicAdd(a.mismatch, 1ull);
+                if (bad && lane == 0) atomicAdd(a.stats + kStatMismatch, 1ull);
             }
         }
     }
-    // one atomic per wave for the counters
-    if (lane == 0) {
-        if (my_evals) atomicAdd(a.evals, (unsigned long long)my_evals);
-        if (my_pairs) atomicAdd(a.pairs, (unsigned long long)my_pairs);
-    }
+    add_stats(reload(args), sh_stats, my_evals, my_pairs, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -933,7 +1032,8 @@ __device__ __forceinline__ void load_cand32_off(const float *aos32, uint32_t byt
 
 template <int D, int QB, bool IND>
 __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av, const JoinArgs *__restrict__ ap) {
-    const JoinArgs &a = IND ? *ap : av;
+    const ArgsPtr args = args_ptr<IND>(ap);
+    const JoinArgs &a0 = reload(args);
     static_assert((D == 2 || D == 6) && QB * D <= 48 && QB <= 16, "FP32 filter: 2-D and 6-D");
     __shared__ RowList rls[kWavesPerBlock];
     __shared__ HitStore hs_all[kWavesPerBlock];
@@ -942,19 +1042,26 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
     RowList &rl = rls[wid];
     F32Lds &fl = fls[wid];
     uint64_t *const hs_lds = hs_all[wid].w;
-    uint64_t *const hs_glb = a.gmask + (uint64_t)(blockIdx.x * (blockDim.x >> 6) + wid) * a.gmask_slots;
+    uint64_t *const hs_glb = a0.gmask + (uint64_t)(blockIdx.x * (blockDim.x >> 6) + wid) * a0.gmask_slots;
     constexpr uint32_t kStride = D * (uint32_t)sizeof(float);
     constexpr uint32_t kChunkBytes = 64u * kStride;
     const uint32_t lane_off = (uint32_t)lane * kStride;
-    const double T = a.g.thresh;
-    const float tacc = a.tacc32, trej = a.trej32;
+    const float tacc = a0.tacc32, trej = a0.trej32;
     uint64_t my_evals = 0, my_pairs = 0, my_band = 0;
     float qregf[QB][D];
-    uint32_t part = (a.part_by_xcc ? xcc_id() : blockIdx.x) % a.n_parts;
-    uint32_t tries = 0, grab = 0, gend = 0;
+    __shared__ unsigned long long sh_stats[3];
+    __shared__ Segment segs[kWavesPerBlock];
+    if (threadIdx.x < 3) sh_stats[threadIdx.x] = 0;
+    if (threadIdx.x < kWavesPerBlock) segs[threadIdx.x] = Segment{0, 0};
+    __syncthreads();
+    Grabs queue;
+    queue.part = (a0.part_by_xcc ? xcc_id() : blockIdx.x) % a0.n_parts;
+    uint32_t grab = 0, gend = 0;
+    Segment &seg = segs[wid];
 
-    while (next_grab(a, part, tries, grab, gend)) {
+    while (next_grab(reload(args), queue, grab, gend)) {
         for (uint32_t ui = grab; ui < gend; ui++) {
+            const JoinArgs &a = reload(args);
             const uint2 unit = a.units[ui];
             const uint32_t cell = wave_bcast_u32(unit.x), qoff = wave_bcast_u32(unit.y);
             const uint32_t cstart = a.ix.cell_start[cell];
@@ -1121,7 +1228,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
                             const double dd = a.ix.soa[(uint64_t)l * n + pos] - a.ix.soa[(uint64_t)l * n + qpos0 + qi];
                             e64 = __builtin_fma(dd, dd, e64);
                         }
-                        hit = e64 <= T;
+                        hit = e64 <= a.g.thresh;
                     }
                     const uint64_t madd = __builtin_amdgcn_ballot_w64(hit);
                     if (madd) {
@@ -1142,16 +1249,14 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
                 if (lane >= o) incl_l += y;
             }
             const uint32_t excl_l = incl_l - cnt_l;
-            const uint32_t total = __shfl(incl_l, QB - 1, 64);
+            const uint32_t total = wave_bcast_u32(__shfl(incl_l, QB - 1, 64));
             if (a.count_only) {
                 my_pairs += total;
                 continue;
             }
             uint64_t base = 0;
             if (total > 0) {
-                if (lane == 0) base = atomicAdd(a.cursor, (unsigned long long)total);
-                base = wave_bcast_u64(base);
-                if (base + total > a.capacity) {
+                if (!reserve(a, seg, total, base)) {
                     if (lane == 0) a.deferred[atomicAdd(a.n_deferred, 1u)] = ui;
                     continue;
                 }
@@ -1236,7 +1341,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
                 // chunk again with the exact chain, one query at a time.  The
                 // writes stay inside each query's reserved row [oq, oend); a
                 // count that differs from the first pass is reported
-                // (a.mismatch), never written past the row.
+                // (kStatMismatch), never written past the row.
                 uint64_t oend[QB];
                 {
                     const uint64_t e_l = base + excl_l + cnt_l;
@@ -1276,7 +1381,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
                                 acc1 = __builtin_fma(dd, dd, acc1);
                             }
                         }
-                        const uint64_t m = __ballot(valid && acc1 <= T);
+                        const uint64_t m = __ballot(valid && acc1 <= a.g.thresh);
                         if (m == 0) continue;
                         const uint64_t room = oend[qi] - oq[qi];
                         const uint64_t pc = (uint64_t)__popcll(m);
@@ -1288,15 +1393,11 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
                 }
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++) bad |= (uint32_t)qi < nq && oq[qi] != oend[qi];
-                if (bad && lane == 0) atomicAdd(a.mismatch, 1ull);
+                if (bad && lane == 0) atomicAdd(a.stats + kStatMismatch, 1ull);
             }
         }
     }
-    if (lane == 0) {
-        if (my_band && a.band) atomicAdd(a.band, (unsigned long long)my_band);
-        if (my_evals) atomicAdd(a.evals, (unsigned long long)my_evals);
-        if (my_pairs) atomicAdd(a.pairs, (unsigned long long)my_pairs);
-    }
+    add_stats(reload(args), sh_stats, my_evals, my_pairs, my_band);
 }
 
 // Per-cell candidate count over the stencil (sortByWorkLoadGlobal).
@@ -1464,7 +1565,8 @@ hegj_status launch_join(const JoinArgs &a, uint32_t qb, uint32_t blocks, hipStre
 // Pair hash of one batch: sum of mix64(query << 32 | neighbour) over the rows
 // the batch holds (row offsets in [out_base, out_base + capacity)).  G lanes
 // per row (G = 64 for long rows), each reading 4 entries per step, so a row
-// is read in runs of 4G entries; one atomic per wave.
+// is read in runs of 4G entries; one atomic per workgroup, on its XCD's line
+// (one per wave, all on one address, took 190 us at 60k points).
 template <bool IND, int G>
 __global__ __launch_bounds__(256) void k_pair_hash(JoinArgs av, const JoinArgs *__restrict__ ap) {
     const JoinArgs &a = IND ? *ap : av;
@@ -1489,7 +1591,12 @@ __global__ __launch_bounds__(256) void k_pair_hash(JoinArgs av, const JoinArgs *
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
-    if ((threadIdx.x & 63) == 0 && h) atomicAdd(a.hash, (unsigned long long)h);
+    __shared__ uint64_t sh[4];
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = h;
+    __syncthreads();
+    h = sh[0] + sh[1] + sh[2] + sh[3];
+    if (threadIdx.x == 0 && h)
+        atomicAdd(a.stats + (xcc_id() % kStatSlots) * (kLineWords / 2) + kStatHash, (unsigned long long)h);
 }
 
 hegj_status launch_pair_hash(const JoinArgs &a, uint64_t pairs_hint, hipStream_t s, const JoinArgs *dev_args) {
