@@ -135,6 +135,10 @@ hegj_status radix_sort_u64(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
 hegj_status radix_sort_u32(uint32_t *keys, uint32_t *vals, uint32_t *keys_alt,
                            uint32_t *vals_alt, uint32_t n, int bits, hipStream_t s);
 
+// The same without values, for keys made of two `bits`-bit numbers at bits 0
+// and 32 (the digits between and above them are skipped).
+hegj_status radix_sort_pairs(uint64_t *keys, uint64_t *keys_alt, uint32_t n, int bits, hipStream_t s);
+
 // Arguments of the join kernel (hegj_join.hip).
 constexpr int kMaxParts = 8;   // one unit range (queue) per XCD
 // Atomics on one address are served one after the other, ~12 ns each (a pair

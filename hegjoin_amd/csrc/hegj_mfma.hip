@@ -433,45 +433,59 @@ __global__ __launch_bounds__(256) void k_gb_recheck(const uint64_t *__restrict__
     if (ok) pairs[b + lanes_below(m)] = key;
 }
 
-// Sorted pair keys -> neighbour rows: per-position counts.
-__global__ __launch_bounds__(256) void k_gb_count(const uint64_t *__restrict__ keys, uint64_t np,
-                                                  uint32_t *__restrict__ cnt) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < np) atomicAdd(&cnt[(uint32_t)(keys[i] >> 32)], 1u);
-}
-
+// Neighbour ids in sorted key order, and the pair hash: one atomic per
+// workgroup of a grid-stride pass (one per wave, all on one address, took
+// 9.9 ms for 53M pairs; the pass itself takes 0.4).
 __global__ __launch_bounds__(256) void k_gb_emit(const uint64_t *__restrict__ keys, uint64_t np,
                                                  const uint32_t *__restrict__ ila,
                                                  uint32_t *__restrict__ out,
                                                  unsigned long long *hash) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    __shared__ uint64_t sh[4];
     uint64_t h = 0;
-    if (i < np) {
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < np; i += (uint64_t)gridDim.x * 256) {
         const uint64_t k = keys[i];
         const uint32_t qid = ila[(uint32_t)(k >> 32)], cid = ila[(uint32_t)k];
         out[i] = cid;
-        h = mix64(((uint64_t)qid << 32) | cid);
+        h += mix64(((uint64_t)qid << 32) | cid);
     }
     for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
-    if ((threadIdx.x & 63) == 0 && h) atomicAdd(hash, (unsigned long long)h);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = h;
+    __syncthreads();
+    h = sh[0] + sh[1] + sh[2] + sh[3];
+    if (threadIdx.x == 0 && h) atomicAdd(hash, (unsigned long long)h);
 }
 
-__global__ __launch_bounds__(256) void k_gb_rows(const uint32_t *__restrict__ cnt,
-                                                 const uint64_t *__restrict__ start, uint32_t n,
-                                                 const uint32_t *__restrict__ ila, uint64_t base,
+// First index in [lo, hi) of the sorted keys with keys[i] >= v.
+__device__ __forceinline__ uint64_t key_bound(const uint64_t *__restrict__ keys, uint64_t lo, uint64_t hi, uint64_t v) {
+    while (lo < hi) {
+        const uint64_t mid = (lo + hi) >> 1;
+        if (keys[mid] < v)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// Row of each query position in the sorted keys: its start by binary search,
+// its end by doubling steps from there (a count per pair by atomics took 3.2
+// ms for 53M pairs of 2M rows).
+__global__ __launch_bounds__(256) void k_gb_rows(const uint64_t *__restrict__ keys, uint64_t np, uint32_t n,
+                                                 const uint32_t *__restrict__ ila,
                                                  uint64_t *__restrict__ row_off,
                                                  uint32_t *__restrict__ row_cnt) {
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     if (p >= n) return;
+    const uint64_t lo = key_bound(keys, 0, np, (uint64_t)p << 32), next = ((uint64_t)p + 1) << 32;
+    uint64_t step = 16, at = lo;
+    while (at + step < np && keys[at + step] < next) {
+        at += step;
+        step *= 2;
+    }
+    const uint64_t hi = key_bound(keys, at, at + step < np ? at + step : np, next);
     const uint32_t q = ila[p];
-    row_off[q] = base + start[p];
-    row_cnt[q] = cnt[p];
-}
-
-__global__ __launch_bounds__(256) void k_u32_u64(const uint32_t *__restrict__ in, uint32_t n,
-                                                 uint64_t *__restrict__ out) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = in[i];
+    row_off[q] = lo;
+    row_cnt[q] = (uint32_t)(hi - lo);
 }
 
 template <int KB>
@@ -692,27 +706,12 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
         int qbits = 0;
         while (qbits < 32 && ((uint64_t)n >> qbits) != 0) qbits++;
         uint64_t *keys_alt;
-        uint32_t *vals, *vals_alt;
         HIP_TRY(it.get(&keys_alt, ntot + 1));
-        HIP_TRY(it.get(&vals, ntot + 1));
-        HIP_TRY(it.get(&vals_alt, ntot + 1));
-        HIP_TRY(hipMemsetAsync(vals, 0, sizeof(uint32_t) * (ntot + 1), s));
-        HEGJ_TRY(radix_sort_u64(pairs, vals, keys_alt, vals_alt, (uint32_t)ntot, 32 + qbits, s));
-        // rows
-        uint32_t *cnt;
-        uint64_t *cnt64, *start;
-        HIP_TRY(it.get(&cnt, n));
-        HIP_TRY(it.get(&cnt64, n));
-        HIP_TRY(it.get(&start, (size_t)n + 1));
-        HIP_TRY(hipMemsetAsync(cnt, 0, sizeof(uint32_t) * n, s));
-        if (nvalid) k_gb_count<<<ceil_div(nvalid, 256), 256, 0, s>>>(pairs, nvalid, cnt);
-        k_u32_u64<<<ceil_div(n, 256), 256, 0, s>>>(cnt, n, cnt64);
-        HIP_TRY(hipGetLastError());
-        HEGJ_TRY(scan_u64(cnt64, start, n, start + n, s));
+        HEGJ_TRY(radix_sort_pairs(pairs, keys_alt, (uint32_t)ntot, qbits, s));
         HIP_TRY(hipMalloc(&out->buf, sizeof(uint32_t) * std::max<uint64_t>(nvalid, 1)));
         if (nvalid)
-            k_gb_emit<<<ceil_div(nvalid, 256), 256, 0, s>>>(pairs, nvalid, ix.ila, out->buf, out->hash);
-        k_gb_rows<<<ceil_div(n, 256), 256, 0, s>>>(cnt, start, n, ix.ila, 0, out->row_off, out->row_cnt);
+            k_gb_emit<<<std::min<uint32_t>(ceil_div(nvalid, 256), 2048), 256, 0, s>>>(pairs, nvalid, ix.ila, out->buf, out->hash);
+        k_gb_rows<<<ceil_div(n, 256), 256, 0, s>>>(pairs, nvalid, n, ix.ila, out->row_off, out->row_cnt);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(s));
         out->pairs = nvalid;

@@ -137,7 +137,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const K *__restrict__ ke
     hist[(uint64_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
 }
 
-template <typename K>
+// VALS: 32-bit values travel with the keys.
+template <typename K, bool VALS>
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K *__restrict__ keys,
                                                            const uint32_t *__restrict__ vals,
                                                            K *__restrict__ okeys,
@@ -156,7 +157,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K *__restrict__
         uint64_t p = base + i * kRsThreads + threadIdx.x;
         bool valid = p < n;
         K key = valid ? keys[p] : K(0);
-        uint32_t val = valid ? vals[p] : 0u;
+        uint32_t val = VALS && valid ? vals[p] : 0u;
         uint32_t d = (uint32_t)(key >> shift) & 255u;
         uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K *__restrict__
             uint32_t off = run[d] + rank;
             for (int w = 0; w < wid; w++) off += wcnt[w][d];
             okeys[off] = key;
-            ovals[off] = val;
+            if (VALS) ovals[off] = val;
         }
         __syncthreads();
         uint32_t add = 0;
@@ -185,31 +186,32 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K *__restrict__
     (void)lane;
 }
 
-template <typename K>
+// One pass per 8 bits of the key bits [0, bits) and [bits2, bits2 + n2).
+template <typename K, bool VALS>
 hegj_status radix_impl(K *keys, uint32_t *vals, K *keys_alt, uint32_t *vals_alt, uint32_t n,
-                       int bits, hipStream_t s) {
-    if (n <= 1 || bits <= 0) return HEGJ_OK;
+                       int bits, int bits2, int n2, hipStream_t s) {
+    if (n <= 1 || bits + n2 <= 0) return HEGJ_OK;
     uint32_t tiles = ceil_div(n, kRsTile);
     Scratch sc;
     uint32_t *hist;
     HIP_TRY(sc.get(&hist, (size_t)tiles * 256));
     K *src_k = keys, *dst_k = keys_alt;
     uint32_t *src_v = vals, *dst_v = vals_alt;
-    int passes = (bits + 7) / 8;
+    const int low = (bits + 7) / 8, passes = low + (n2 + 7) / 8;
     for (int p = 0; p < passes; p++) {
-        int shift = p * 8;
+        const int shift = p < low ? p * 8 : bits2 + (p - low) * 8;
         k_rs_hist<K><<<tiles, kRsThreads, 0, s>>>(src_k, n, shift, hist, tiles);
         HIP_TRY(hipGetLastError());
         HEGJ_TRY(scan_u32(hist, hist, tiles * 256, nullptr, s));
-        k_rs_scatter<K><<<tiles, kRsThreads, 0, s>>>(src_k, src_v, dst_k, dst_v, n, shift, hist,
-                                                     tiles);
+        k_rs_scatter<K, VALS><<<tiles, kRsThreads, 0, s>>>(src_k, src_v, dst_k, dst_v, n, shift, hist,
+                                                           tiles);
         HIP_TRY(hipGetLastError());
         std::swap(src_k, dst_k);
         std::swap(src_v, dst_v);
     }
     if (src_k != keys) {
         HIP_TRY(hipMemcpyAsync(keys, src_k, sizeof(K) * n, hipMemcpyDeviceToDevice, s));
-        HIP_TRY(hipMemcpyAsync(vals, src_v, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
+        if (VALS) HIP_TRY(hipMemcpyAsync(vals, src_v, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
     }
     HIP_TRY(hipStreamSynchronize(s));
     return HEGJ_OK;
@@ -229,12 +231,16 @@ hegj_status scan_u64(const uint64_t *in, uint64_t *out, uint32_t n, uint64_t *d_
 
 hegj_status radix_sort_u64(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
                            uint32_t *vals_alt, uint32_t n, int bits, hipStream_t s) {
-    return radix_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, bits, s);
+    return radix_impl<uint64_t, true>(keys, vals, keys_alt, vals_alt, n, bits, 0, 0, s);
+}
+
+hegj_status radix_sort_pairs(uint64_t *keys, uint64_t *keys_alt, uint32_t n, int bits, hipStream_t s) {
+    return radix_impl<uint64_t, false>(keys, nullptr, keys_alt, nullptr, n, bits, 32, bits, s);
 }
 
 hegj_status radix_sort_u32(uint32_t *keys, uint32_t *vals, uint32_t *keys_alt,
                            uint32_t *vals_alt, uint32_t n, int bits, hipStream_t s) {
-    return radix_impl<uint32_t>(keys, vals, keys_alt, vals_alt, n, bits, s);
+    return radix_impl<uint32_t, true>(keys, vals, keys_alt, vals_alt, n, bits, 0, 0, s);
 }
 
 }  // namespace hegj
