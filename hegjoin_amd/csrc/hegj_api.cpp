@@ -5,6 +5,7 @@
 // here only sizes buffers, launches kernels on the handle's stream and reads
 // back scalars; every per-point and per-pair step runs on the device.
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -46,47 +47,116 @@ static bool in_arena(const void *p) {
     return g_arena && (const char *)p >= g_arena->base && (const char *)p < g_arena->base + g_arena->cap;
 }
 
+static thread_local CallScope *g_scope = nullptr;
+
+CallScope::CallScope(hipStream_t s) : stream(s), active(g_scope == nullptr && g_arena == nullptr) {
+    if (active) g_scope = this;
+}
+
+CallScope::~CallScope() {
+    if (!active) return;
+    g_scope = nullptr;
+    if (ptrs.empty()) return;
+    (void)hipStreamSynchronize(stream);
+    for (void *p : ptrs) dev_free(p);
+}
+
+bool scratch_outlives() { return g_scope != nullptr || g_arena != nullptr; }
+
+hegj_status scratch_done(hipStream_t s) {
+    if (!scratch_outlives()) HIP_TRY(hipStreamSynchronize(s));
+    return HEGJ_OK;
+}
+
 hipError_t Scratch::alloc(void **p, size_t bytes) {
     if (g_arena) return arena_alloc(p, bytes);
+    if (g_scope) {
+        hipError_t e = dev_malloc(p, bytes);
+        if (e == hipSuccess) {
+            g_scope->ptrs.push_back(*p);
+            ptrs.push_back(*p);
+            scoped = true;
+        }
+        return e;
+    }
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipSuccess) ptrs.push_back(*p);
     return e;
 }
 
+hegj_status Scratch::drop(hipStream_t s) {
+    HIP_TRY(hipStreamSynchronize(s));
+    for (void *p : ptrs) {
+        if (scoped) {
+            auto &v = g_scope->ptrs;
+            v.erase(std::remove(v.begin(), v.end(), p), v.end());
+            dev_free(p);
+        } else {
+            (void)hipFree(p);
+        }
+    }
+    ptrs.clear();
+    return HEGJ_OK;
+}
+
 Scratch::~Scratch() {
-    for (void *p : ptrs) (void)hipFree(p);
+    if (!scoped)
+        for (void *p : ptrs) (void)hipFree(p);
 }
 
 namespace {
+// Freed device buffers by (device, size), each with the tick it was freed at.
+struct Cached {
+    void *p;
+    uint64_t tick;
+};
 std::mutex g_cache_mu;
-std::map<void *, std::pair<int, size_t>> g_cache_live;           // ptr -> (device, size)
-std::multimap<std::pair<int, size_t>, void *> g_cache_free;      // (device, size) -> ptr
+std::map<void *, std::pair<int, size_t>> g_cache_live;          // ptr -> (device, size)
+std::multimap<std::pair<int, size_t>, Cached> g_cache_free;
 size_t g_cache_bytes = 0;
+uint64_t g_cache_tick = 0;
 constexpr size_t kCacheCap = 16ull << 30;
 
+// Sizes are rounded up to an eighth of their power of two (256 bytes at
+// least), so calls of similar sizes find each other's buffers.
 size_t cache_round(size_t b) {
-    if (b <= ((size_t)1 << 20)) {
-        size_t s = 256;
-        while (s < b) s <<= 1;
-        return s;
+    size_t g = 256;
+    while (g * 16 <= b) g <<= 1;
+    return std::max<size_t>((b + g - 1) / g * g, 256);
+}
+
+// Takes cached buffers of one device (dev >= 0: all of it) or, for dev < 0,
+// the longest unused ones until at most `keep` bytes are held.
+std::vector<void *> cache_take(int dev, size_t keep) {
+    std::vector<void *> rel;
+    if (dev >= 0) {
+        for (auto it = g_cache_free.begin(); it != g_cache_free.end();) {
+            if (it->first.first != dev) {
+                ++it;
+                continue;
+            }
+            rel.push_back(it->second.p);
+            g_cache_bytes -= it->first.second;
+            it = g_cache_free.erase(it);
+        }
+        return rel;
     }
-    const size_t g = (size_t)2 << 20;
-    return (b + g - 1) / g * g;
+    while (g_cache_bytes > keep && !g_cache_free.empty()) {
+        auto old = g_cache_free.begin();
+        for (auto it = g_cache_free.begin(); it != g_cache_free.end(); ++it)
+            if (it->second.tick < old->second.tick) old = it;
+        rel.push_back(old->second.p);
+        g_cache_bytes -= old->first.second;
+        g_cache_free.erase(old);
+    }
+    return rel;
 }
 
 void cache_release(int dev) {
     std::vector<void *> rel;
     {
         std::lock_guard<std::mutex> lk(g_cache_mu);
-        for (auto it = g_cache_free.begin(); it != g_cache_free.end();) {
-            if (it->first.first == dev) {
-                rel.push_back(it->second);
-                g_cache_bytes -= it->first.second;
-                it = g_cache_free.erase(it);
-            } else {
-                ++it;
-            }
-        }
+        rel = cache_take(dev, 0);
     }
     for (void *p : rel) (void)hipFree(p);
 }
@@ -101,13 +171,14 @@ hipError_t dev_malloc(void **p, size_t bytes) {
     if (e != hipSuccess) return e;
     const size_t rs = cache_round(bytes);
     {
+        // the smallest cached buffer that holds it, if not over a quarter larger
         std::lock_guard<std::mutex> lk(g_cache_mu);
-        auto it = g_cache_free.find({dev, rs});
-        if (it != g_cache_free.end()) {
-            *p = it->second;
+        auto it = g_cache_free.lower_bound({dev, rs});
+        if (it != g_cache_free.end() && it->first.first == dev && it->first.second <= rs + rs / 4) {
+            *p = it->second.p;
+            g_cache_bytes -= it->first.second;
+            g_cache_live[*p] = it->first;
             g_cache_free.erase(it);
-            g_cache_bytes -= rs;
-            g_cache_live[*p] = {dev, rs};
             return hipSuccess;
         }
     }
@@ -126,20 +197,164 @@ hipError_t dev_malloc(void **p, size_t bytes) {
 
 void dev_free(void *p) {
     if (!p || in_arena(p)) return;
+    std::vector<void *> rel;
     {
         std::lock_guard<std::mutex> lk(g_cache_mu);
         auto it = g_cache_live.find(p);
-        if (it != g_cache_live.end()) {
+        if (it == g_cache_live.end() || it->second.second > kCacheCap) {
+            if (it != g_cache_live.end()) g_cache_live.erase(it);
+            rel.push_back(p);
+        } else {
             const auto key = it->second;
             g_cache_live.erase(it);
-            if (g_cache_bytes + key.second <= kCacheCap) {
-                g_cache_free.insert({key, p});
-                g_cache_bytes += key.second;
+            // over the bound the longest unused buffers go, not the newest
+            if (g_cache_bytes + key.second > kCacheCap) rel = cache_take(-1, kCacheCap - key.second);
+            g_cache_free.insert({key, Cached{p, g_cache_tick++}});
+            g_cache_bytes += key.second;
+        }
+    }
+    for (void *q : rel) (void)hipFree(q);
+}
+
+// ---- pinned host memory and events, kept for reuse --------------------------
+// Both pools are process-wide and bounded; what exceeds the bound is freed.
+namespace {
+constexpr size_t kPinnedSmall = 16u << 10, kPinnedChunk = 4u << 20;
+constexpr size_t kPinnedSmallMax = 32, kPinnedChunkMax = 8;  // 32 MiB of chunks
+constexpr size_t kEventsMax = 64;                            // per device
+std::mutex g_pin_mu;
+std::vector<void *> g_pin_small, g_pin_chunk;
+std::map<int, std::vector<hipEvent_t>> g_events;
+
+struct Pinned {
+    void *p = nullptr;
+    bool chunk;
+    explicit Pinned(bool chunk_) : chunk(chunk_) {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        auto &v = chunk ? g_pin_chunk : g_pin_small;
+        if (!v.empty()) {
+            p = v.back();
+            v.pop_back();
+        }
+    }
+    hipError_t get() {
+        if (p) return hipSuccess;
+        if (g_arena) return hipErrorOutOfMemory;  // code that must not allocate
+        return hipHostMalloc(&p, chunk ? kPinnedChunk : kPinnedSmall, hipHostMallocPortable);
+    }
+    ~Pinned() {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lk(g_pin_mu);
+            auto &v = chunk ? g_pin_chunk : g_pin_small;
+            if (v.size() < (chunk ? kPinnedChunkMax : kPinnedSmallMax)) {
+                v.push_back(p);
                 return;
             }
         }
+        (void)hipHostFree(p);
     }
-    (void)hipFree(p);
+};
+
+hipEvent_t event_get(int dev) {
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        auto &v = g_events[dev];
+        if (!v.empty()) {
+            hipEvent_t e = v.back();
+            v.pop_back();
+            return e;
+        }
+    }
+    hipEvent_t e = nullptr;
+    return hipEventCreate(&e) == hipSuccess ? e : nullptr;
+}
+
+void event_put(int dev, hipEvent_t e) {
+    if (!e) return;
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        auto &v = g_events[dev];
+        if (v.size() < kEventsMax) {
+            v.push_back(e);
+            return;
+        }
+    }
+    (void)hipEventDestroy(e);
+}
+}  // namespace
+
+void pinned_release() {
+    std::vector<void *> rel;
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        rel.swap(g_pin_small);
+        rel.insert(rel.end(), g_pin_chunk.begin(), g_pin_chunk.end());
+        g_pin_chunk.clear();
+    }
+    for (void *p : rel) (void)hipHostFree(p);
+}
+
+hegj_status read_back_bytes(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    Pinned pin(false);
+    if (bytes > kPinnedSmall || pin.get() != hipSuccess) {
+        (void)hipGetLastError();
+        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return HEGJ_OK;
+    }
+    HIP_TRY(hipMemcpyAsync(pin.p, src, bytes, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    std::memcpy(dst, pin.p, bytes);
+    return HEGJ_OK;
+}
+
+hegj_status copy_to_host(void *dst, const void *src, size_t bytes, int device, hipStream_t s) {
+    // Below 4 MiB starting threads costs more than they save (2.7 MB: 0.15 ms
+    // the plain way, 0.25 in chunks).  Above, one thread per 2 MiB up to eight,
+    // two chunks each at least.
+    if (bytes <= kPinnedSmall) return read_back_bytes(dst, src, bytes, s);
+    if (bytes < ((size_t)4 << 20)) {
+        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return HEGJ_OK;
+    }
+    const size_t threads = std::min<size_t>({bytes >> 21, 8, std::max(1u, std::thread::hardware_concurrency())});
+    size_t chunk = (bytes / (threads * 2) + 0xFFFF) & ~(size_t)0xFFFF;
+    chunk = std::max<size_t>((size_t)1 << 20, std::min(chunk, kPinnedChunk));
+    const size_t n = (bytes + chunk - 1) / chunk;
+    std::atomic<int> bad{0};
+    // Thread t moves chunks t, t + threads, ..: while it copies one out, the
+    // other threads' transfers keep the link busy.
+    auto work = [&](size_t t) {
+        Pinned pin(true);
+        hipEvent_t ev = nullptr;
+        hipError_t e = t ? hipSetDevice(device) : hipSuccess;
+        if (e == hipSuccess) e = pin.get();
+        if (e == hipSuccess && !(ev = event_get(device))) e = hipErrorUnknown;
+        for (size_t c = t; e == hipSuccess && c < n; c += threads) {
+            const size_t at = c * chunk, len = std::min(chunk, bytes - at);
+            e = hipMemcpyAsync(pin.p, static_cast<const char *>(src) + at, len, hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(ev, s);
+            if (e == hipSuccess) e = hipEventSynchronize(ev);
+            if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + at, pin.p, len);
+        }
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(s);  // nothing may still write the pinned chunk
+            (void)hipGetLastError();
+            bad.store((int)e);
+        }
+        event_put(device, ev);
+    };
+    std::vector<std::thread> pool;
+    for (size_t t = 1; t < std::min(threads, n); t++) pool.emplace_back(work, t);
+    work(0);
+    for (auto &t : pool) t.join();
+    if (bad.load()) {  // no pinned memory or a failed transfer: the plain way
+        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
+    return HEGJ_OK;
 }
 
 // S7: largest s with RN(sqrt(s)) <= eps.  sqrt is monotone, so
@@ -164,21 +379,27 @@ float sqrt_threshold_f(float eps) {
 struct EventTimer {
     hipEvent_t a = nullptr, b = nullptr;
     hipStream_t s;
+    int dev = 0;
     explicit EventTimer(hipStream_t st) : s(st) {
-        (void)hipEventCreate(&a);
-        (void)hipEventCreate(&b);
+        (void)hipGetDevice(&dev);
+        a = event_get(dev);
+        b = event_get(dev);
         (void)hipEventRecord(a, s);
     }
-    float stop() {
-        float ms = 0;
-        (void)hipEventRecord(b, s);
+    void mark() { (void)hipEventRecord(b, s); }  // the interval's end
+    float ms() {                                 // after the stream has drained past it
+        float v = 0;
         (void)hipEventSynchronize(b);
-        (void)hipEventElapsedTime(&ms, a, b);
-        return ms;
+        (void)hipEventElapsedTime(&v, a, b);
+        return v;
+    }
+    float stop() {
+        mark();
+        return ms();
     }
     ~EventTimer() {
-        if (a) (void)hipEventDestroy(a);
-        if (b) (void)hipEventDestroy(b);
+        event_put(dev, a);
+        event_put(dev, b);
     }
 };
 
@@ -223,22 +444,16 @@ struct hegj_result {
     std::vector<uint32_t *> batches;
     std::vector<uint64_t> bases;  // global offset of each batch
     uint64_t *d_row_off = nullptr;
-    uint32_t *d_row_cnt = nullptr;
+    uint32_t *d_row_cnt = nullptr;  // behind d_row_off, in the same buffer
     hegj_result_info info{};
     bool hybrid = false;        // made by hegj_selfjoin_hybrid
     hegj_hybrid_info hinfo{};
-    hipEvent_t done = nullptr;  // recorded when the join handed the result out
+    bool done = false;  // its rows are complete (the join's stream drained)
     ~hegj_result() {
         // the buffers go back to the cache: nothing may still be writing them
-        if (done) {
-            (void)hipEventSynchronize(done);
-            (void)hipEventDestroy(done);
-        } else if (idx && idx->stream) {
-            (void)hipStreamSynchronize(idx->stream);  // failed inside the join
-        }
+        if (!done && idx && idx->stream) (void)hipStreamSynchronize(idx->stream);  // failed inside the join
         for (uint32_t *b : batches) dev_free(b);
         dev_free(d_row_off);
-        dev_free(d_row_cnt);
     }
 };
 
@@ -292,7 +507,11 @@ hegj_status new_index(const hegj_index_opts *o, hegj_index **out, F fill) {
     h->device = o->device;
     HEGJ_TRY(set_device(o->device));
     HIP_TRY(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-    hegj_status s = fill(h.get());
+    hegj_status s;
+    {
+        CallScope scope(h->stream);
+        s = fill(h.get());
+    }
     if (s != HEGJ_OK) {
         std::string msg = g_last_error;
         hegj_index_free(h.release());
@@ -306,8 +525,8 @@ hegj_status new_index(const hegj_index_opts *o, hegj_index **out, F fill) {
 hegj_status ensure_workload(hegj_index *h) {
     if (h->have_workload) return HEGJ_OK;
     const uint32_t C = h->ix.C;
-    HIP_TRY(hipMalloc(&h->d_work, sizeof(uint32_t) * (C + 1)));
-    HIP_TRY(hipMalloc(&h->d_order, sizeof(uint32_t) * (C + 1)));
+    HIP_TRY(dev_malloc_n(&h->d_work, (size_t)C + 1));
+    HIP_TRY(dev_malloc_n(&h->d_order, (size_t)C + 1));
     EventTimer t(h->stream);
     HEGJ_TRY(launch_workload(h->g, h->ix, h->d_work, h->stream));
     HEGJ_TRY(workload_order(h->ix, h->d_work, h->d_order, &h->total_candidates, h->stream));
@@ -338,7 +557,7 @@ struct Counters {
 
 hegj_status ensure_morton(hegj_index *h) {
     if (h->d_morton) return HEGJ_OK;
-    HIP_TRY(hipMalloc(&h->d_morton, sizeof(uint32_t) * (h->ix.C + 1)));
+    HIP_TRY(dev_malloc_n(&h->d_morton, (size_t)h->ix.C + 1));
     return morton_order(h->g, h->ix, h->d_morton, &h->morton_ok, h->stream);
 }
 
@@ -383,6 +602,7 @@ namespace {
 
 hegj_status ensure_soa32(hegj_index *h) {
     if (h->soa32) return HEGJ_OK;
+    CallScope scope(h->stream);
     return make_soa32(h->g, h->ix, &h->soa32, &h->aos32, &h->f32_radius, &h->f32_centre, h->stream);
 }
 
@@ -419,6 +639,14 @@ struct JoinPlan {
             dev_free(p);
     }
 };
+
+// The result's row table, cleared (silenced queries have no row).
+hegj_status alloc_rows(hegj_result *r, uint32_t n, hipStream_t s) {
+    HIP_TRY(dev_malloc(reinterpret_cast<void **>(&r->d_row_off), (sizeof(uint64_t) + sizeof(uint32_t)) * (size_t)n));
+    r->d_row_cnt = reinterpret_cast<uint32_t *>(r->d_row_off + n);
+    HIP_TRY(hipMemsetAsync(r->d_row_off, 0, (sizeof(uint64_t) + sizeof(uint32_t)) * (size_t)n, s));
+    return HEGJ_OK;
+}
 
 // About 32 grabs per wave keeps the queue atomics off the critical path.
 uint32_t grab_for(const JoinPlan &P, uint32_t nu) {
@@ -475,6 +703,14 @@ JoinArgs base_args(const hegj_index *h, const hegj_join_opts &opts, const JoinPl
         a.trej32 = P.trej32;
     }
     return a;
+}
+
+// At most 60% of the free device memory for one batch.
+hegj_status cap_to_free(uint64_t *capacity) {
+    size_t free_b = 0, total_b = 0;
+    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    *capacity = std::min<uint64_t>(*capacity, (uint64_t)(free_b * 0.6) / sizeof(uint32_t));
+    return HEGJ_OK;
 }
 
 // all_cells: units also for the cells the cell-0 wrap silences (the hybrid
@@ -535,8 +771,7 @@ hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, co
         set_parts(e, 1, &one_end);
         HEGJ_TRY(launch_join(e, qb, blocks_for(P, ns, e.units_per_grab), s));
         Counters c;
-        HIP_TRY(hipMemcpyAsync(&c, P.d_ctr, sizeof(c), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HEGJ_TRY(read_back(&c, P.d_ctr, s));
         const double est = (double)c.sum(kStatPairs) * ((double)U / (double)ns);
         P.estimated_pairs = (uint64_t)est;
         const uint32_t nb = opts.batches ? opts.batches : 1u;
@@ -553,9 +788,8 @@ hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, co
                 P.capacity += (uint64_t)(est * 0.15 + waves * chunk);
             }
         }
-        size_t free_b = 0, total_b = 0;
-        HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-        P.capacity = std::min<uint64_t>(P.capacity, (uint64_t)(free_b * 0.6) / sizeof(uint32_t));
+        // small batches are cut to the free memory only when they do not fit
+        if (P.capacity > (64u << 20)) HEGJ_TRY(cap_to_free(&P.capacity));
         P.estimate_ms = t.stop();
     }
     if (P.capacity == 0) P.capacity = 1;
@@ -580,6 +814,7 @@ struct BatchRunner {
     JoinArgs a{};
     uint64_t base = 0, capacity = 0, used = 0;
     bool open = false;
+    bool cleared = false;  // the counters are all zero (nothing ran since init)
     double join_ms = 0;
     uint32_t launches = 0;
     Counters c{};
@@ -593,14 +828,12 @@ struct BatchRunner {
         r->info.n_units = P.U;
         r->info.estimate_ms = P.estimate_ms;
         r->info.estimated_pairs = P.estimated_pairs;
-        HIP_TRY(dev_malloc_n(&r->d_row_off, n));
-        HIP_TRY(dev_malloc_n(&r->d_row_cnt, n));
-        HIP_TRY(hipMemsetAsync(r->d_row_off, 0, sizeof(uint64_t) * n, s));
-        HIP_TRY(hipMemsetAsync(r->d_row_cnt, 0, sizeof(uint32_t) * n, s));
+        HEGJ_TRY(alloc_rows(r, n, s));
         a = base_args(h, opts, P);
         a.row_off = r->d_row_off;
         a.row_cnt = r->d_row_cnt;
         HIP_TRY(hipMemsetAsync(P.d_ctr, 0, sizeof(Counters), s));
+        cleared = true;
         capacity = P.capacity;
         return HEGJ_OK;
     }
@@ -609,11 +842,18 @@ struct BatchRunner {
         if (r->batches.size() >= (size_t)kMaxBatches)
             return fail(HEGJ_ERR_CAPACITY, "result needs more than 64 batches");
         uint32_t *buf = nullptr;
-        HIP_TRY(dev_malloc_n(&buf, capacity));
+        hipError_t e = dev_malloc_n(&buf, capacity);
+        if (e == hipErrorOutOfMemory && !opts.result_capacity) {
+            (void)hipGetLastError();
+            HEGJ_TRY(cap_to_free(&capacity));
+            capacity = std::max<uint64_t>(capacity, 1);
+            e = dev_malloc_n(&buf, capacity);
+        }
+        HIP_TRY(e);
         r->batches.push_back(buf);
         r->bases.push_back(base);
         // the batch cursor starts at zero (hash / evals / pairs accumulate)
-        HIP_TRY(hipMemsetAsync(&P.d_ctr->cursor, 0, sizeof(P.d_ctr->cursor), h->stream));
+        if (!cleared) HIP_TRY(hipMemsetAsync(&P.d_ctr->cursor, 0, sizeof(P.d_ctr->cursor), h->stream));
         a.out = buf;
         a.out_base = base;
         a.capacity = capacity;
@@ -637,7 +877,8 @@ struct BatchRunner {
             if (!open) HEGJ_TRY(open_batch());
             const uint64_t before = used;
             // queue heads and the deferral count restart; the cursor continues
-            HIP_TRY(hipMemsetAsync(P.d_ctr, 0, offsetof(Counters, cursor), s));
+            if (!cleared) HIP_TRY(hipMemsetAsync(P.d_ctr, 0, offsetof(Counters, cursor), s));
+            cleared = false;
             a.units = cur;
             a.n_units = cur_n;
             a.units_per_grab = opts.units_per_grab ? opts.units_per_grab : grab_for(P, cur_n);
@@ -654,12 +895,12 @@ struct BatchRunner {
             {
                 EventTimer t(s);
                 HEGJ_TRY(launch_join(a, qb, blocks_for(P, cur_n, a.units_per_grab), s));
-                join_ms += t.stop();
+                t.mark();
+                if (last) HEGJ_TRY(launch_pair_hash(a, capacity, s));
+                HEGJ_TRY(read_back(&c, P.d_ctr, s));
+                join_ms += t.ms();
                 launches++;
             }
-            if (last) HEGJ_TRY(launch_pair_hash(a, capacity, s));
-            HIP_TRY(hipMemcpyAsync(&c, P.d_ctr, sizeof(c), hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
             if (c.sum(kStatMismatch))
                 return fail(HEGJ_ERR_HIP, "join: the write pass of " + std::to_string(c.sum(kStatMismatch)) +
                                               " work units disagreed with their counts");
@@ -705,8 +946,7 @@ struct BatchRunner {
             HIP_TRY(hipMemsetAsync(P.d_ctr2, 0, sizeof(Counters), s));
             HEGJ_TRY(launch_join(e, qb, blocks_for(P, e.n_units, e.units_per_grab), s));
             Counters c2;
-            HIP_TRY(hipMemcpyAsync(&c2, P.d_ctr2, sizeof(c2), hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
+            HEGJ_TRY(read_back(&c2, P.d_ctr2, s));
             if (!opts.result_capacity) {
                 capacity = std::max<uint64_t>(c2.sum(kStatPairs), 1);
                 // a requested batch count keeps every batch at the first one's size
@@ -721,8 +961,7 @@ struct BatchRunner {
         hipStream_t s = h->stream;
         if (open) {
             HEGJ_TRY(close_batch(false));
-            HIP_TRY(hipMemcpyAsync(&c, P.d_ctr, sizeof(c), hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
+            HEGJ_TRY(read_back(&c, P.d_ctr, s));
         }
         r->info.total_neighbors = c.sum(kStatPairs);
         r->info.pair_hash = c.sum(kStatHash);
@@ -1040,10 +1279,7 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
     r->info.n_units = G.P.U;
     r->info.estimate_ms = G.P.estimate_ms;
     r->info.estimated_pairs = G.P.estimated_pairs;
-    HIP_TRY(dev_malloc_n(&r->d_row_off, n));
-    HIP_TRY(dev_malloc_n(&r->d_row_cnt, n));
-    HIP_TRY(hipMemsetAsync(r->d_row_off, 0, sizeof(uint64_t) * n, s));
-    HIP_TRY(hipMemsetAsync(r->d_row_cnt, 0, sizeof(uint32_t) * n, s));
+    HEGJ_TRY(alloc_rows(r, n, s));
     uint32_t *buf = nullptr;
     HIP_TRY(dev_malloc_n(&buf, G.P.capacity));
     r->batches.push_back(buf);
@@ -1126,10 +1362,7 @@ hegj_status selfjoin_mfma(hegj_index *h, const uint32_t *order, uint64_t result_
     else
         HEGJ_TRY(build_units(h->g, h->ix, gb_unit_queries(h->gb.kp / 32), order, &units, &U, s));
     r->info.n_units = U;
-    HIP_TRY(dev_malloc_n(&r->d_row_off, n));
-    HIP_TRY(dev_malloc_n(&r->d_row_cnt, n));
-    HIP_TRY(hipMemsetAsync(r->d_row_off, 0, sizeof(uint64_t) * n, s));
-    HIP_TRY(hipMemsetAsync(r->d_row_cnt, 0, sizeof(uint32_t) * n, s));
+    HEGJ_TRY(alloc_rows(r, n, s));
     unsigned long long *d_hash;
     HIP_TRY(sc.get(&d_hash, 1));
     HIP_TRY(hipMemsetAsync(d_hash, 0, sizeof(*d_hash), s));
@@ -1210,6 +1443,7 @@ void hegj_release_cached_memory(int device) {
         hegj::cache_release_device(device);
         return;
     }
+    hegj::pinned_release();
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess) return;
     for (int d = 0; d < n; d++) hegj::cache_release_device(d);
@@ -1238,7 +1472,7 @@ hegj_status hegj_index_build(const double *database, uint32_t n, double epsilon,
     HEGJ_TRY(check_opts(opts, n, epsilon));
     return new_index(opts, out, [&](hegj_index *h) -> hegj_status {
         size_t bytes = sizeof(double) * (size_t)n * opts->dim;
-        HIP_TRY(hipMalloc(&h->ix.pts, bytes));
+        HIP_TRY(dev_malloc(reinterpret_cast<void **>(&h->ix.pts), bytes));
         HIP_TRY(hipMemcpyAsync(h->ix.pts, database, bytes, hipMemcpyHostToDevice, h->stream));
         return build_common(h, n, epsilon, opts);
     });
@@ -1250,7 +1484,7 @@ hegj_status hegj_index_build_device(const double *dev_database, uint32_t n, doub
     HEGJ_TRY(check_opts(opts, n, epsilon));
     return new_index(opts, out, [&](hegj_index *h) -> hegj_status {
         size_t bytes = sizeof(double) * (size_t)n * opts->dim;
-        HIP_TRY(hipMalloc(&h->ix.pts, bytes));
+        HIP_TRY(dev_malloc(reinterpret_cast<void **>(&h->ix.pts), bytes));
         HIP_TRY(hipMemcpyAsync(h->ix.pts, dev_database, bytes, hipMemcpyDeviceToDevice, h->stream));
         return build_common(h, n, epsilon, opts);
     });
@@ -1261,16 +1495,10 @@ hegj_status hegj_index_free(hegj_index *h) {
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     free_index(&h->ix);
-    if (h->d_work) (void)hipFree(h->d_work);
-    if (h->d_order) (void)hipFree(h->d_order);
-    if (h->d_morton) (void)hipFree(h->d_morton);
-    if (h->gb.A) (void)hipFree(h->gb.A);
-    if (h->gb.B) (void)hipFree(h->gb.B);
-    if (h->gb.w) (void)hipFree(h->gb.w);
+    for (void *p : {(void *)h->d_work, (void *)h->d_order, (void *)h->d_morton, (void *)h->gb.A, (void *)h->gb.B,
+                    (void *)h->gb.w, (void *)h->soa32, (void *)h->aos32, (void *)h->f32_centre})
+        dev_free(p);
     if (h->gplan) free_graph_plan(h->gplan);
-    if (h->soa32) (void)hipFree(h->soa32);
-    if (h->aos32) (void)hipFree(h->aos32);
-    if (h->f32_centre) (void)hipFree(h->f32_centre);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
     return HEGJ_OK;
@@ -1318,8 +1546,7 @@ hegj_status hegj_index_copy_grid(const hegj_index *h, hegj_grid *index,
         }
     }
     if (ila) {
-        HIP_TRY(hipMemcpyAsync(ila, h->ix.ila, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
+        HEGJ_TRY(copy_to_host(ila, h->ix.ila, sizeof(uint32_t) * n, h->device, h->stream));
     }
     return HEGJ_OK;
 }
@@ -1337,6 +1564,7 @@ hegj_status hegj_sort_by_workload(hegj_index *h, hegj_scheduling_cell *sorted, u
                                   uint64_t *total_candidates) {
     if (!h) return fail(HEGJ_ERR_INVALID_ARG, "NULL index");
     HEGJ_TRY(set_device(h->device));
+    CallScope scope(h->stream);
     HEGJ_TRY(ensure_workload(h));
     const uint32_t C = h->ix.C, n = h->g.n;
     if (total_candidates) *total_candidates = h->total_candidates;
@@ -1427,8 +1655,8 @@ hegj_status hegj_tuning_load(const char *path, uint32_t *n_loaded) {
 }
 
 static hegj_status mark_done(hegj_result *r, hipStream_t s) {
-    HIP_TRY(hipEventCreateWithFlags(&r->done, hipEventDisableTiming));
-    HIP_TRY(hipEventRecord(r->done, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    r->done = true;
     return HEGJ_OK;
 }
 
@@ -1460,6 +1688,7 @@ hegj_status hegj_selfjoin(hegj_index *h, const hegj_join_opts *opts_in, hegj_res
     hipStream_t s = h->stream;
     const uint32_t n = h->g.n;
 
+    CallScope scope(s);
     std::unique_ptr<hegj_result> r(new hegj_result());
     r->idx = h;
     HEGJ_TRY(ensure_workload(h));
@@ -1706,6 +1935,7 @@ hegj_status hegj_selfjoin_hybrid(hegj_index *h, const hegj_join_opts *opts_in,
     if (qb != 4 && qb != 8 && qb != 16) return fail(HEGJ_ERR_INVALID_ARG, "queries_per_unit must be 4, 8 or 16");
     if (!valid_waves_batches(opts))
         return fail(HEGJ_ERR_INVALID_ARG, "block_waves must be 0, 1, 2 or 4 and batches at most 32");
+    CallScope scope(h->stream);
     std::unique_ptr<hegj_result> r(new hegj_result());
     r->idx = h;
     HEGJ_TRY(ensure_workload(h));
@@ -1773,11 +2003,7 @@ hegj_status hegj_result_get_info(const hegj_result *r, hegj_result_info *info) {
 hegj_status hegj_result_copy_counts(const hegj_result *r, uint32_t *counts) {
     if (!r || !counts) return fail(HEGJ_ERR_INVALID_ARG, "NULL argument");
     HEGJ_TRY(set_device(r->idx->device));
-    hipStream_t s = r->idx->stream;
-    HIP_TRY(hipMemcpyAsync(counts, r->d_row_cnt, sizeof(uint32_t) * r->idx->g.n,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return copy_to_host(counts, r->d_row_cnt, sizeof(uint32_t) * r->idx->g.n, r->idx->device, r->idx->stream);
 }
 
 hegj_status hegj_result_copy_csr(const hegj_result *r, uint64_t *offsets, uint32_t *nbrs,
@@ -1786,19 +2012,19 @@ hegj_status hegj_result_copy_csr(const hegj_result *r, uint64_t *offsets, uint32
     HEGJ_TRY(set_device(r->idx->device));
     hipStream_t s = r->idx->stream;
     const uint32_t n = r->idx->g.n;
+    const int dev = r->idx->device;
+    CallScope scope(s);
     Scratch sc;
     uint64_t *d_off;
     HIP_TRY(sc.get(&d_off, (size_t)n + 1));
     HEGJ_TRY(csr_offsets(r->d_row_cnt, n, d_off, s));
-    HIP_TRY(hipMemcpyAsync(offsets, d_off, sizeof(uint64_t) * (n + 1), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    const uint64_t total = offsets[n];
-    if (!nbrs || total == 0) return HEGJ_OK;
+    const uint64_t total = r->info.total_neighbors;
+    if (!nbrs || total == 0) return copy_to_host(offsets, d_off, sizeof(uint64_t) * ((size_t)n + 1), dev, s);
     uint32_t *d_nb;
     HIP_TRY(sc.get(&d_nb, total));
     HEGJ_TRY(gather_rows(r->batches, r->bases, r->d_row_off, r->d_row_cnt, d_off, n, d_nb, sort_rows != 0, s));
-    HIP_TRY(hipMemcpyAsync(nbrs, d_nb, sizeof(uint32_t) * total, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(copy_to_host(offsets, d_off, sizeof(uint64_t) * ((size_t)n + 1), dev, s));
+    HEGJ_TRY(copy_to_host(nbrs, d_nb, sizeof(uint32_t) * total, dev, s));
     return HEGJ_OK;
 }
 

@@ -570,8 +570,7 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     k_g16_maxnorm<<<std::min<uint32_t>(ceil_div(n, 256), 2048), 256, 0, s>>>(ix.soa, n, dim, mean, d_bits);
     HIP_TRY(hipGetLastError());
     unsigned long long bits = 0;
-    HIP_TRY(hipMemcpyAsync(&bits, d_bits, sizeof(bits), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&bits, d_bits, s));
     double max2;
     std::memcpy(&max2, &bits, sizeof(max2));
     if (!std::isfinite(max2)) return HEGJ_OK;
@@ -589,13 +588,14 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
         uint16_t *&A, *&B;
         float *&w;
         ~Guard() {
-            for (void *p : {(void *)A, (void *)B, (void *)w})
-                if (p) (void)hipFree(p);
+            if (A || B || w) (void)hipStreamSynchronize(s);  // a failed launch's stream
+            for (void *p : {(void *)A, (void *)B, (void *)w}) dev_free(p);
         }
-    } guard{A, B, w};
-    HIP_TRY(hipMalloc(&A, sizeof(uint16_t) * rows * kb * 32));
-    HIP_TRY(hipMalloc(&B, sizeof(uint16_t) * rows * kb * 32));
-    HIP_TRY(hipMalloc(&w, sizeof(float) * rows));
+        hipStream_t s;
+    } guard{A, B, w, s};
+    HIP_TRY(dev_malloc_n(&A, rows * kb * 32));
+    HIP_TRY(dev_malloc_n(&B, rows * kb * 32));
+    HIP_TRY(dev_malloc_n(&w, rows));
     const uint32_t blocks = ceil_div(rows, 256);
     const double gamma = g16_gamma(kb);
     switch (kb) {
@@ -606,8 +606,7 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     }
     HIP_TRY(hipGetLastError());
     double err = 0;
-    HIP_TRY(hipMemcpyAsync(&err, d_err, sizeof(err), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&err, d_err, s));
     if (!(err / n <= tau / 16.0)) return HEGJ_OK;
     ops->A = A;
     ops->B = B;
@@ -644,14 +643,12 @@ hegj_status g16_units(const DevIndex &ix, const uint32_t *order, const uint32_t 
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(scan_u32(cnt, off, C, d_total, s));
     uint32_t U = 0;
-    HIP_TRY(hipMemcpyAsync(&U, d_total, sizeof(U), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&U, d_total, s));
     HIP_TRY(dev_malloc_n(units, (size_t)U + 1));
     if (U) k_g16_unit_fill<<<ceil_div(U, 256), 256, 0, s>>>(ix, order, work, (uint32_t)seg, off, U, *units);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));
     *n_units = U;
-    return HEGJ_OK;
+    return scratch_done(s);
 }
 
 hegj_status g16_occupancy(uint32_t kp, int device, uint32_t *blocks) {

@@ -224,8 +224,8 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
     HIP_TRY(sc.get(&keys_alt, n));
     HIP_TRY(sc.get(&vals_alt, n));
     HIP_TRY(sc.get(&dead, 1));
-    HIP_TRY(hipMalloc(&ix->point_key, sizeof(uint64_t) * n));
-    HIP_TRY(hipMalloc(&ix->ila, sizeof(uint32_t) * n));
+    HIP_TRY(dev_malloc_n(&ix->point_key, (size_t)n));
+    HIP_TRY(dev_malloc_n(&ix->ila, (size_t)n));
     HIP_TRY(hipMemsetAsync(dead, 0, sizeof(uint32_t), s));
     uint32_t blocks = ceil_div(n, kT);
     k_cell_ids<<<blocks, kT, 0, s>>>(ix->pts, *g, keys, ix->point_key, ix->ila, dead);
@@ -240,12 +240,11 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
     k_run_flags<<<blocks, kT, 0, s>>>(keys, n, 1, flags);
     HEGJ_TRY(scan_u32(flags, rank, n, d_count, s));
     uint32_t C;
-    HIP_TRY(hipMemcpyAsync(&C, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(n_dead, dead, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&C, d_count, s));
+    HEGJ_TRY(read_back(n_dead, dead, s));
     ix->C = C;
-    HIP_TRY(hipMalloc(&ix->cell_start, sizeof(uint32_t) * (C + 1)));
-    HIP_TRY(hipMalloc(&ix->cell_key, sizeof(uint64_t) * C));
+    HIP_TRY(dev_malloc_n(&ix->cell_start, (size_t)C + 1));
+    HIP_TRY(dev_malloc_n(&ix->cell_key, (size_t)C));
     k_run_compact<<<blocks, kT, 0, s>>>(keys, n, 1, flags, rank, ix->cell_start, ix->cell_key);
     k_set_u32<<<1, 1, 0, s>>>(ix->cell_start + C, n);
     HIP_TRY(hipGetLastError());
@@ -256,11 +255,10 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
     k_run_flags<<<cb, kT, 0, s>>>(ix->cell_key, C, div, flags);
     HEGJ_TRY(scan_u32(flags, rank, C, d_count, s));
     uint32_t R;
-    HIP_TRY(hipMemcpyAsync(&R, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&R, d_count, s));
     ix->R = R;
-    HIP_TRY(hipMalloc(&ix->row_start, sizeof(uint32_t) * (R + 1)));
-    HIP_TRY(hipMalloc(&ix->row_key, sizeof(uint64_t) * R));
+    HIP_TRY(dev_malloc_n(&ix->row_start, (size_t)R + 1));
+    HIP_TRY(dev_malloc_n(&ix->row_key, (size_t)R));
     k_run_compact<<<cb, kT, 0, s>>>(ix->cell_key, C, div, flags, rank, ix->row_start, ix->row_key);
     k_set_u32<<<1, 1, 0, s>>>(ix->row_start + R, C);
     HIP_TRY(hipGetLastError());
@@ -269,18 +267,18 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
     uint32_t hsize = 1024;
     while (hsize < 2 * R) hsize <<= 1;
     ix->hmask = hsize - 1;
-    HIP_TRY(hipMalloc(&ix->hkeys, sizeof(uint64_t) * hsize));
-    HIP_TRY(hipMalloc(&ix->hvals, sizeof(uint32_t) * hsize));
+    HIP_TRY(dev_malloc_n(&ix->hkeys, (size_t)hsize));
+    HIP_TRY(dev_malloc_n(&ix->hvals, (size_t)hsize));
     k_hash_fill<<<ceil_div(hsize, kT), kT, 0, s>>>(ix->hkeys, hsize);
     k_hash_insert<<<ceil_div(R, kT), kT, 0, s>>>(ix->row_key, R, ix->hkeys, ix->hvals, ix->hmask);
     HIP_TRY(hipGetLastError());
 
     // -- coordinates in cell order ---------------------------------------------
-    HIP_TRY(hipMalloc(&ix->soa, sizeof(double) * (size_t)n * dim));
+    HIP_TRY(dev_malloc_n(&ix->soa, (size_t)n * dim));
     k_gather_soa<<<blocks, kT, 0, s>>>(ix->pts, ix->ila, n, dim, ix->soa);
     HIP_TRY(hipGetLastError());
     if (dim <= kAosMaxDim) {
-        HIP_TRY(hipMalloc(&ix->aos, sizeof(double) * (size_t)n * dim));
+        HIP_TRY(dev_malloc_n(&ix->aos, (size_t)n * dim));
         k_gather_aos<<<blocks, kT, 0, s>>>(ix->pts, ix->ila, n, dim, ix->aos);
         HIP_TRY(hipGetLastError());
     }
@@ -291,8 +289,7 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
 void free_index(DevIndex *ix) {
     void *ps[] = {ix->pts, ix->soa, ix->aos, ix->ila, ix->point_key, ix->cell_key, ix->cell_start,
                   ix->row_start, ix->row_key, ix->hkeys, ix->hvals};
-    for (void *p : ps)
-        if (p) (void)hipFree(p);
+    for (void *p : ps) dev_free(p);
     *ix = DevIndex{};
 }
 

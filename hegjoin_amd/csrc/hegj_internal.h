@@ -91,10 +91,31 @@ void set_thread_arena(Arena *a);  // nullptr: back to hipMalloc
 constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
 hegj_status noalloc_scratch(int device, void **ptr);
 
-// Scratch allocator for temporaries of one call (freed by the destructor).
+// One public call on one stream.  While a thread has one open, its Scratch
+// buffers come from the buffer cache and are returned when the call ends (after
+// the stream has drained), so the steps of a call need no synchronisation or
+// hipFree between them: a self-join of 20k points spent 10x its kernels' time
+// on them.  Only the outermost scope of a thread acts.
+struct CallScope {
+    explicit CallScope(hipStream_t s);
+    ~CallScope();
+    hipStream_t stream;
+    bool active;
+    std::vector<void *> ptrs;
+};
+// Whether a Scratch's memory outlives the function that owns it (an open call
+// scope or an installed arena).
+bool scratch_outlives();
+// Before a Scratch goes out of scope with kernels still using it.
+hegj_status scratch_done(hipStream_t s);
+
+// Scratch allocator for temporaries of one call (freed by the destructor, or
+// by the call scope).
 struct Scratch {
     std::vector<void *> ptrs;
+    bool scoped = false;  // ptrs belong to the thread's call scope
     hipError_t alloc(void **p, size_t bytes);
+    hegj_status drop(hipStream_t s);  // gives everything back now
     template <typename T>
     hipError_t get(T **p, size_t count) {
         return alloc(reinterpret_cast<void **>(p), count * sizeof(T) + 16);
@@ -106,9 +127,9 @@ struct Scratch {
 // from a cache: a freed buffer is kept for the next join of the same shape
 // instead of going back through hipFree / hipMalloc, each of which costs
 // ~0.1 ms and synchronises the device.  dev_free only when the work using the
-// buffer has completed.  At most 16 GiB of freed buffers are kept; an
-// allocation that fails first releases them.  Pointers not from dev_malloc
-// are passed to hipFree.
+// buffer has completed.  At most 16 GiB of freed buffers are kept (the longest
+// unused go first); an allocation that fails first releases them.  Pointers
+// not from dev_malloc are passed to hipFree.
 hipError_t dev_malloc(void **p, size_t bytes);
 template <typename T>
 hipError_t dev_malloc_n(T **p, size_t count) {
@@ -116,6 +137,18 @@ hipError_t dev_malloc_n(T **p, size_t count) {
 }
 void dev_free(void *p);
 void cache_release_device(int dev);  // hipFree the cached buffers of one device
+
+// Device -> host.  read_back: small structures through pinned memory; the
+// stream is synchronised.  copy_to_host: results into the caller's pageable
+// memory, in chunks through pinned buffers with several threads copying out
+// (a plain hipMemcpy to pageable memory ran at 18 GB/s, the link does 57).
+hegj_status read_back_bytes(void *dst, const void *src, size_t bytes, hipStream_t s);
+template <typename T>
+hegj_status read_back(T *dst, const T *src, hipStream_t s, size_t count = 1) {
+    return read_back_bytes(dst, src, sizeof(T) * count, s);
+}
+hegj_status copy_to_host(void *dst, const void *src, size_t bytes, int device, hipStream_t s);
+void pinned_release();  // free the unused pinned buffers
 
 // Largest s with RN(sqrt(s)) <= eps (the distance predicate without sqrt).
 double sqrt_threshold(double eps);

@@ -1474,14 +1474,12 @@ hegj_status build_units(const GridGeom &g, const DevIndex &ix, uint32_t qb, cons
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(scan_u32(ucount, uoff, C, d_total, s));
     uint32_t U;
-    HIP_TRY(hipMemcpyAsync(&U, d_total, sizeof(U), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&U, d_total, s));
     HIP_TRY(dev_malloc_n(units, (size_t)U + 1));
     k_unit_fill<<<ceil_div(C, 256), 256, 0, s>>>(ix, qb, order, ucount, uoff, *units);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));
     *n_units = U;
-    return HEGJ_OK;
+    return scratch_done(s);
 }
 
 // Threads per workgroup of a join launch: 64 per wave, `block_waves` waves
@@ -1672,10 +1670,10 @@ hegj_status join_occupancy(uint32_t dim, uint32_t qb, int device, uint32_t *bloc
     if (lds > kMaxQueryLds)
         return fail(HEGJ_ERR_UNSUPPORTED, "queries_per_unit * dim too large for LDS; lower queries_per_unit");
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * kWavesPerBlock, lds));
-    hipDeviceProp_t prop;
-    HIP_TRY(hipGetDeviceProperties(&prop, device));
+    int cus = 0;  // (the whole property structure takes ~0.1 ms to fetch)
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     if (per_cu < 1) per_cu = 1;
-    *blocks = (uint32_t)per_cu * (uint32_t)prop.multiProcessorCount;
+    *blocks = (uint32_t)per_cu * (uint32_t)cus;
     return HEGJ_OK;
 }
 

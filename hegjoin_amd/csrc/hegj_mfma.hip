@@ -500,9 +500,9 @@ hegj_status occ_gb(int device, uint32_t *blocks) {
     int per_cu = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, reinterpret_cast<const void *>(&k_gb_join<KB>), 64 * gb_waves(KB), 0));
-    hipDeviceProp_t prop;
-    HIP_TRY(hipGetDeviceProperties(&prop, device));
-    *blocks = (uint32_t)std::max(per_cu, 1) * (uint32_t)prop.multiProcessorCount;
+    int cus = 0;
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    *blocks = (uint32_t)std::max(per_cu, 1) * (uint32_t)cus;
     return HEGJ_OK;
 }
 
@@ -553,9 +553,9 @@ hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, GbOperands *ops, h
     if (ops->A) return HEGJ_OK;
     const uint32_t kb = gb_kblocks(dim), kp = kb * 32;
     if (kb == 0) return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA refine for this dimensionality");
-    HIP_TRY(hipMalloc(&ops->A, sizeof(uint16_t) * (size_t)n * kp));
-    HIP_TRY(hipMalloc(&ops->B, sizeof(uint16_t) * (size_t)n * kp));
-    HIP_TRY(hipMalloc(&ops->w, sizeof(float) * n));
+    HIP_TRY(dev_malloc_n(&ops->A, (size_t)n * kp));
+    HIP_TRY(dev_malloc_n(&ops->B, (size_t)n * kp));
+    HIP_TRY(dev_malloc_n(&ops->w, n));
     ops->kp = kp;
     k_gb_prepare<<<ceil_div(n, 256), 256, 0, s>>>(ix.soa, n, dim, kp, mean, gb_coefficient(dim, kp),
                                                  ops->A, ops->B, ops->w);
@@ -667,8 +667,7 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
         HEGJ_TRY(gb_launch(ops, a, blocks, s));
         HIP_TRY(hipEventRecord(e1, s));
         if (ops.f16) HEGJ_TRY(g16_decide(a, 2048, s));
-        HIP_TRY(hipMemcpyAsync(&c, d, sizeof(Ctr), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HEGJ_TRY(read_back(&c, d, s));
         float kms = 0;
         HIP_TRY(hipEventElapsedTime(&kms, e0, e1));
         (void)hipEventDestroy(e0);
@@ -678,11 +677,13 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
             if (need > 0xFFFFFF00ull) return fail(HEGJ_ERR_UNSUPPORTED, "more than 2^32 pair slots");
             raw_cap = need;
             pair_cap = std::max(pair_cap, need * (mirror ? 2 : 1));
+            HEGJ_TRY(it.drop(s));
             continue;
         }
         if (c.overflow) {
             pair_cap = std::max(pair_cap * 2, (uint64_t)((c.n_accept + (ops.f16 ? 0 : c.n_band)) * 1.25) + (1u << 22));
             band_cap = std::max(band_cap * 2, (uint64_t)(c.n_band * 1.25) + (1u << 22));
+            HEGJ_TRY(it.drop(s));
             continue;
         }
         // exact FP64 recheck of the band
@@ -692,10 +693,10 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
                                                           pair_cap, &d->pair_cursor, &d->n_accept,
                                                           &d->overflow);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(&c, d, sizeof(Ctr), hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
+            HEGJ_TRY(read_back(&c, d, s));
             if (c.overflow) {
                 pair_cap = std::max(pair_cap * 2, (uint64_t)(c.n_accept * 1.25) + (1u << 22));
+                HEGJ_TRY(it.drop(s));
                 continue;
             }
         }
@@ -708,7 +709,7 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
         uint64_t *keys_alt;
         HIP_TRY(it.get(&keys_alt, ntot + 1));
         HEGJ_TRY(radix_sort_pairs(pairs, keys_alt, (uint32_t)ntot, qbits, s));
-        HIP_TRY(hipMalloc(&out->buf, sizeof(uint32_t) * std::max<uint64_t>(nvalid, 1)));
+        HIP_TRY(dev_malloc_n(&out->buf, std::max<uint64_t>(nvalid, 1)));
         if (nvalid)
             k_gb_emit<<<std::min<uint32_t>(ceil_div(nvalid, 256), 2048), 256, 0, s>>>(pairs, nvalid, ix.ila, out->buf, out->hash);
         k_gb_rows<<<ceil_div(n, 256), 256, 0, s>>>(pairs, nvalid, n, ix.ila, out->row_off, out->row_cnt);

@@ -106,9 +106,7 @@ hegj_status scan_impl(const T *in, T *out, uint32_t n, T *d_total, hipStream_t s
     k_scan_sums<T><<<1, 1024, 0, s>>>(sums, tiles, d_total);
     k_scan_apply<T><<<tiles, kScanThreads, 0, s>>>(in, out, sums, n);
     HIP_TRY(hipGetLastError());
-    // Scratch is freed on return: make sure the kernels are done with it.
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return scratch_done(s);
 }
 
 // ---------------------------------------------------------------------------
@@ -213,8 +211,7 @@ hegj_status radix_impl(K *keys, uint32_t *vals, K *keys_alt, uint32_t *vals_alt,
         HIP_TRY(hipMemcpyAsync(keys, src_k, sizeof(K) * n, hipMemcpyDeviceToDevice, s));
         if (VALS) HIP_TRY(hipMemcpyAsync(vals, src_v, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
     }
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return scratch_done(s);
 }
 
 }  // namespace

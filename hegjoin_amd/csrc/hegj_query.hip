@@ -681,8 +681,7 @@ hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const d
     k_qrun_fill<<<ceil_div(nq, 256), 256, 0, s>>>(flag, rank, nq, p->starts);
     HIP_TRY(hipGetLastError());
     uint32_t h[2];
-    HIP_TRY(hipMemcpyAsync(h, d_small, sizeof(h), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(h, d_small, s, 2));
     const uint32_t runs = h[0];
     p->n_live = h[1];
     // starts[runs] = end of the live queries
@@ -701,14 +700,12 @@ hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const d
         k_sub_fill<<<ceil_div(runs, 256), 256, 0, s>>>(p->starts, runs, first, sub_starts);
         HIP_TRY(hipGetLastError());
         uint32_t units = 0;
-        HIP_TRY(hipMemcpyAsync(&units, d_total, sizeof(units), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HEGJ_TRY(read_back(&units, d_total, s));
         HIP_TRY(hipMemcpyAsync(p->starts, sub_starts, sizeof(uint32_t) * units, hipMemcpyDeviceToDevice, s));
         HIP_TRY(hipMemcpyAsync(p->starts + units, &p->n_live, sizeof(uint32_t), hipMemcpyHostToDevice, s));
         p->n_units = units;
     }
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return scratch_done(s);  // the plan outlives the copies from it
 }
 
 hegj_status query_run(const QJoinArgs &base, bool fill, int device, hipStream_t s) {

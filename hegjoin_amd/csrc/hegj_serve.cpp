@@ -194,8 +194,7 @@ hegj_status hegj_server::run(Request *r, hipStream_t s, Arena &arena, void *ctr_
         HIP_TRY(keep.get(&q32, (size_t)nq * dim));
         HEGJ_TRY(query_to_f32(q, nq, dim, L.centre, q32, &ctr->rbits, s));
         unsigned long long rb = 0;
-        HIP_TRY(hipMemcpyAsync(&rb, &ctr->rbits, sizeof(rb), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HEGJ_TRY(read_back(&rb, &ctr->rbits, s));
         double rq;
         std::memcpy(&rq, &rb, sizeof(rq));
         const double R = std::max(L.radius, rq) * (1.0 + 1e-12);
@@ -228,8 +227,7 @@ hegj_status hegj_server::run(Request *r, hipStream_t s, Arena &arena, void *ctr_
     HEGJ_TRY(query_run(a, false, device, s));
     HEGJ_TRY(query_offsets(counts, nq, offsets, s));
     uint64_t total = 0;
-    HIP_TRY(hipMemcpyAsync(&total, offsets + nq, sizeof(total), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&total, offsets + nq, s));
     r->t_counted = Clock::now();
     const uint64_t off_bytes = align_up(sizeof(uint64_t) * ((uint64_t)nq + 1));
     HEGJ_TRY(admit(this, r, off_bytes + sizeof(uint32_t) * std::max<uint64_t>(total, 1)));
@@ -243,8 +241,7 @@ hegj_status hegj_server::run(Request *r, hipStream_t s, Arena &arena, void *ctr_
     HEGJ_TRY(query_run(a, true, device, s));
     HEGJ_TRY(query_hash(res_off, res_nb, nq, total, &ctr->hash, s));
     Ctr c;
-    HIP_TRY(hipMemcpyAsync(&c, ctr, sizeof(c), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HEGJ_TRY(read_back(&c, ctr, s));
     r->pairs = total;
     r->hash = c.hash;
     r->evals = c.evals;
@@ -513,12 +510,11 @@ hegj_status hegj_serve_copy(hegj_server *S, uint64_t ticket, uint64_t *offsets, 
     }
     HEGJ_TRY(select_device(S->device));
     const uint64_t off_bytes = align_up(sizeof(uint64_t) * ((uint64_t)r->nq + 1));
-    HIP_TRY(hipMemcpyAsync(offsets, S->pool_base + r->pool_off, sizeof(uint64_t) * ((size_t)r->nq + 1),
-                           hipMemcpyDeviceToHost, S->copy_stream));
+    HEGJ_TRY(copy_to_host(offsets, S->pool_base + r->pool_off, sizeof(uint64_t) * ((size_t)r->nq + 1), S->device,
+                          S->copy_stream));
     if (neighbors && r->pairs)
-        HIP_TRY(hipMemcpyAsync(neighbors, S->pool_base + r->pool_off + off_bytes,
-                               sizeof(uint32_t) * r->pairs, hipMemcpyDeviceToHost, S->copy_stream));
-    HIP_TRY(hipStreamSynchronize(S->copy_stream));
+        HEGJ_TRY(copy_to_host(neighbors, S->pool_base + r->pool_off + off_bytes, sizeof(uint32_t) * r->pairs,
+                              S->device, S->copy_stream));
     return HEGJ_OK;
 }
 

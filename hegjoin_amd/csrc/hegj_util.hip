@@ -321,8 +321,9 @@ hegj_status workload_order(const DevIndex &ix, const uint32_t *work, uint32_t *o
     k_total_candidates<<<ceil_div(C, kT), kT, 0, s>>>(ix.cell_start, work, C, tot);
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(radix_sort_u32(keys, order, keys_alt, vals_alt, C, 32, s));
-    HIP_TRY(hipMemcpyAsync(total_candidates, tot, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    unsigned long long t = 0;
+    HEGJ_TRY(read_back(&t, tot, s));
+    *total_candidates = t;
     return HEGJ_OK;
 }
 
@@ -339,8 +340,7 @@ hegj_status origin_point_index(const DevIndex &ix, const uint32_t *order, uint32
     k_origin_scatter<<<ceil_div((uint64_t)C * 64, kT), kT, 0, s>>>(ix.cell_start, ix.ila, order, offs,
                                                                  C, opi);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return scratch_done(s);
 }
 
 hegj_status stride_units(const uint2 *in, uint32_t n_out, uint32_t stride, uint2 *out,
@@ -366,8 +366,7 @@ hegj_status csr_offsets(const uint32_t *row_cnt, uint32_t n, uint64_t *csr_off, 
     k_u32_to_u64<<<ceil_div(n, kT), kT, 0, s>>>(row_cnt, n, tmp);
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(scan_u64(tmp, csr_off, n, csr_off + n, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return scratch_done(s);
 }
 
 hegj_status gather_rows(const std::vector<uint32_t *> &batches, const std::vector<uint64_t> &bases,
@@ -391,8 +390,7 @@ hegj_status gather_rows(const std::vector<uint32_t *> &batches, const std::vecto
         HIP_TRY(hipGetLastError());
         k_sort_long<<<512, kLongT, 0, s>>>(row_cnt, csr_off, out, longs, longs + n);
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipStreamSynchronize(s));
-        return HEGJ_OK;
+        return scratch_done(s);
     }
     k_gather_rows<<<ceil_div((uint64_t)n * 64, kT), kT, 0, s>>>(bt, row_off, row_cnt, csr_off, n, out);
     HIP_TRY(hipGetLastError());
@@ -559,9 +557,7 @@ hegj_status split_units(const DevIndex &ix, const uint2 *units, uint32_t n_units
     HEGJ_TRY(scan_u64(w, prefix, n_units, total, s));
     k_find_splits<<<1, 64, 0, s>>>(prefix, n_units, total, n_parts, d_end);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(part_end, d_end, sizeof(uint32_t) * n_parts, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return HEGJ_OK;
+    return read_back(part_end, d_end, s, n_parts);
 }
 
 namespace {
@@ -622,7 +618,7 @@ hegj_status make_soa32(const GridGeom &g, const DevIndex &ix, float **soa32, flo
     Scratch sc;
     double *part, *centre;
     HIP_TRY(sc.get(&part, (size_t)blocks * dim * 2));
-    HIP_TRY(hipMalloc(centre_dev, sizeof(double) * dim));
+    HIP_TRY(dev_malloc_n(centre_dev, dim));
     centre = *centre_dev;
     k_dim_minmax<<<blocks, 256, 0, s>>>(ix.soa, n, dim, part);
     HIP_TRY(hipGetLastError());
@@ -642,12 +638,12 @@ hegj_status make_soa32(const GridGeom &g, const DevIndex &ix, float **soa32, flo
     }
     *radius = R * (1.0 + 1e-12);
     HIP_TRY(hipMemcpyAsync(centre, c.data(), sizeof(double) * dim, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMalloc(soa32, sizeof(float) * (size_t)n * dim));
+    HIP_TRY(dev_malloc_n(soa32, (size_t)n * dim));
     const uint64_t total = (uint64_t)n * dim;
     k_soa32<<<ceil_div(total, 256), 256, 0, s>>>(ix.soa, total, n, centre, *soa32);
     HIP_TRY(hipGetLastError());
     if (aos32 && dim <= kAosMaxDim) {
-        HIP_TRY(hipMalloc(aos32, sizeof(float) * ((size_t)n + kAos32Pad) * dim));
+        HIP_TRY(dev_malloc_n(aos32, ((size_t)n + kAos32Pad) * dim));
         k_aos32<<<ceil_div((uint64_t)n + kAos32Pad, 256), 256, 0, s>>>(*soa32, n, dim, *aos32);
         HIP_TRY(hipGetLastError());
     }

@@ -81,10 +81,12 @@ int hegj_device_count(void);
  * of the reference; it is the measured roof the join's HBM figures are
  * compared with. */
 hegj_status hegj_stream_copy_bandwidth(uint64_t bytes, int device, double *gbps);
-/* The self-join keeps the device buffers of finished calls (work units, row
- * tables, result batches) for reuse by later calls, up to 16 GiB per process
- * (an allocation that fails releases them first).  This returns the unused
- * ones on `device` (-1: every device).  No reference counterpart. */
+/* The library keeps the device buffers of finished calls and freed indexes
+ * (index arrays, work units, temporaries, row tables, result batches) for
+ * reuse by later calls, up to 16 GiB per process (an allocation that fails
+ * releases them first), and up to 33 MiB of pinned host memory.  This returns
+ * the unused buffers on `device` (-1: every device, and the pinned memory).
+ * No reference counterpart. */
 void hegj_release_cached_memory(int device);
 
 /* ------------------------------------------------------------------------ */
