@@ -48,6 +48,16 @@ __global__ __launch_bounds__(kT) void k_minmax(const double *__restrict__ pts, u
 
 // S2 + S3 (kernel.cu:54-60): FP64 subtract, IEEE FP64 divide, truncation to
 // unsigned, linear id with dim 0 fastest.  Also the identity permutation.
+// Indexed coordinates of each non-empty cell, one plane per dim.
+__global__ __launch_bounds__(kT) void k_cell_xyz(const uint64_t *__restrict__ cell_key, uint32_t C, GridGeom g,
+                                                 uint32_t *__restrict__ xyz) {
+    const uint32_t i = blockIdx.x * kT + threadIdx.x;
+    if (i >= C) return;
+    uint32_t c[kMaxK];
+    decode_cell(cell_key[i], g, c);
+    for (uint32_t j = 0; j < g.k; j++) xyz[(uint64_t)j * C + i] = c[j];
+}
+
 __global__ __launch_bounds__(kT) void k_cell_ids(const double *__restrict__ pts, GridGeom g,
                                                  uint64_t *__restrict__ keys,
                                                  uint64_t *__restrict__ point_key,
@@ -97,24 +107,25 @@ __global__ __launch_bounds__(kT) void k_run_compact(const uint64_t *__restrict__
 
 __global__ void k_set_u32(uint32_t *p, uint32_t v) { *p = v; }
 
-__global__ __launch_bounds__(kT) void k_hash_fill(uint64_t *__restrict__ hkeys, uint32_t size) {
+__global__ __launch_bounds__(kT) void k_hash_fill(RowSlot *__restrict__ hrows, uint32_t size) {
     uint32_t i = blockIdx.x * kT + threadIdx.x;
-    if (i < size) hkeys[i] = ~0ull;
+    if (i < size) hrows[i] = RowSlot{~0ull, 0u, 0u};
 }
 
 __global__ __launch_bounds__(kT) void k_hash_insert(const uint64_t *__restrict__ row_key,
-                                                    uint32_t R, uint64_t *__restrict__ hkeys,
-                                                    uint32_t *__restrict__ hvals,
+                                                    const uint32_t *__restrict__ row_start,
+                                                    uint32_t R, RowSlot *__restrict__ hrows,
                                                     uint32_t hmask) {
     uint32_t r = blockIdx.x * kT + threadIdx.x;
     if (r >= R) return;
     uint64_t key = row_key[r];
     uint32_t s = hash_slot(key) & hmask;
     while (true) {
-        unsigned long long prev = atomicCAS((unsigned long long *)&hkeys[s], ~0ull,
+        unsigned long long prev = atomicCAS((unsigned long long *)&hrows[s].key, ~0ull,
                                             (unsigned long long)key);
         if (prev == ~0ull || prev == key) {
-            hvals[s] = r;
+            hrows[s].first = row_start[r];
+            hrows[s].end = row_start[r + 1];
             return;
         }
         s = (s + 1) & hmask;
@@ -247,6 +258,8 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
     HIP_TRY(dev_malloc_n(&ix->cell_key, (size_t)C));
     k_run_compact<<<blocks, kT, 0, s>>>(keys, n, 1, flags, rank, ix->cell_start, ix->cell_key);
     k_set_u32<<<1, 1, 0, s>>>(ix->cell_start + C, n);
+    HIP_TRY(dev_malloc_n(&ix->cell_xyz, (size_t)C * k));
+    k_cell_xyz<<<ceil_div(C, kT), kT, 0, s>>>(ix->cell_key, C, *g, ix->cell_xyz);
     HIP_TRY(hipGetLastError());
 
     // -- rows: cells sharing coordinates 1..k-1 ----------------------------------
@@ -267,10 +280,9 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
     uint32_t hsize = 1024;
     while (hsize < 2 * R) hsize <<= 1;
     ix->hmask = hsize - 1;
-    HIP_TRY(dev_malloc_n(&ix->hkeys, (size_t)hsize));
-    HIP_TRY(dev_malloc_n(&ix->hvals, (size_t)hsize));
-    k_hash_fill<<<ceil_div(hsize, kT), kT, 0, s>>>(ix->hkeys, hsize);
-    k_hash_insert<<<ceil_div(R, kT), kT, 0, s>>>(ix->row_key, R, ix->hkeys, ix->hvals, ix->hmask);
+    HIP_TRY(dev_malloc_n(&ix->hrows, (size_t)hsize));
+    k_hash_fill<<<ceil_div(hsize, kT), kT, 0, s>>>(ix->hrows, hsize);
+    k_hash_insert<<<ceil_div(R, kT), kT, 0, s>>>(ix->row_key, ix->row_start, R, ix->hrows, ix->hmask);
     HIP_TRY(hipGetLastError());
 
     // -- coordinates in cell order ---------------------------------------------
@@ -287,8 +299,8 @@ hegj_status build_index(GridGeom *g, double *maxArr, uint64_t *totalCells, DevIn
 }
 
 void free_index(DevIndex *ix) {
-    void *ps[] = {ix->pts, ix->soa, ix->aos, ix->ila, ix->point_key, ix->cell_key, ix->cell_start,
-                  ix->row_start, ix->row_key, ix->hkeys, ix->hvals};
+    void *ps[] = {ix->pts, ix->soa, ix->aos, ix->ila, ix->point_key, ix->cell_key, ix->cell_xyz, ix->cell_start,
+                  ix->row_start, ix->row_key, ix->hrows};
     for (void *p : ps) dev_free(p);
     *ix = DevIndex{};
 }

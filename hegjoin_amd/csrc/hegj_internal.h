@@ -55,6 +55,12 @@ struct GridGeom {
                         // values; cell ids and distances are computed in FP32
 };
 
+// Entry of the row hash table: one 16-byte load finds a row's cells.
+struct alignas(16) RowSlot {
+    uint64_t key;         // ~0: empty
+    uint32_t first, end;  // the row's cells
+};
+
 // Device-resident grid index.  Naming follows the reference: a "cell" is a
 // non-empty grid cell (gridCellLookupArr entry), a "row" groups the cells that
 // share indexed coordinates 1..k-1 (they differ only in coordinate 0 and are
@@ -67,11 +73,11 @@ struct DevIndex {
     uint32_t *ila = nullptr;      // [n] indexLookupArr: cell-order position -> point id
     uint64_t *point_key = nullptr;// [n] linear cell id per point (original order)
     uint64_t *cell_key = nullptr; // [C] gridLinearID of each non-empty cell
+    uint32_t *cell_xyz = nullptr; // [k][C] its indexed coordinates
     uint32_t *cell_start = nullptr;// [C+1] first cell-order position of each cell
     uint32_t *row_start = nullptr;// [R+1] first cell of each row
     uint64_t *row_key = nullptr;  // [R] row key = cell_key / nCells[0]
-    uint64_t *hkeys = nullptr;    // row hash table keys (empty = ~0)
-    uint32_t *hvals = nullptr;    // row hash table values (row index)
+    RowSlot *hrows = nullptr;     // row hash table, open addressing
     uint32_t hmask = 0;
     uint32_t C = 0, R = 0;
 };
@@ -407,8 +413,14 @@ __host__ __device__ __forceinline__ uint64_t mix64(uint64_t x) {
     return z ^ (z >> 31);
 }
 
+// Slot hash of a row key: two multiplicative rounds in 32 bits (the 64-bit
+// products of mix64 are eight quarter-rate instructions; a unit hashes 243
+// keys).
 __device__ __forceinline__ uint32_t hash_slot(uint64_t key) {
-    return (uint32_t)(mix64(key) >> 16);
+    uint32_t x = (uint32_t)key * 0x9E3779B1u ^ (uint32_t)(key >> 32) * 0x85EBCA77u;
+    x ^= x >> 15;
+    x *= 0x2C1B3C6Du;
+    return x ^ (x >> 13);
 }
 
 // Lanes below the calling lane.
@@ -432,15 +444,16 @@ __device__ __forceinline__ uint64_t wave_bcast_u64(uint64_t v) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-// Row hash lookup: returns the row index or ~0u.
-__device__ __forceinline__ uint32_t row_lookup(const uint64_t *__restrict__ hkeys,
-                                               const uint32_t *__restrict__ hvals,
-                                               uint32_t hmask, uint64_t key) {
+// Row hash lookup: the row's cells, false when it has none.
+__device__ __forceinline__ bool row_lookup(const RowSlot *__restrict__ hrows, uint32_t hmask, uint64_t key,
+                                           uint32_t *first, uint32_t *end) {
     uint32_t s = hash_slot(key) & hmask;
     while (true) {
-        uint64_t kk = hkeys[s];
-        if (kk == key) return hvals[s];
-        if (kk == ~0ull) return ~0u;
+        const RowSlot e = hrows[s];
+        *first = e.first;
+        *end = e.end;
+        if (e.key == key) return true;
+        if (e.key == ~0ull) return false;
         s = (s + 1) & hmask;
     }
 }
@@ -502,9 +515,8 @@ __device__ __forceinline__ void stencil_row(const uint32_t *c, const uint32_t *l
         rkey += (uint64_t)cj * mult;
         mult *= g.nCells[j];
     }
-    uint32_t row = row_lookup(ix.hkeys, ix.hvals, ix.hmask, rkey);
-    if (row == ~0u) return;
-    uint32_t rs = ix.row_start[row], re = ix.row_start[row + 1];
+    uint32_t rs, re;
+    if (!row_lookup(ix.hrows, ix.hmask, rkey, &rs, &re)) return;
     uint64_t base = rkey * g.nCells[0];
     uint32_t a, b;
     if (re - rs <= 8) {  // short rows (the common case at k >= 4): scan

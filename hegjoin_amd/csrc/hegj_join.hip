@@ -31,7 +31,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "hegj_internal.h"
+#include "hegj_stencil.h"
 
 namespace hegj {
 
@@ -44,13 +44,10 @@ constexpr int kWavesPerBlockQ = kWavesPerBlock;
 // hit masks the workgroup stays within 64 KiB)
 constexpr uint32_t kMaxQueryLds = 36u << 10;
 
-// Compacted stencil-row list of one unit in LDS.
-constexpr int kBandList = 64;  // FP32 filter: (query, chunk) pairs awaiting the FP64 recheck
-struct RowList {
-    uint32_t start[kMaxRows + 1];  // first candidate position of slot s (+1: the FP32 kernel's padding slot)
-    uint32_t off[kMaxRows + 1];    // prefix of slot lengths
-    float2 gap[16 * kMaxK];      // per (query, indexed dim): squared gaps to the -1 / +1 cell
-    uint32_t band[kBandList];    // (chunk << 4) | query
+// Stencil rows of one unit in LDS, and the FP32 filter's list.
+constexpr int kBandList = 64;  // (query, chunk) pairs awaiting the FP64 recheck
+struct RowList : StencilList {
+    uint32_t band[kBandList];  // (chunk << 4) | query
 };
 
 // Enumerate the stencil rows of cell `cell` into rl; returns the number of
@@ -67,192 +64,52 @@ struct RowList {
 // than the exact one: the pair set is unchanged, fewer candidates are
 // evaluated.  All points of a unit lie in one cell.
 template <int QB>
-__device__ uint32_t build_rows(const JoinArgs &a, uint32_t cell, RowList &rl, uint32_t *nslots,
-                               bool *live, uint32_t qpos0, uint32_t nq) {
+__device__ uint32_t build_rows(const JoinArgs &a, uint32_t cell, RowList &rl, StencilTabs<QB> &tb,
+                               uint32_t *nslots, bool *live, uint32_t qpos0, uint32_t nq) {
     const GridGeom &g = a.g;
     const DevIndex &ix = a.ix;
     const int lane = threadIdx.x & 63;
-    uint32_t c[kMaxK], lo[kMaxK], hi[kMaxK];
-    decode_cell(ix.cell_key[cell], g, c);
-    bool ok = true;
-    for (uint32_t j = 0; j < g.k; j++) ok &= stencil_dim(c[j], g.nCells[j], g.emulate_cell0, &lo[j], &hi[j]);
+    CellBox b;
+    const bool ok = cell_box(g, ix, cell, b);
     *live = ok;
     if (!ok) {
         *nslots = 0;
         return 0;
     }
     // squared gaps of query q to its -1 / +1 neighbour along indexed dim j,
-    // into rl.gap[q * kMaxK + j] (read back below as wave-uniform broadcasts)
-    static_assert(QB <= 16, "gap table holds 16 queries");
+    // into tb.gap[q * kMaxK + j]
     const uint32_t k = g.k;
-    for (uint32_t e = (uint32_t)lane; e < nq * k; e += 64) {
+    wave_lds_sync();  // the tables lie over the previous unit's hit masks
+    for (uint32_t e = (uint32_t)lane; a.prune && e < nq * k; e += 64) {
         const uint32_t qi = e / k, j = e - qi * k;
         uint32_t cj = 0;
+        double mn = 0.0;
 #pragma unroll
-        for (int jj = 0; jj < kMaxK; jj++)
-            if ((uint32_t)jj == j) cj = c[jj];
+        for (int jj = 0; jj < kMaxK; jj++) {
+            cj = (uint32_t)jj == j ? b.c[jj] : cj;
+            mn = (uint32_t)jj == j ? g.minArr[jj] : mn;
+        }
         const double x = ix.soa[(uint64_t)j * g.n + qpos0 + qi];
-        double f = (x - g.minArr[j]) / g.eps - (double)cj;
+        double f = (x - mn) / g.eps - (double)cj;
         f = f < 0.0 ? 0.0 : (f > 1.0 ? 1.0 : f);
         // DTYPE=float assigns cells in FP32: two roundings of relative 2^-24
         // move a point by at most 1.2e-7 (c_j + 2) cells
         const double mg = g.f32dt ? 1e-6 + 3e-7 * ((double)cj + 2.0) : 1e-6 + 2e-15 * ((double)cj + 2.0);
         const double gm = f - mg > 0.0 ? f - mg : 0.0, gp = 1.0 - f - mg > 0.0 ? 1.0 - f - mg : 0.0;
-        rl.gap[qi * kMaxK + j] = make_float2((float)(gm * gm), (float)(gp * gp));
+        tb.gap[qi * kMaxK + j] = make_float2((float)(gm * gm), (float)(gp * gp));
     }
     wave_lds_sync();
     // DTYPE=float: the FP32 chain accepts squared distances up to about
     // (1 + (dim + 4) 2^-23) T
     const float rel = 1e-5f + (g.f32dt ? 1.2e-7f * (float)(g.dim + 4) : 0.0f);
     const float thr = a.prune ? (float)(g.thresh / (g.eps * g.eps)) * (1.0f + rel) : INFINITY;
-    const uint32_t nrows = pow3(k - 1);
-    // Lane l takes rows l, l + 64, l + 128, l + 192: each dependent step
-    // below (hash probe, row bounds, dim-0 window, cell bounds) issues the
-    // loads of all its rows at once, so a unit waits for ~6 round trips to
-    // memory instead of ~6 per group of 64 rows.
-    constexpr int R = (kMaxRows + 63) / 64;
-    uint64_t rkey[R];
-    uint32_t wlo[R], whi[R], slot[R];
-    bool want[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        const uint32_t r = (uint32_t)lane + 64u * i;
-        want[i] = false;
-        rkey[i] = 0;
-        wlo[i] = lo[0];
-        whi[i] = hi[0];
-        if (r >= nrows) continue;
-        // offset digits of row r along dims 1..k-1 (0: -1, 1: 0, 2: +1)
-        uint32_t o[kMaxK];
-        uint32_t rr = r;
-        bool inside = true;
-        uint64_t key = 0, mult = 1;
-#pragma unroll
-        for (int j = 1; j < kMaxK; j++) {
-            o[j] = rr % 3;
-            rr /= 3;
-            if ((uint32_t)j < k) {
-                const uint32_t cj = c[j] + o[j] - 1;  // wraps for c[j] == 0, rejected here
-                inside &= cj >= lo[j] && cj <= hi[j];
-                key += (uint64_t)cj * mult;
-                mult *= g.nCells[j];
-            }
-        }
-        if (!inside) continue;
-        // cell-box pruning: the row's squared box distance to the nearest
-        // query (mid: dim-0 offset 0; left / right: offset -1 / +1)
-        float mmid = 3.4e38f, mleft = 3.4e38f, mright = 3.4e38f;
-#pragma unroll 1
-        for (uint32_t qi = 0; qi < nq; qi++) {
-            float rd = 0.0f;
-#pragma unroll
-            for (int j = 1; j < kMaxK; j++) {
-                if ((uint32_t)j >= k) break;
-                const float2 v = rl.gap[qi * kMaxK + j];
-                rd += o[j] == 0 ? v.x : (o[j] == 2 ? v.y : 0.0f);
-            }
-            const float2 v0 = rl.gap[qi * kMaxK];
-            mmid = fminf(mmid, rd);
-            mleft = fminf(mleft, rd + v0.x);
-            mright = fminf(mright, rd + v0.y);
-        }
-        if (!(mmid <= thr)) continue;
-        if (!(mleft <= thr) && wlo[i] < c[0]) wlo[i] = c[0];
-        if (!(mright <= thr) && whi[i] > c[0]) whi[i] = c[0];
-        want[i] = true;
-        rkey[i] = key;
-    }
-    // hash probes: first slots together, collisions (rare) one by one
-    uint64_t hk[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        slot[i] = hash_slot(rkey[i]) & ix.hmask;
-        hk[i] = want[i] ? ix.hkeys[slot[i]] : ~0ull;
-    }
-    uint32_t row[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        uint32_t sl = slot[i];
-        uint64_t q = hk[i];
-        while (want[i] && q != rkey[i] && q != ~0ull) {
-            sl = (sl + 1) & ix.hmask;
-            q = ix.hkeys[sl];
-        }
-        slot[i] = sl;
-        want[i] = want[i] && q == rkey[i];
-    }
-#pragma unroll
-    for (int i = 0; i < R; i++) row[i] = want[i] ? ix.hvals[slot[i]] : 0u;
-    uint32_t rs[R], re[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        rs[i] = want[i] ? ix.row_start[row[i]] : 0u;
-        re[i] = want[i] ? ix.row_start[row[i] + 1] : 0u;
-    }
-    // dim-0 window [wlo, whi] inside the row: rows of up to 4 cells compare
-    // their keys loaded together, longer rows binary-search
-    constexpr int kShort = 4;
-    uint32_t ca[R], cb[R];
-    uint64_t ck[R][kShort];
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        const uint32_t len = re[i] - rs[i];
-#pragma unroll
-        for (int j = 0; j < kShort; j++)
-            ck[i][j] = (len > 0 && len <= (uint32_t)kShort) ? ix.cell_key[rs[i] + min((uint32_t)j, len - 1)] : 0ull;
-    }
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        const uint32_t len = re[i] - rs[i];
-        const uint64_t base = rkey[i] * g.nCells[0];
-        uint32_t na = 0, nb = 0;
-#pragma unroll
-        for (int j = 0; j < kShort; j++) {
-            na += ((uint32_t)j < len && ck[i][j] < base + wlo[i]) ? 1u : 0u;
-            nb += ((uint32_t)j < len && ck[i][j] <= base + whi[i]) ? 1u : 0u;
-        }
-        ca[i] = rs[i] + na;
-        cb[i] = rs[i] + nb;
-        if (len > (uint32_t)kShort) {
-            ca[i] = lower_bound_u64(ix.cell_key, rs[i], re[i], base + wlo[i]);
-            cb[i] = lower_bound_u64(ix.cell_key, ca[i], re[i], base + whi[i] + 1);
-        }
-    }
-    uint32_t pstart[R], plen[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        const bool any = cb[i] > ca[i];
-        pstart[i] = any ? ix.cell_start[ca[i]] : 0u;
-        plen[i] = any ? ix.cell_start[cb[i]] - pstart[i] : 0u;
-    }
-    // compact the non-empty rows, in row order, into the LDS list
-    uint32_t slots = 0, total = 0;
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-        if (64u * i >= nrows) break;
-        const uint64_t nz = __ballot(plen[i] > 0);
-        uint32_t x = plen[i];
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (plen[i] > 0) {
-            const uint32_t s = slots + lanes_below(nz);
-            rl.start[s] = pstart[i];
-            rl.off[s] = total + x - plen[i];
-        }
-        slots += (uint32_t)__popcll(nz);
-        total += __shfl(x, 63, 64);
-    }
-    if (lane == 0) rl.off[slots] = total;
-    *nslots = slots;
-    return total;
+    return stencil_rows<QB>(g, ix, rl, tb, b, (int64_t)b.c[0], a.prune ? nq : 0u, thr, nslots);
 }
 
 // Candidate position of flattened candidate index t (t < M), by binary search
 // over the slot prefix.
-__device__ __forceinline__ uint32_t cand_pos(const RowList &rl, uint32_t nslots, uint32_t t) {
+template <typename L>
+__device__ __forceinline__ uint32_t cand_pos(const L &rl, uint32_t nslots, uint32_t t) {
     uint32_t lo = 0, hi = nslots;  // last slot with off <= t
     while (hi - lo > 1) {
         uint32_t mid = (lo + hi) >> 1;
@@ -596,7 +453,7 @@ __device__ __forceinline__ void add_stats(const JoinArgs &a, unsigned long long 
 // registers); 1 above.
 template <int D, int QB>
 constexpr int join_min_waves() {
-    return (D > 0 && D <= 8 && QB <= 8) ? (q_in_sgprs<D, QB>() ? 4 : 2) : 1;
+    return (D > 0 && D <= 8 && QB <= 8) ? (q_in_sgprs<D, QB>() ? 4 : 2) : (D == 0 && QB == 4) ? 4 : 1;
 }
 
 // The exact FP64 chain for every dimensionality (the FP32 filter is
@@ -615,6 +472,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     RowList &rl = rls[wid];
     uint64_t *const hs_lds = hs_all[wid].w;
+    static_assert(sizeof(StencilTabs<QB>) <= sizeof(HitStore), "the build's tables share the masks' LDS");
     uint64_t *const hs_glb = a0.gmask + (uint64_t)(blockIdx.x * (blockDim.x >> 6) + wid) * a0.gmask_slots;
     const double T = a0.g.thresh;
     constexpr bool kRegs = (D > 0 && D <= kRegDims);
@@ -648,7 +506,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
             uint32_t nslots;
             bool live;
             const uint32_t M = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)build_rows<QB>(a, cell, rl, &nslots, &live, qpos0, nq));
+                (int)build_rows<QB>(a, cell, rl, *reinterpret_cast<StencilTabs<QB> *>(hs_lds), &nslots, &live, qpos0, nq));
             nslots = (uint32_t)__builtin_amdgcn_readfirstlane((int)nslots);
             // the unit's query coordinates, once: lane i loads element i
             if constexpr (kQS) {
@@ -962,7 +820,8 @@ __device__ __forceinline__ void wave_lds_order() {
 // off[s] and sets bit (off[s] - 1) % 64 of chunk (off[s] - 1) / 64.  S of
 // chunk c is the number of slots s >= 1 with off[s] <= 64 c: the slot of its
 // lane 0 (off[0] = 0 and the offsets increase strictly).
-__device__ __forceinline__ void build_tab(F32Lds &f, const RowList &rl, uint32_t nslots, uint32_t c0) {
+template <typename L>
+__device__ __forceinline__ void build_tab(F32Lds &f, const L &rl, uint32_t nslots, uint32_t c0) {
     const int lane = threadIdx.x & 63;
     wave_lds_order();
     f.tab[lane] = make_uint4(0u, 0u, 0u, 0u);
@@ -1042,6 +901,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
     RowList &rl = rls[wid];
     F32Lds &fl = fls[wid];
     uint64_t *const hs_lds = hs_all[wid].w;
+    static_assert(sizeof(StencilTabs<QB>) <= sizeof(HitStore), "the build's tables share the masks' LDS");
     uint64_t *const hs_glb = a0.gmask + (uint64_t)(blockIdx.x * (blockDim.x >> 6) + wid) * a0.gmask_slots;
     constexpr uint32_t kStride = D * (uint32_t)sizeof(float);
     constexpr uint32_t kChunkBytes = 64u * kStride;
@@ -1071,7 +931,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
             uint32_t nslots;
             bool live;
             const uint32_t M = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)build_rows<QB>(a, cell, rl, &nslots, &live, qpos0, nq));
+                (int)build_rows<QB>(a, cell, rl, *reinterpret_cast<StencilTabs<QB> *>(hs_lds), &nslots, &live, qpos0, nq));
             nslots = (uint32_t)__builtin_amdgcn_readfirstlane((int)nslots);
             // the unit's query coordinates, once (lane i loads element i);
             // padding queries are +inf
@@ -1400,25 +1260,21 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, 4) void k_join_f32(JoinArgs av
     add_stats(reload(args), sh_stats, my_evals, my_pairs, my_band);
 }
 
-// Per-cell candidate count over the stencil (sortByWorkLoadGlobal).
+// Per-cell candidate count over the stencil (sortByWorkLoadGlobal), one wave
+// per cell (one thread per cell walked its 243 rows one after the other:
+// 7.3 ms for the 1.85M cells of the 5M-point 6-D set).
 __global__ __launch_bounds__(256) void k_cell_workload(GridGeom g, DevIndex ix,
                                                        uint32_t *__restrict__ work) {
-    uint32_t cell = blockIdx.x * 256 + threadIdx.x;
-    if (cell >= ix.C) return;
-    uint32_t c[kMaxK], lo[kMaxK], hi[kMaxK];
-    decode_cell(ix.cell_key[cell], g, c);
-    bool ok = true;
-    for (uint32_t j = 0; j < g.k; j++) ok &= stencil_dim(c[j], g.nCells[j], g.emulate_cell0, &lo[j], &hi[j]);
-    uint32_t total = 0;
-    if (ok) {
-        uint32_t nrows = pow3(g.k - 1);
-        for (uint32_t r = 0; r < nrows; r++) {
-            uint32_t cf, cl;
-            stencil_row(c, lo, hi, r, g, ix, &cf, &cl);
-            if (cl > cf) total += ix.cell_start[cl] - ix.cell_start[cf];
-        }
+    __shared__ StencilList rls[4];
+    __shared__ StencilTabs<1> tabs[4];
+    const uint32_t wid = threadIdx.x >> 6, waves = gridDim.x * 4;
+    for (uint32_t cell = wave_bcast_u32(blockIdx.x * 4 + wid); cell < ix.C; cell += waves) {
+        CellBox b;
+        uint32_t slots, total = 0;
+        if (cell_box(g, ix, cell, b)) total = stencil_rows<1>(g, ix, rls[wid], tabs[wid], b, (int64_t)b.c[0], 0, INFINITY, &slots);
+        if ((threadIdx.x & 63) == 0) work[cell] = total;
+        wave_lds_sync();
     }
-    work[cell] = total;
 }
 
 // Units: cell c contributes ceil(|c| / qb) units when its stencil is live
@@ -1457,7 +1313,7 @@ __global__ __launch_bounds__(256) void k_unit_fill(DevIndex ix, uint32_t qb,
 // ---------------------------------------------------------------------------
 hegj_status launch_workload(const GridGeom &g, const DevIndex &ix, uint32_t *work, hipStream_t s) {
     if (ix.C == 0) return HEGJ_OK;
-    k_cell_workload<<<ceil_div(ix.C, 256), 256, 0, s>>>(g, ix, work);
+    k_cell_workload<<<std::min<uint32_t>(ceil_div(ix.C, 4), 8192), 256, 0, s>>>(g, ix, work);
     HIP_TRY(hipGetLastError());
     return HEGJ_OK;
 }

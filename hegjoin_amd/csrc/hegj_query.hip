@@ -27,7 +27,7 @@
 //                   no atomics, deterministic.
 #include <type_traits>
 
-#include "hegj_internal.h"
+#include "hegj_stencil.h"
 
 namespace hegj {
 
@@ -41,14 +41,7 @@ constexpr int kQWaves = 4;
 // and its registers spill.
 constexpr int kQB = 4;
 constexpr int kQBF32 = 4;
-constexpr int kMaxQB = 16;
 constexpr uint32_t kHitWords = kQueryHitWords;
-
-struct QRowList {
-    uint32_t start[kMaxRows];
-    uint32_t off[kMaxRows + 1];
-    float2 gap[kMaxQB * kMaxK];  // per (query, indexed dim): squared gaps to the -1 / +1 cell
-};
 
 __global__ __launch_bounds__(256) void k_qcell_keys(const double *__restrict__ q, uint32_t nq,
                                                     QueryGeom qg, uint64_t *__restrict__ keys,
@@ -124,24 +117,39 @@ __global__ __launch_bounds__(256) void k_sub_fill(const uint32_t *__restrict__ s
 // (FP32 sums), so the kept set can only be larger than the exact one.
 template <int QB>
 __device__ uint32_t qbuild_rows(const QJoinArgs &a, uint64_t key, const uint32_t *qid, uint32_t nqg,
-                                QRowList &rl, uint32_t *nslots) {
+                                StencilList &rl, StencilTabs<QB> &tb, uint32_t *nslots) {
     const GridGeom &g = a.qg.g;
     const int lane = threadIdx.x & 63;
-    uint32_t c[kMaxK], lo[kMaxK], hi[kMaxK];
-    int64_t cs[kMaxK];
+    // lane j takes coordinate j of the widened cell (-1 .. nCells): two
+    // divisions for all of them
+    int64_t cl = 0;
+    {
+        uint64_t stride = 1, w = 1;
+#pragma unroll
+        for (int j = 0; j < kMaxK; j++) {
+            if ((uint32_t)j >= g.k) break;
+            const uint64_t wj = (uint64_t)g.nCells[j] + 2;
+            if (lane > j) stride *= wj;
+            if (lane == j) w = wj;
+        }
+        if ((uint32_t)lane < g.k) cl = (int64_t)((key / stride) % w) - 1;
+    }
+    CellBox box;
+    int64_t c0 = 0;
     bool ok = true;
-    for (uint32_t j = 0; j < g.k; j++) {
-        const uint64_t w = (uint64_t)g.nCells[j] + 2;
-        const uint64_t qq = key / w;
-        const int64_t cj = (int64_t)(key - qq * w) - 1;  // -1 .. nCells
-        key = qq;
+#pragma unroll
+    for (int j = 0; j < kMaxK; j++) {
+        // a coordinate of -1 wraps; the offset is added modulo 2^32
+        box.c[j] = lane_u32((uint32_t)cl, j);
+        box.lo[j] = box.hi[j] = 0;
+        if ((uint32_t)j >= g.k) continue;
+        const int64_t cj = (int64_t)(((uint64_t)lane_u32((uint32_t)((uint64_t)cl >> 32), j) << 32) | box.c[j]);
+        if (j == 0) c0 = cj;
         const int64_t l = cj - 1 < 0 ? 0 : cj - 1;
         const int64_t h = cj + 1 > (int64_t)g.nCells[j] - 1 ? (int64_t)g.nCells[j] - 1 : cj + 1;
         ok &= l <= h;
-        c[j] = (uint32_t)cj;  // -1 wraps; stencil_row adds the offset modulo 2^32
-        cs[j] = cj;
-        lo[j] = (uint32_t)l;
-        hi[j] = (uint32_t)(h < 0 ? 0 : h);
+        box.lo[j] = (uint32_t)l;
+        box.hi[j] = (uint32_t)(h < 0 ? 0 : h);
     }
     if (!ok) {
         *nslots = 0;
@@ -153,88 +161,26 @@ __device__ uint32_t qbuild_rows(const QJoinArgs &a, uint64_t key, const uint32_t
     for (uint32_t e = (uint32_t)lane; e < nqg * k; e += 64) {
         const uint32_t qi = e / k, j = e - qi * k;
         uint32_t id = 0;
-        int64_t cj = 0;
 #pragma unroll
         for (int t = 0; t < QB; t++) id = (uint32_t)t == qi ? qid[t] : id;
+        uint32_t cu = 0;
+        double mn = 0.0;
 #pragma unroll
-        for (int jj = 0; jj < kMaxK; jj++) cj = (uint32_t)jj == j ? cs[jj] : cj;
+        for (int jj = 0; jj < kMaxK; jj++) {
+            cu = (uint32_t)jj == j ? box.c[jj] : cu;
+            mn = (uint32_t)jj == j ? g.minArr[jj] : mn;
+        }
+        const double cj = cu == ~0u ? -1.0 : (double)cu;  // (a grid has under 2^32 - 1 cells a dim with two more)
         const double x = a.queries[(uint64_t)id * dim + j];
-        double f = (x - g.minArr[j]) * inv_side - (double)cj;
+        double f = (x - mn) * inv_side - cj;
         f = f < 0.0 ? 0.0 : (f > 1.0 ? 1.0 : f);
-        const double mg = 1e-6 + 2e-15 * ((double)(cj < 0 ? -cj : cj) + 2.0);
+        const double mg = 1e-6 + 2e-15 * (fabs(cj) + 2.0);
         const double gm = f - mg > 0.0 ? f - mg : 0.0, gp = 1.0 - f - mg > 0.0 ? 1.0 - f - mg : 0.0;
-        rl.gap[qi * kMaxK + j] = make_float2((float)(gm * gm), (float)(gp * gp));
+        tb.gap[qi * kMaxK + j] = make_float2((float)(gm * gm), (float)(gp * gp));
     }
     wave_lds_sync();
     const float thr = (float)(a.thresh * inv_side * inv_side) * (1.0f + 1e-5f);
-    const uint32_t nrows = pow3(k - 1);
-    uint32_t slots = 0, total = 0;
-    for (uint32_t r0 = 0; r0 < nrows; r0 += 64) {
-        const uint32_t r = r0 + lane;
-        uint32_t pstart = 0, plen = 0;
-        if (r < nrows) {
-            // offset digits of row r along dims 1..k-1 (0: -1, 1: 0, 2: +1)
-            uint32_t o[kMaxK];
-            uint32_t rr = r;
-#pragma unroll
-            for (int j = 1; j < kMaxK; j++) {
-                o[j] = rr % 3;
-                rr /= 3;
-            }
-            float mmid = 3.4e38f, mleft = 3.4e38f, mright = 3.4e38f;
-            for (uint32_t qi = 0; qi < nqg; qi++) {
-                float rd = 0.0f;
-#pragma unroll
-                for (int j = 1; j < kMaxK; j++) {
-                    if ((uint32_t)j >= k) break;
-                    const float2 v = rl.gap[qi * kMaxK + j];
-                    rd += o[j] == 0 ? v.x : (o[j] == 2 ? v.y : 0.0f);
-                }
-                const float2 v0 = rl.gap[qi * kMaxK];
-                mmid = fminf(mmid, rd);
-                mleft = fminf(mleft, rd + v0.x);
-                mright = fminf(mright, rd + v0.y);
-            }
-            if (mmid <= thr) {
-                // dim-0 window, without the -1 / +1 cell when no query reaches it
-                int64_t wlo = lo[0], whi = hi[0];
-                if (!(mleft <= thr) && cs[0] > wlo) wlo = cs[0];
-                if (!(mright <= thr) && cs[0] < whi) whi = cs[0];
-                if (wlo <= whi) {
-                    uint32_t lo2[kMaxK], hi2[kMaxK];
-#pragma unroll
-                    for (int j = 0; j < kMaxK; j++) {
-                        lo2[j] = lo[j];
-                        hi2[j] = hi[j];
-                    }
-                    lo2[0] = (uint32_t)wlo;
-                    hi2[0] = (uint32_t)whi;
-                    uint32_t cf, cl;
-                    stencil_row(c, lo2, hi2, r, g, a.ix, &cf, &cl);
-                    if (cl > cf) {
-                        pstart = a.ix.cell_start[cf];
-                        plen = a.ix.cell_start[cl] - pstart;
-                    }
-                }
-            }
-        }
-        const uint64_t nz = __ballot(plen > 0);
-        uint32_t x = plen;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (plen > 0) {
-            const uint32_t s = slots + lanes_below(nz);
-            rl.start[s] = pstart;
-            rl.off[s] = total + x - plen;
-        }
-        slots += (uint32_t)__popcll(nz);
-        total += __shfl(x, 63, 64);
-    }
-    if (lane == 0) rl.off[slots] = total;
-    *nslots = slots;
+    const uint32_t total = stencil_rows<QB>(g, a.ix, rl, tb, box, c0, nqg, thr, nslots);
     wave_lds_sync();
     return total;
 }
@@ -250,9 +196,10 @@ __device__ uint32_t qbuild_rows(const QJoinArgs &a, uint64_t key, const uint32_t
 template <int D, bool FILL, bool F32 = false, int QB = kQB>
 __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_qjoin(QJoinArgs a) {
     static_assert(!F32 || D > 0, "FP32 filter needs a fixed dimensionality");
-    __shared__ QRowList rls[kQWaves];
+    __shared__ StencilList rls[kQWaves];
+    __shared__ StencilTabs<QB> tabs[kQWaves];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    QRowList &rl = rls[wid];
+    StencilList &rl = rls[wid];
     const uint32_t dim = D > 0 ? (uint32_t)D : a.qg.g.dim;
     const uint64_t n = a.qg.g.n;
     const double T = a.thresh;
@@ -277,7 +224,7 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                 cnt[qi] = 0;
             }
             uint32_t nslots;
-            const uint32_t M = qbuild_rows<QB>(a, ukey, qid, nqg, rl, &nslots);
+            const uint32_t M = qbuild_rows<QB>(a, ukey, qid, nqg, rl, tabs[wid], &nslots);
             // the group's query coordinates, once (lane i loads element i;
             // scalar registers), so no load in the candidate loop waits on
             // anything but the candidates
