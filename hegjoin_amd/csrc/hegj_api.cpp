@@ -622,6 +622,8 @@ struct JoinPlan {
     uint32_t waves = 4;  // waves per workgroup
     uint32_t parts = 1;
     uint32_t part_end[kMaxParts] = {};
+    uint32_t *runs = nullptr;  // runs of units of about equal work (units_per_grab 0)
+    uint32_t n_runs = 0;
     uint64_t capacity = 0;
     uint32_t chunk = 0;  // output entries a wave reserves at a time in the first batch
     double estimate_ms = 0;
@@ -635,7 +637,7 @@ struct JoinPlan {
     ~JoinPlan() {
         if (stream) (void)hipStreamSynchronize(stream);
         for (void *p : {(void *)units, (void *)units_next, (void *)units_tmp, (void *)deferred,
-                        (void *)d_ctr, (void *)d_ctr2, (void *)gmask})
+                        (void *)d_ctr, (void *)d_ctr2, (void *)gmask, (void *)runs})
             dev_free(p);
     }
 };
@@ -647,6 +649,9 @@ hegj_status alloc_rows(hegj_result *r, uint32_t n, hipStream_t s) {
     HIP_TRY(hipMemsetAsync(r->d_row_off, 0, (sizeof(uint64_t) + sizeof(uint32_t)) * (size_t)n, s));
     return HEGJ_OK;
 }
+
+// Runs per wave: enough that the last ones even out.
+constexpr uint32_t kRunsPerWave = 32;
 
 // About 32 grabs per wave keeps the queue atomics off the critical path.
 uint32_t grab_for(const JoinPlan &P, uint32_t nu) {
@@ -679,6 +684,15 @@ void set_parts(JoinArgs &x, uint32_t parts, const uint32_t *ends) {
         x.part_begin[p] = p == 0 ? 0u : ends[p - 1];
         x.part_end[p] = ends[p];
     }
+}
+
+// The queue of the plan's whole unit list: its runs, or grabs of `grab` units;
+// returns the workgroups to launch.
+uint32_t set_queue(JoinArgs &x, const JoinPlan &P, uint32_t grab) {
+    x.runs = P.runs;
+    x.units_per_grab = P.runs ? 1u : grab;
+    set_parts(x, P.parts, P.part_end);
+    return blocks_for(P, P.runs ? P.n_runs : P.U, x.units_per_grab);
 }
 
 JoinArgs base_args(const hegj_index *h, const hegj_join_opts &opts, const JoinPlan &P) {
@@ -748,7 +762,14 @@ hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, co
     // unit ranges per XCD, split by estimated work
     P.parts = opts.xcd_parts ? std::min<uint32_t>(opts.xcd_parts, kMaxParts) : kMaxParts;
     if (U < P.parts * 256) P.parts = 1;
-    HEGJ_TRY(split_units(h->ix, P.units, U, qb, h->d_work, P.parts, P.part_end, s));
+    if (opts.units_per_grab || all_cells || U == 0) {
+        HEGJ_TRY(split_units(h->ix, P.units, U, qb, h->d_work, P.parts, P.part_end, s));
+    } else {
+        P.n_runs = (uint32_t)std::min<uint64_t>(U, (uint64_t)P.max_blocks * P.waves * kRunsPerWave);
+        HIP_TRY(dev_malloc_n(&P.runs, (size_t)P.n_runs + 1));
+        HEGJ_TRY(unit_runs(h->ix, P.units, U, qb, h->g.dim, h->d_work, P.n_runs, P.runs, s));
+        for (uint32_t p = 0; p < P.parts; p++) P.part_end[p] = (uint32_t)((uint64_t)P.n_runs * (p + 1) / P.parts);
+    }
     // batch estimate: count-only pass over a strided sample of ~8192 units
     // (a few per cent of the join's work at most)
     P.capacity = opts.result_capacity;
@@ -767,8 +788,10 @@ hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, co
         e.units_per_grab = grab_for(P, ns);
         e.count_only = 1;
         e.gmask_slots = 0;
-        uint32_t one_end = ns;
-        set_parts(e, 1, &one_end);
+        // equal ranges: eight queues' lines instead of one
+        uint32_t ends[kMaxParts];
+        for (uint32_t p = 0; p < (uint32_t)kMaxParts; p++) ends[p] = (uint32_t)((uint64_t)ns * (p + 1) / kMaxParts);
+        set_parts(e, kMaxParts, ends);
         HEGJ_TRY(launch_join(e, qb, blocks_for(P, ns, e.units_per_grab), s));
         Counters c;
         HEGJ_TRY(read_back(&c, P.d_ctr, s));
@@ -881,12 +904,16 @@ struct BatchRunner {
             cleared = false;
             a.units = cur;
             a.n_units = cur_n;
-            a.units_per_grab = opts.units_per_grab ? opts.units_per_grab : grab_for(P, cur_n);
+            const uint32_t grab = opts.units_per_grab ? opts.units_per_grab : grab_for(P, cur_n);
+            uint32_t blocks;
             if (parts && cur == units && cur_n == P.U) {
-                set_parts(a, P.parts, P.part_end);
+                blocks = set_queue(a, P, grab);
             } else {
+                a.runs = nullptr;
+                a.units_per_grab = grab;
                 uint32_t one_end = cur_n;
                 set_parts(a, 1, &one_end);
+                blocks = blocks_for(P, cur_n, grab);
             }
             a.count_only = 0;
             // later batches are sized exactly, and launches that share a
@@ -894,7 +921,7 @@ struct BatchRunner {
             a.chunk = last && cur == units ? P.chunk : 0u;
             {
                 EventTimer t(s);
-                HEGJ_TRY(launch_join(a, qb, blocks_for(P, cur_n, a.units_per_grab), s));
+                HEGJ_TRY(launch_join(a, qb, blocks, s));
                 t.mark();
                 if (last) HEGJ_TRY(launch_pair_hash(a, capacity, s));
                 HEGJ_TRY(read_back(&c, P.d_ctr, s));
@@ -934,6 +961,7 @@ struct BatchRunner {
             JoinArgs e = a;
             e.units = cur;
             e.n_units = cur_n;
+            e.runs = nullptr;
             e.units_per_grab = grab_for(P, e.n_units);
             uint32_t one_end = e.n_units;
             set_parts(e, 1, &one_end);
@@ -1267,7 +1295,8 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
         G->qb = qb;
         HEGJ_TRY(make_plan(h, opts, qb, order, G->P));
         G->grab = opts.units_per_grab ? opts.units_per_grab : grab_for(G->P, G->P.U);
-        G->blocks = blocks_for(G->P, G->P.U, G->grab);
+        JoinArgs q{};
+        G->blocks = set_queue(q, G->P, G->grab);
         HIP_TRY(hipMalloc(&G->d_args, sizeof(JoinArgs)));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&G->h_args), sizeof(JoinArgs), hipHostMallocDefault));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&G->h_ctr), sizeof(Counters), hipHostMallocDefault));
@@ -1289,8 +1318,7 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
     a.row_cnt = r->d_row_cnt;
     a.units = G.P.units;
     a.n_units = G.P.U;
-    a.units_per_grab = G.grab;
-    set_parts(a, G.P.parts, G.P.part_end);
+    (void)set_queue(a, G.P, G.grab);
     a.out = buf;
     a.out_base = 0;
     a.capacity = G.P.capacity;

@@ -192,6 +192,8 @@ struct JoinArgs {
     const uint2 *units;           // (cell, first query offset in cell)
     uint32_t n_units;
     uint32_t units_per_grab;
+    const uint32_t *runs;         // grab i is units [runs[i], runs[i + 1]) (units_per_grab 1,
+                                  // ranges counted in runs); null: grabs of units_per_grab units
     uint32_t block_waves;        // waves per workgroup of the launch (host side)
     uint32_t n_parts;             // unit ranges; a workgroup starts on its XCD's range
     uint32_t part_by_xcc;         // 1: range = hardware XCC id, 0: blockIdx % n_parts
@@ -381,6 +383,10 @@ hegj_status morton_order(const GridGeom &g, const DevIndex &ix, uint32_t *order,
 hegj_status split_units(const DevIndex &ix, const uint2 *units, uint32_t n_units, uint32_t qb,
                         const uint32_t *work, uint32_t n_parts, uint32_t *part_end,
                         hipStream_t s);
+// Cuts the unit list into n_runs runs of about equal estimated time (dim
+// coordinates per distance); runs[n_runs + 1], some may be empty.
+hegj_status unit_runs(const DevIndex &ix, const uint2 *units, uint32_t n_units, uint32_t qb, uint32_t dim,
+                      const uint32_t *work, uint32_t n_runs, uint32_t *runs, hipStream_t s);
 hegj_status gather_units(const uint2 *in, const uint32_t *idx, uint32_t n, uint2 *out,
                          hipStream_t s);
 hegj_status csr_offsets(const uint32_t *row_cnt, uint32_t n, uint64_t *csr_off, hipStream_t s);

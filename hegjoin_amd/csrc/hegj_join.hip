@@ -358,7 +358,7 @@ struct Grabs {
     bool first = true;
 };
 
-__device__ __forceinline__ bool next_grab(const JoinArgs &a, Grabs &q, uint32_t &grab, uint32_t &gend) {
+__device__ __forceinline__ bool next_item(const JoinArgs &a, Grabs &q, uint32_t &grab, uint32_t &gend) {
     const int lane = threadIdx.x & 63;
     const uint32_t wpb = blockDim.x >> 6;
     if (q.first) {
@@ -392,6 +392,21 @@ __device__ __forceinline__ bool next_grab(const JoinArgs &a, Grabs &q, uint32_t 
         }
         q.part = p + 1 == a.n_parts ? 0 : p + 1;
         q.tries++;
+    }
+    return false;
+}
+
+// The units of the next grab: with a.runs an item is a run of units.  Runs
+// hold about equal work, so neighbouring light units, which share most of
+// their stencil and candidates, come to one wave and find them in its CU's L1,
+// while heavy units stay alone (6-D 5M, 2.4M units: 4 units a grab 31.3 ms, 8
+// 28.5, 16 31.7, 64 53: the first 64 dense units are the critical path).
+__device__ __forceinline__ bool next_grab(const JoinArgs &a, Grabs &q, uint32_t &grab, uint32_t &gend) {
+    while (next_item(a, q, grab, gend)) {
+        if (!a.runs) return true;
+        gend = wave_bcast_u32(a.runs[grab + 1]);
+        grab = wave_bcast_u32(a.runs[grab]);
+        if (grab < gend) return true;
     }
     return false;
 }

@@ -538,6 +538,52 @@ hegj_status morton_order(const GridGeom &g, const DevIndex &ix, uint32_t *order,
     return HEGJ_OK;
 }
 
+namespace {
+// A unit's time in vector instructions of a grid join: its stencil build and
+// bookkeeping, and per chunk of 64 candidates the loads and the distances.
+__global__ __launch_bounds__(256) void k_unit_time(const uint2 *__restrict__ units, uint32_t n,
+                                                   const uint32_t *__restrict__ cell_start,
+                                                   const uint32_t *__restrict__ work, uint32_t qb, uint32_t dim,
+                                                   uint64_t *__restrict__ w) {
+    const uint32_t u = blockIdx.x * 256 + threadIdx.x;
+    if (u >= n) return;
+    const uint2 un = units[u];
+    const uint32_t nq = min(qb, cell_start[un.x + 1] - cell_start[un.x] - un.y);
+    w[u] = 1500ull + (uint64_t)((work[un.x] + 63) / 64) * (20u + nq * (2u * dim + 6u));
+}
+
+__global__ __launch_bounds__(256) void k_find_runs(const uint64_t *__restrict__ prefix, uint32_t n,
+                                                   const uint64_t *__restrict__ total, uint32_t n_runs,
+                                                   uint32_t *__restrict__ runs) {
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    if (r > n_runs) return;
+    const uint64_t target = (uint64_t)((double)*total * ((double)r / (double)n_runs));
+    uint32_t lo = 0, hi = r == n_runs ? 0 : n;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (prefix[mid] < target)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    runs[r] = r == n_runs ? n : lo;
+}
+}  // namespace
+
+hegj_status unit_runs(const DevIndex &ix, const uint2 *units, uint32_t n_units, uint32_t qb, uint32_t dim,
+                      const uint32_t *work, uint32_t n_runs, uint32_t *runs, hipStream_t s) {
+    Scratch sc;
+    uint64_t *w, *total;
+    HIP_TRY(sc.get(&w, n_units));
+    HIP_TRY(sc.get(&total, 1));
+    k_unit_time<<<ceil_div(n_units, 256), 256, 0, s>>>(units, n_units, ix.cell_start, work, qb, dim, w);
+    HIP_TRY(hipGetLastError());
+    HEGJ_TRY(scan_u64(w, w, n_units, total, s));
+    k_find_runs<<<ceil_div((uint64_t)n_runs + 1, 256), 256, 0, s>>>(w, n_units, total, n_runs, runs);
+    HIP_TRY(hipGetLastError());
+    return scratch_done(s);
+}
+
 hegj_status split_units(const DevIndex &ix, const uint2 *units, uint32_t n_units, uint32_t qb,
                         const uint32_t *work, uint32_t n_parts, uint32_t *part_end,
                         hipStream_t s) {

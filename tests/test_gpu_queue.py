@@ -25,7 +25,7 @@ def test_unit_distribution(H, oracle, n, dim):
     print("case", n, dim, len(enb), flush=True)
     with H.GridIndex(pts, eps) as ix:
         for parts in (1, 3, 8):
-            for grab in (1, 3, 64):
+            for grab in (0, 1, 3, 64):
                 for waves in (1, 2, 4):
                     for by_block in (0, 1):
                         t = ix.selfjoin(xcd_parts=parts, units_per_grab=grab, block_waves=waves,
