@@ -284,7 +284,8 @@ typedef struct {
     uint32_t reserved;
     uint64_t estimated_pairs;  /* the batch estimator's pair estimate ("[GPU | RESULT] ~
                                   Total estimated workload", GPU.cu:635); the MFMA
-                                  refine sizes its output exactly, so it reports that */
+                                  refine and joins of up to 2^27 candidates size
+                                  their output without it and report the pairs */
 } hegj_result_info;
 hegj_status hegj_result_get_info(const hegj_result *res, hegj_result_info *info);
 
