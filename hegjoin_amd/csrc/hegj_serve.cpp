@@ -11,8 +11,8 @@
 //     a request that arrives while others run is taken by the next free slot
 //     and its kernels overlap with theirs on the device;
 //   * per request: count pass -> exact result size -> admission into the
-//     result-buffer pool (first come, first served) -> fill pass writing CSR
-//     rows in place.  Results stay in the pool until released.
+//     result-buffer pool (in the order of submission, see admit) -> fill pass
+//     writing CSR rows in place.  Results stay in the pool until released.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
@@ -21,6 +21,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <thread>
 #include <vector>
 
@@ -122,9 +123,10 @@ struct hegj_server {
     std::mutex mu;
     std::condition_variable cv_work, cv_done, cv_mem;
     std::deque<Request *> pending;
-    // counted requests waiting for pool memory, served first come, first
-    // served (a request still counting does not hold up later ones)
+    // counted requests waiting for pool memory, in the order of submission,
+    // and the tickets of the running requests that are not counted yet
     std::deque<Request *> mem_wait;
+    std::set<uint64_t> counting;
     std::map<uint64_t, std::unique_ptr<Request>> reqs;
     uint64_t next_ticket = 1;
     bool stopping = false;
@@ -143,14 +145,30 @@ struct hegj_server {
 
 namespace {
 
+// Pool memory for a counted request.  Memory goes to the waiting requests in
+// the order of submission; a request still counting holds up later ones only
+// once half of the pool is taken.  So a client that collects its results in
+// the order it submitted them is served whatever the order in which the counts
+// end, as long as no result is larger than half of the pool: before, the later
+// requests' results could take all of it, and were not released before the
+// earlier one was done.
 hegj_status admit(hegj_server *S, Request *r, uint64_t bytes) {
     std::unique_lock<std::mutex> lk(S->mu);
+    S->counting.erase(r->ticket);
+    S->cv_mem.notify_all();
     if (bytes > S->pool.cap)
         return fail(HEGJ_ERR_CAPACITY, "request result (" + std::to_string(bytes) +
                                            " bytes) exceeds the result-buffer pool");
     uint64_t off = 0;
-    S->mem_wait.push_back(r);
-    S->cv_mem.wait(lk, [&] { return S->mem_wait.front() == r && S->pool.alloc(bytes, &off); });
+    S->mem_wait.insert(std::find_if(S->mem_wait.begin(), S->mem_wait.end(),
+                                    [&](const Request *o) { return o->ticket > r->ticket; }),
+                       r);
+    S->cv_mem.wait(lk, [&] {
+        if (S->mem_wait.front() != r) return false;
+        const bool passes = !S->counting.empty() && *S->counting.begin() < r->ticket;
+        if (passes && S->pool.in_use + align_up(bytes) > S->pool.cap / 2) return false;
+        return S->pool.alloc(bytes, &off);
+    });
     S->mem_wait.pop_front();
     r->holds_pool = true;
     r->pool_off = off;
@@ -273,6 +291,7 @@ void hegj_server::worker(uint32_t slot) {
             r = pending.front();
             pending.pop_front();
             r->state = kRunning;
+            counting.insert(r->ticket);
             r->t_start = Clock::now();
         }
         hegj_status st = init_err.empty() ? run(r, s, arena, ctr) : fail(HEGJ_ERR_HIP, init_err);
@@ -291,6 +310,8 @@ void hegj_server::worker(uint32_t slot) {
                 last_done = r->t_done;
             } else {
                 r->state = kFailed;
+                counting.erase(r->ticket);
+                cv_mem.notify_all();
                 r->status = st;
                 r->error = msg;
                 failed++;

@@ -418,8 +418,9 @@ hegj_status hegj_result_copy_csr(const hegj_result *res, uint64_t *offsets, uint
  * others run start as soon as a slot frees up (continuous batching).  Each
  * request first counts its result exactly, then is admitted into the
  * result-buffer pool of `result_bytes` when its result fits (requests that
- * wait for memory are served first come, first served; a request whose
- * count finishes early does not wait for earlier ones still counting).
+ * wait for memory are served in the order of submission; a request whose
+ * count finishes early waits for earlier ones still counting only once half
+ * of the pool is taken).
  * Results stay in the pool until released, so a client should release
  * finished results (hegj_serve_poll) rather than hold them while waiting for
  * another request.  A request whose result alone is larger than the pool
