@@ -318,8 +318,11 @@ struct QueryGeom {
 struct QueryPlan {
     uint64_t *keys = nullptr;    // [nq] sorted widened cell keys
     uint32_t *ids = nullptr;     // [nq] query ids in key order
-    uint32_t *starts = nullptr;  // [n_units + 1] first sorted slot of each unit
-    uint32_t nq = 0, n_units = 0, n_live = 0;
+    uint2 *items = nullptr;      // units of up to 4 queries of one cell, or segments of them
+    uint32_t *counts = nullptr;  // [nq] zeroed
+    uint32_t *seg_counts = nullptr;  // [4 * items], where units may be split
+    uint32_t n_items = 0;        // at most this many where items_dev holds the number
+    uint32_t *items_dev = nullptr;
 };
 struct QJoinArgs {
     QueryGeom qg;
@@ -327,11 +330,13 @@ struct QJoinArgs {
     const double *queries;       // [nq * dim] row-major
     const uint64_t *keys;
     const uint32_t *ids;
-    const uint32_t *starts;
-    uint32_t n_units;
+    const uint2 *items;
+    uint32_t n_items;
+    const uint32_t *items_dev;   // the number of items, where the host does not know it
     uint32_t *queue_head;        // zeroed before each launch
     double thresh;               // largest s with sqrt(s) <= eps of the request
     uint32_t *counts;            // [nq] (count pass)
+    uint32_t *seg_counts;        // [4 * items] of split units: written by the count pass, read by the fill pass
     const uint64_t *offsets;     // [nq + 1] (fill pass)
     uint32_t *out;               // neighbour ids (fill pass)
     unsigned long long *hash;
@@ -357,8 +362,8 @@ hegj_status query_to_f32(const double *q, uint32_t nq, uint32_t dim, const doubl
 const GridGeom &index_geom(const hegj_index *h);
 const DevIndex &index_dev(const hegj_index *h);
 hegj_status select_device(int device);
-// Sort the queries by cell and build the units; the plan's arrays come from `keep`.
-hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const double *queries,
+// Sort the queries by cell and build the items; the plan's arrays come from `keep`.
+hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const DevIndex &ix, const double *queries,
                        uint32_t nq, hipStream_t s);
 hegj_status query_run(const QJoinArgs &a, bool fill, int device, hipStream_t s);
 // *hash += sum of mix64(query << 32 | neighbour) over the CSR rows

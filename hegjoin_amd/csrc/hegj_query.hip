@@ -16,9 +16,11 @@
 //                   on each side (coordinates -1 .. nCells), or `dead` when
 //                   the query lies further out (no point can be in range);
 //   radix sort      (key, query id), dead keys last;
-//   k_qruns         one unit per run of equal keys (up to 16 queries of one
-//                   cell); each group of 4 of them builds its stencil rows,
-//                   pruned to the cells within eps of one of its queries;
+//   items           units of up to 4 queries of one cell, heavy ones split into
+//                   segments of their candidates; each builds its stencil
+//                   rows, pruned to the cells within eps of one of its queries
+//                   (requests of at most 4096 queries: these three steps in
+//                   three launches, without a readback);
 //   k_qjoin<count>  per-query neighbour counts, and per group a bitmap of the
 //                   candidate chunks in which one of its queries has a hit;
 //   scan            CSR offsets, exact result size (admission happens here);
@@ -84,24 +86,213 @@ __global__ __launch_bounds__(256) void k_qrun_fill(const uint32_t *__restrict__ 
     if (i < nq && flag[i]) starts[rank[i]] = i;
 }
 
-// Units of at most kUnitQueries queries: a run of queries sharing a cell is
-// split so that a dense cell spreads over many waves instead of one.
-constexpr uint32_t kUnitQueries = 16;
+// A unit is one group: at most kQB queries of one cell, so the groups of a
+// dense cell go to different waves (with units of four groups the heaviest
+// unit was the request's critical path: 6-D, 10M points, 150k queries, with
+// the sweeps by group size below, count pass 13.5 -> 6.4 ms, fill 5.8 -> 3.1).
+constexpr uint32_t kUnitQueries = kQB;
+static_assert(kQB == kQBF32, "a unit is one group on either path");
 
-__global__ __launch_bounds__(256) void k_sub_counts(const uint32_t *__restrict__ starts, uint32_t nr,
-                                                    uint32_t *__restrict__ cnt) {
-    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
-    if (r < nr) cnt[r] = (starts[r + 1] - starts[r] + kUnitQueries - 1) / kUnitQueries;
+// An item is a unit, or one of up to 16 equal segments of a unit's candidates
+// where the unit looks heavy: a request of fewer units than the chip's 3072
+// resident waves takes as long as its densest group.  Each wave builds the
+// group's rows for itself (about 20 us at 6-D), so a segment is meant to have
+// kSegCandidates.  A unit's candidates are estimated from the points of its
+// home row's three cells, times the 3^(k-1) rows of the stencil, of which the
+// box pruning leaves a share that falls with k (0.25 at 6-D).  6-D, 2M points,
+// 3000 queries: request 0.78 -> 0.43 ms, 12000 queries 1.33 -> 0.84; segments
+// of 2048 measured 0.47 and 0.89.
+// .x = first sorted query, .y = segment | segments << 8 | queries << 16.
+constexpr uint32_t kMaxSegments = 16;
+constexpr float kSegCandidates = 4096.0f;
+
+__device__ uint32_t unit_segments(const QueryGeom &qg, const DevIndex &ix, uint64_t key, uint32_t min_seg, uint32_t max_seg) {
+    if (max_seg <= min_seg) return max_seg;
+    const GridGeom &g = qg.g;
+    uint64_t rkey = 0, mult = 1;
+    int64_t c0 = 0;
+    float rows = 1.0f;
+    for (uint32_t j = 0; j < g.k; j++) {
+        const uint64_t w = (uint64_t)g.nCells[j] + 2, rest = key / w;
+        const int64_t c = (int64_t)(key - rest * w) - 1;
+        key = rest;
+        if (j == 0) {
+            c0 = c;
+            continue;
+        }
+        if (c < 0 || c >= (int64_t)g.nCells[j]) return min_seg;
+        rkey += (uint64_t)c * mult;
+        mult *= g.nCells[j];
+        rows *= 3.0f;
+    }
+    uint32_t a, e;
+    if (!row_lookup(ix.hrows, ix.hmask, rkey, &a, &e)) return min_seg;
+    // the row's cells by coordinate 0: [c0 - 1, c0 + 1]
+    auto lower = [&](int64_t v) {
+        uint32_t lo = a, hi = e;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if ((int64_t)ix.cell_xyz[mid] < v)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return lo;
+    };
+    const uint32_t first = lower(c0 - 1), last = lower(c0 + 2);
+    const float est = (float)(ix.cell_start[last] - ix.cell_start[first]) * rows * (1.15f - 0.15f * (float)g.k);
+    return min(max((uint32_t)fminf(est / kSegCandidates, 1024.0f), min_seg), max_seg);
 }
 
-__global__ __launch_bounds__(256) void k_sub_fill(const uint32_t *__restrict__ starts, uint32_t nr,
-                                                  const uint32_t *__restrict__ first,
-                                                  uint32_t *__restrict__ sub) {
+__device__ __forceinline__ uint2 make_item(uint32_t g0, uint32_t nqg, uint32_t seg, uint32_t nseg) {
+    return make_uint2(g0, seg | nseg << 8 | nqg << 16);
+}
+
+// ---- requests of at most kSmallPlan queries: the plan in three launches ----
+// The general plan (a radix sort of up to 8 passes, two scans, two readbacks)
+// is about 40 launches, 0.25 ms of a 1 ms request; here each key's place is
+// its rank among all of them, and nothing is read back: the join reads the
+// number of units on the device.
+constexpr uint32_t kSmallPlan = 4096;
+constexpr uint32_t kSmallScan = 16384;  // counts scanned by one workgroup
+// Largest number of items that splitting may make of a request (131072
+// measured the same within 5% either way).
+constexpr uint32_t kSplitItems = 49152;
+// A request of fewer items leaves waves idle whatever it does: its units are
+// split, up to 8 times, without asking for their weight (20 queries: 0.18 ms
+// without, 0.13 with; at 2048 items 500 queries took 0.27 ms instead of 0.245).
+constexpr uint32_t kSpareItems = 1024;
+
+// place[i] = keys below keys[i] + equal keys before i (the stable sort's
+// order); the second term also says which queries begin a unit.  64 queries
+// a workgroup, its four waves a quarter of the keys each: bound by the LDS
+// broadcasts (a key and its compare for every lane), 4096 keys 12 us.
+__global__ __launch_bounds__(256) void k_qsmall_rank(const uint64_t *__restrict__ keys, uint32_t nq, QueryGeom qg,
+                                                     DevIndex ix, uint32_t min_seg, uint32_t max_seg,
+                                                     uint64_t *__restrict__ skeys,
+                                                     uint32_t *__restrict__ sids, uint32_t *__restrict__ flags,
+                                                     uint32_t *__restrict__ counts) {
+    __shared__ uint64_t sh[kSmallPlan];
+    __shared__ uint32_t part[2][4][64];
+    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (uint32_t j = threadIdx.x; j < nq; j += 256) sh[j] = keys[j];
+    __syncthreads();
+    const uint32_t i = blockIdx.x * 64 + lane;
+    const uint64_t k = sh[min(i, nq - 1)];
+    const uint32_t per = (nq + 3) / 4, b = min(w * per, nq), e = min(b + per, nq);
+    uint32_t below = 0, before = 0;
+#pragma unroll 8
+    for (uint32_t j = b; j < e; j++) {
+        const uint64_t o = sh[j];
+        below += o < k;
+        before += o == k && j < i;
+    }
+    part[0][w][lane] = below;
+    part[1][w][lane] = before;
+    __syncthreads();
+    if (w != 0 || i >= nq) return;
+    below = part[0][0][lane] + part[0][1][lane] + part[0][2][lane] + part[0][3][lane];
+    before = part[1][0][lane] + part[1][1][lane] + part[1][2][lane] + part[1][3][lane];
+    const uint32_t at = below + before;
+    skeys[at] = k;
+    sids[at] = i;
+    // 2: live, 1: first of a unit, with the unit's segments above
+    uint32_t f = k == qg.dead_key ? 0 : 2u;
+    if (f && before % kUnitQueries == 0) f |= 1u | unit_segments(qg, ix, k, min_seg, max_seg) << 8;
+    flags[at] = f;
+    counts[i] = 0;
+}
+
+// Exclusive prefix of one value per thread over a workgroup of 1024.
+__device__ uint64_t block_prefix(uint64_t v, uint64_t *sh, uint64_t *total) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint64_t x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) sh[w] = x;
+    __syncthreads();
+    uint64_t base = 0, all = 0;
+    for (int i = 0; i < 16; i++) {
+        base += i < w ? sh[i] : 0;
+        all += sh[i];
+    }
+    *total = all;
+    return base + x - v;
+}
+
+// The items and their number from the flags in sorted order.
+__global__ __launch_bounds__(1024) void k_qsmall_items(const uint32_t *__restrict__ flags, uint32_t nq,
+                                                       uint2 *__restrict__ items, uint32_t *__restrict__ n_items) {
+    constexpr uint32_t kPer = kSmallPlan / 1024;
+    __shared__ uint64_t sh[16];
+    const uint32_t i0 = threadIdx.x * kPer;
+    uint32_t f[kPer + kUnitQueries - 1], mine = 0;
+#pragma unroll
+    for (uint32_t t = 0; t < kPer + kUnitQueries - 1; t++) {
+        f[t] = i0 + t < nq ? flags[i0 + t] : 0;
+        if (t < kPer) mine += f[t] >> 8;
+    }
+    uint64_t total;
+    uint32_t o = (uint32_t)block_prefix(mine, sh, &total);
+#pragma unroll
+    for (uint32_t t = 0; t < kPer; t++) {
+        uint32_t nqg = 1;
+        bool more = true;
+#pragma unroll
+        for (uint32_t x = 1; x < kUnitQueries; x++) {
+            more = more && (f[t + x] & 3) == 2;
+            nqg += more;
+        }
+        for (uint32_t seg = 0; seg < f[t] >> 8; seg++) items[o++] = make_item(i0 + t, nqg, seg, f[t] >> 8);
+    }
+    if (threadIdx.x == 0) *n_items = (uint32_t)total;
+}
+
+// CSR offsets of at most kSmallScan counts in one workgroup.
+__global__ __launch_bounds__(1024) void k_qsmall_offsets(const uint32_t *__restrict__ counts, uint32_t nq,
+                                                         uint64_t *__restrict__ offsets) {
+    constexpr uint32_t kPer = kSmallScan / 1024;
+    __shared__ uint64_t sh[16];
+    const uint32_t i0 = threadIdx.x * kPer;
+    uint32_t c[kPer];
+    uint64_t mine = 0, total;
+#pragma unroll
+    for (uint32_t t = 0; t < kPer; t++) {
+        c[t] = i0 + t < nq ? counts[i0 + t] : 0;
+        mine += c[t];
+    }
+    uint64_t o = block_prefix(mine, sh, &total);
+#pragma unroll
+    for (uint32_t t = 0; t < kPer; t++) {
+        if (i0 + t < nq) offsets[i0 + t] = o;
+        o += c[t];
+    }
+    if (threadIdx.x == 0) offsets[nq] = total;
+}
+
+// Items of each run of queries sharing a cell: its units times their segments.
+__global__ __launch_bounds__(256) void k_item_counts(const uint32_t *__restrict__ starts, uint32_t nr,
+                                                     const uint64_t *__restrict__ keys, QueryGeom qg, DevIndex ix,
+                                                     uint32_t max_seg, uint32_t *__restrict__ nseg,
+                                                     uint32_t *__restrict__ cnt) {
     const uint32_t r = blockIdx.x * 256 + threadIdx.x;
     if (r >= nr) return;
-    const uint32_t b = starts[r], e = starts[r + 1];
+    nseg[r] = unit_segments(qg, ix, keys[starts[r]], 1, max_seg);
+    cnt[r] = (starts[r + 1] - starts[r] + kUnitQueries - 1) / kUnitQueries * nseg[r];
+}
+
+__global__ __launch_bounds__(256) void k_item_fill(const uint32_t *__restrict__ starts, uint32_t nr,
+                                                   const uint32_t *__restrict__ nseg,
+                                                   const uint32_t *__restrict__ first,
+                                                   uint2 *__restrict__ items) {
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= nr) return;
+    const uint32_t b = starts[r], e = starts[r + 1], ns = nseg[r];
     uint32_t o = first[r];
-    for (uint32_t i = b; i < e; i += kUnitQueries) sub[o++] = i;
+    for (uint32_t i = b; i < e; i += kUnitQueries)
+        for (uint32_t seg = 0; seg < ns; seg++) items[o++] = make_item(i, min(kUnitQueries, e - i), seg, ns);
 }
 
 // Stencil rows of a group of queries (all in the cell whose widened key is
@@ -185,6 +376,14 @@ __device__ uint32_t qbuild_rows(const QJoinArgs &a, uint64_t key, const uint32_t
     return total;
 }
 
+// The kernel arguments, to be read again from here on: kept live through a
+// unit's loops they would be spilled to vector lanes.
+typedef __attribute__((address_space(4))) const QJoinArgs *QArgsPtr;
+__device__ __forceinline__ const QJoinArgs &reload(QArgsPtr p) {
+    __asm__ volatile("" : "+s"(p));
+    return *(const QJoinArgs *)p;
+}
+
 // D > 0: coordinates in registers; D == 0: any dimensionality, one
 // dimension at a time.
 // F32: candidates from the level's centred FP32 copy, queries from the
@@ -194,26 +393,30 @@ __device__ uint32_t qbuild_rows(const QJoinArgs &a, uint64_t key, const uint32_t
 // candidate loads of too few waves are in flight (6-D, 10M points, 93k
 // queries: 290 -> 270 ms per request).
 template <int D, bool FILL, bool F32 = false, int QB = kQB>
-__global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_qjoin(QJoinArgs a) {
+__global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_qjoin(QJoinArgs) {
     static_assert(!F32 || D > 0, "FP32 filter needs a fixed dimensionality");
     __shared__ StencilList rls[kQWaves];
     __shared__ StencilTabs<QB> tabs[kQWaves];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     StencilList &rl = rls[wid];
-    const uint32_t dim = D > 0 ? (uint32_t)D : a.qg.g.dim;
-    const uint64_t n = a.qg.g.n;
-    const double T = a.thresh;
-    const double *__restrict__ soa = a.ix.soa;
+    const QArgsPtr args = (QArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    __shared__ unsigned long long sh_stats[2];
+    if (threadIdx.x < 2) sh_stats[threadIdx.x] = 0;
+    __syncthreads();
     uint64_t my_evals = 0, my_band = 0;
-    while (true) {
-        uint32_t u = 0;
-        if (lane == 0) u = atomicAdd(a.queue_head, 1u);
-        u = __shfl(u, 0, 64);
-        if (u >= a.n_units) break;
-        const uint32_t s0 = a.starts[u], s1 = a.starts[u + 1];
-        const uint64_t ukey = a.keys[s0];
-        for (uint32_t g0 = s0; g0 < s1; g0 += QB) {
-            const uint32_t nqg = min((uint32_t)QB, s1 - g0);
+    uint32_t n_items;
+    {
+        const QJoinArgs &a = reload(args);
+        n_items = a.items_dev ? *a.items_dev : a.n_items;
+    }
+    // the first item of a wave is its number, the others come from the queue
+    for (uint32_t w = blockIdx.x * kQWaves + wid; w < n_items;) {
+        const QJoinArgs &a = reload(args);
+        const uint32_t dim = D > 0 ? (uint32_t)D : a.qg.g.dim;
+        const uint2 item = a.items[w];
+        const uint32_t g0 = wave_bcast_u32(item.x), iy = wave_bcast_u32(item.y);
+        const uint32_t seg = iy & 0xFF, nseg = (iy >> 8) & 0xFF, nqg = iy >> 16;
+        {
             uint32_t qid[QB];
             uint64_t base[QB];
             uint32_t cnt[QB];
@@ -223,8 +426,15 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                 base[qi] = FILL ? a.offsets[qid[qi]] : 0;
                 cnt[qi] = 0;
             }
+            if (FILL && seg > 0) {  // behind the unit's segments before this one
+                uint32_t v = (uint32_t)lane / QB < seg ? a.seg_counts[(uint64_t)(w - seg) * QB + lane] : 0;
+#pragma unroll
+                for (int o = QB; o < 64; o *= 2) v += __shfl_xor(v, o, 64);
+#pragma unroll
+                for (int qi = 0; qi < QB; qi++) base[qi] += lane_u32(v, qi);
+            }
             uint32_t nslots;
-            const uint32_t M = qbuild_rows<QB>(a, ukey, qid, nqg, rl, tabs[wid], &nslots);
+            const uint32_t M = qbuild_rows<QB>(a, a.keys[g0], qid, nqg, rl, tabs[wid], &nslots);
             // the group's query coordinates, once (lane i loads element i;
             // scalar registers), so no load in the candidate loop waits on
             // anything but the candidates
@@ -264,8 +474,23 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                     qreg[j / DQ][j % DQ] = __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
                 }
             }
+            // this wave's segment of the candidates, in whole chunks
+            const uint32_t nch_all = (M + 63) / 64;
+            const uint32_t per = nseg > 1 ? (nch_all + nseg - 1) / nseg : nch_all;
+            const uint32_t clo = min(seg * per, nch_all), nch = min(clo + per, nch_all);
+            const uint32_t mend = min(M, nch * 64);
             SlotCursor cur;
             cur.reset(rl);
+            // NQ >= nqg queries evaluated: most cells of a sparse request hold
+            // a single query (72% of the groups of 150k queries over 10M 6-D
+            // points), and a group's unused places would cost as much as its
+            // queries.
+            auto sweep = [&](auto nqc) __attribute__((always_inline)) {
+            constexpr int NQ = decltype(nqc)::value;
+            const QJoinArgs &a = reload(args);
+            const uint64_t n = a.qg.g.n;
+            const double T = a.thresh;
+            const double *__restrict__ soa = a.ix.soa;
             if constexpr (D > 0) {
                 // Candidate chunks kDepth ahead in a register ring (coordinates,
                 // positions and, when filling, point ids), so a wave keeps
@@ -278,7 +503,7 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                 uint32_t posr[kDepth], pidr[kDepth];
                 auto load = [&](uint32_t t0, int p) __attribute__((always_inline)) {
                     const uint32_t t = t0 + lane;
-                    const uint32_t pos = t < M ? cur.pos(rl, t) : 0u;
+                    const uint32_t pos = t < mend ? cur.pos(rl, t) : 0u;
                     posr[p] = pos;
                     if constexpr (F32) {
                         if constexpr (DQ % 2 == 0) {
@@ -309,12 +534,12 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                 // `span` chunks.  The count pass sets the bits of chunks in
                 // which some query of the group has a neighbour; the fill
                 // pass, which does the same arithmetic, visits only those.
-                const uint32_t nch = (M + 63) / 64;
-                uint64_t *hb = a.hitbits ? a.hitbits + (uint64_t)g0 * kHitWords : nullptr;
-                const uint32_t capb = nqg * kHitWords * 64;
-                const uint32_t span = nch > capb ? (nch + capb - 1) / capb : 1u;
-                const uint32_t nw = ((nch + span - 1) / span + 63) / 64;
-                uint32_t cur = 0, cend = 0, wi = 0, bitpos = 0, subc = 0;
+                const uint32_t words = nqg * kHitWords / nseg, nown = nch - clo;
+                uint64_t *hb = a.hitbits ? a.hitbits + (uint64_t)g0 * kHitWords + seg * words : nullptr;
+                const uint32_t capb = words * 64;
+                const uint32_t span = nown > capb ? (nown + capb - 1) / capb : 1u;
+                const uint32_t nw = ((nown + span - 1) / span + 63) / 64;
+                uint32_t cur = clo, cend = 0, wi = 0, bitpos = 0, subc = 0;
                 uint64_t w = (FILL && hb && nw > 0) ? hb[0] : 0ull, hitw = 0;
                 // next chunk to visit (nch when none is left)
                 auto next = [&]() __attribute__((always_inline)) -> uint32_t {
@@ -326,7 +551,7 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                     }
                     const uint32_t b = wi * 64 + (uint32_t)__builtin_ctzll(w);
                     w &= w - 1;
-                    cur = b * span;
+                    cur = clo + b * span;
                     cend = min(cur + span, nch);
                     return cur;
                 };
@@ -341,13 +566,13 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                     for (int p = 0; p < kDepth; p++) {
                         const uint32_t ch = chr[p];
                         const uint32_t t0 = ch * 64;
-                        const bool valid = t0 + lane < M;
+                        const bool valid = t0 + lane < mend;
                         const uint64_t vmask = __builtin_amdgcn_ballot_w64(valid);
                         const uint32_t pos = posr[p];
                         const uint32_t pid = FILL ? pidr[p] : 0u;
-                        CT accv[QB];
+                        CT accv[NQ];
 #pragma unroll
-                        for (int qi = 0; qi < QB; qi++) {
+                        for (int qi = 0; qi < NQ; qi++) {
                             accv[qi] = (CT)0;
 #pragma unroll
                             for (int l = 0; l < DQ; l++) {
@@ -361,12 +586,12 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                             }
                         }
 #pragma unroll
-                        for (int qi = 0; qi < QB; qi++) __asm__ volatile("" ::"v"(accv[qi]) : "memory");
+                        for (int qi = 0; qi < NQ; qi++) __asm__ volatile("" ::"v"(accv[qi]) : "memory");
                         chr[p] = next();
                         load(chr[p] * 64, p);
                         uint64_t anyhit = 0;
 #pragma unroll
-                        for (int qi = 0; qi < QB; qi++) {
+                        for (int qi = 0; qi < NQ; qi++) {
                             const uint64_t vq = (uint32_t)qi < nqg ? vmask : 0ull;
                             uint64_t m;
                             if constexpr (F32) {
@@ -409,95 +634,26 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                 }
                 if (!FILL && hb && ((bitpos & 63) != 0 || subc != 0) && lane == 0) hb[bitpos >> 6] = hitw;
             } else {
-                for (uint32_t t0 = 0; t0 < M; t0 += 64) {
+                for (uint32_t t0 = clo * 64; t0 < mend; t0 += 64) {
                     const uint32_t t = t0 + lane;
-                    const bool valid = t < M;
+                    const bool valid = t < mend;
                     const uint32_t pos = valid ? cur.pos(rl, t) : 0u;
                     // one compare per ballot, validity applied to the scalar
                     // masks; the hit lanes of a fill store under the mask itself
                     const uint64_t vmask = __builtin_amdgcn_ballot_w64(valid);
                     uint32_t pid = 0;
-                    if (FILL) pid = a.ix.ila[valid ? pos : 0u];
-                    double acc[QB];
-    #pragma unroll
-                    for (int qi = 0; qi < QB; qi++) acc[qi] = 0.0;
-                    if constexpr (F32) {
-                        float x[DQ];
-                        if constexpr (DQ % 2 == 0) {
-                            typedef float f2 __attribute__((ext_vector_type(2)));
-                            const f2 *src = reinterpret_cast<const f2 *>(a.aos32 + (uint64_t)pos * DQ);
-    #pragma unroll
-                            for (int l = 0; l < DQ / 2; l++) {
-                                const f2 v = src[l];
-                                x[2 * l] = v.x;
-                                x[2 * l + 1] = v.y;
-                            }
-                        } else {
-    #pragma unroll
-                            for (int l = 0; l < DQ; l++) x[l] = a.soa32[(uint64_t)l * n + pos];
-                        }
-    #pragma unroll
-                        for (int qi = 0; qi < QB; qi++) {
-                            float accf = 0.0f;
-    #pragma unroll
-                            for (int l = 0; l < DQ; l++) {
-                                const float d = x[l] - qregf[qi][l];
-                                accf = __builtin_fmaf(d, d, accf);
-                            }
-                            const uint64_t vq = (uint32_t)qi < nqg ? vmask : 0ull;
-                            uint64_t m = __builtin_amdgcn_ballot_w64(accf <= a.tacc32) & vq;
-                            const uint64_t mb = vq & ~m & ~__builtin_amdgcn_ballot_w64(accf > a.trej32);
-                            if (mb) {
-                                // the band: the exact FP64 chain decides
-                                bool hit = false;
-                                if (__builtin_amdgcn_inverse_ballot_w64(mb)) {
-                                    double e = 0.0;
-    #pragma unroll
-                                    for (int l = 0; l < DQ; l++) {
-                                        const double d = soa[(uint64_t)l * n + pos] - a.queries[(uint64_t)qid[qi] * dim + l];
-                                        e = __builtin_fma(d, d, e);
-                                    }
-                                    hit = e <= T;
-                                }
-                                m |= __builtin_amdgcn_ballot_w64(hit);
-                                my_band += (uint64_t)__popcll(mb);
-                            }
-                            if (FILL && m && __builtin_amdgcn_inverse_ballot_w64(m))
-                                a.out[base[qi] + cnt[qi] + lanes_below(m)] = pid;
-                            cnt[qi] += (uint32_t)__popcll(m);
-                        }
-                        continue;
-                    } else if constexpr (D > 0) {
-                        double x[DQ];
-                        // unconditional (invalid lanes read position 0, masked below)
-                        if constexpr (D <= (int)kAosMaxDim) {
-                            const double *src = a.ix.aos + (uint64_t)pos * DQ;
-    #pragma unroll
-                            for (int l = 0; l < DQ; l++) x[l] = src[l];
-                        } else {
-    #pragma unroll
-                            for (int l = 0; l < DQ; l++) x[l] = soa[(uint64_t)l * n + pos];
-                        }
-    #pragma unroll
-                        for (int qi = 0; qi < QB; qi++) {
-    #pragma unroll
-                            for (int l = 0; l < DQ; l++) {
-                                const double d = x[l] - qreg[qi][l];
-                                acc[qi] = __builtin_fma(d, d, acc[qi]);
-                            }
-                        }
-                    } else {
-                        for (uint32_t l = 0; l < dim; l++) {
-                            const double xl = valid ? soa[(uint64_t)l * n + pos] : 0.0;
-    #pragma unroll
-                            for (int qi = 0; qi < QB; qi++) {
-                                const double d = xl - a.queries[(uint64_t)qid[qi] * dim + l];
-                                acc[qi] = __builtin_fma(d, d, acc[qi]);
-                            }
+                    if (FILL) pid = a.ix.ila[pos];
+                    double acc[NQ] = {};
+                    for (uint32_t l = 0; l < dim; l++) {
+                        const double xl = valid ? soa[(uint64_t)l * n + pos] : 0.0;
+#pragma unroll
+                        for (int qi = 0; qi < NQ; qi++) {
+                            const double d = xl - a.queries[(uint64_t)qid[qi] * dim + l];
+                            acc[qi] = __builtin_fma(d, d, acc[qi]);
                         }
                     }
-    #pragma unroll
-                    for (int qi = 0; qi < QB; qi++) {
+#pragma unroll
+                    for (int qi = 0; qi < NQ; qi++) {
                         const uint64_t m = __builtin_amdgcn_ballot_w64(acc[qi] <= T) & ((uint32_t)qi < nqg ? vmask : 0ull);
                         if (FILL && m && __builtin_amdgcn_inverse_ballot_w64(m))
                             a.out[base[qi] + cnt[qi] + lanes_below(m)] = pid;
@@ -505,24 +661,49 @@ __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3)
                     }
                 }
             }
+            };
+            if (nqg == 1)
+                sweep(std::integral_constant<int, 1>());
+            else if (nqg == 2)
+                sweep(std::integral_constant<int, 2>());
+            else
+                sweep(std::integral_constant<int, QB>());
             if (!FILL && lane < (int)nqg) {
-                uint32_t mine = 0;
+                uint32_t mine = 0, id = 0;
 #pragma unroll
-                for (int qi = 0; qi < QB; qi++)
-                    if (qi == lane) mine = cnt[qi];
-                a.counts[qid[lane]] = mine;
+                for (int qi = 0; qi < QB; qi++) {
+                    mine = qi == lane ? cnt[qi] : mine;
+                    id = qi == lane ? qid[qi] : id;
+                }
+                if (nseg == 1) {
+                    a.counts[id] = mine;
+                } else {
+                    a.seg_counts[(uint64_t)w * QB + lane] = mine;
+                    if (mine) atomicAdd(&a.counts[id], mine);
+                }
             }
-            if (lane == 0) my_evals += (uint64_t)M * nqg;
+            if (lane == 0) my_evals += (uint64_t)(mend - min(mend, clo * 64)) * nqg;
         }
+        if (lane == 0) w = gridDim.x * kQWaves + atomicAdd(reload(args).queue_head, 1u);
+        w = (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
     }
-    if (lane == 0) {
-        if (!FILL && my_evals) atomicAdd(a.evals, (unsigned long long)my_evals);
-        if (!FILL && my_band && a.band) atomicAdd(a.band, (unsigned long long)my_band);
+    if (!FILL) {
+        if (lane == 0) {
+            atomicAdd(&sh_stats[0], (unsigned long long)my_evals);
+            atomicAdd(&sh_stats[1], (unsigned long long)my_band);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const QJoinArgs &a = reload(args);
+            if (sh_stats[0]) atomicAdd(a.evals, sh_stats[0]);
+            if (sh_stats[1] && a.band) atomicAdd(a.band, sh_stats[1]);
+        }
     }
 }
 
 // Pair hash of a request's CSR result: sum of mix64(query << 32 | neighbour)
-// over its rows, G lanes per row; one atomic per wave.
+// over its rows, G lanes per row; one atomic per workgroup (atomics on one
+// address take 12 ns each, one after the other).
 template <int G>
 __global__ __launch_bounds__(256) void k_csr_hash(const uint64_t *__restrict__ off, const uint32_t *__restrict__ nb,
                                                   uint32_t n, unsigned long long *hash) {
@@ -535,7 +716,10 @@ __global__ __launch_bounds__(256) void k_csr_hash(const uint64_t *__restrict__ o
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
-    if ((threadIdx.x & 63) == 0 && h) atomicAdd(hash, (unsigned long long)h);
+    __shared__ uint64_t sh[4];
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = h;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(hash, (unsigned long long)(sh[0] + sh[1] + sh[2] + sh[3]));
 }
 
 // q32 = fl32(fl64(q - centre)) and the largest |q - centre| (as ordered bits).
@@ -601,23 +785,40 @@ hegj_status query_geom(const GridGeom &g, QueryGeom *qg) {
     return HEGJ_OK;
 }
 
-hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const double *queries,
+hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const DevIndex &ix, const double *queries,
                        uint32_t nq, hipStream_t s) {
-    p->nq = nq;
-    p->n_units = 0;
-    p->n_live = 0;
+    *p = QueryPlan{};
     if (nq == 0) return HEGJ_OK;
+    const uint32_t max_seg = std::min(std::max(kSplitItems / nq, 1u), kMaxSegments);
     HIP_TRY(keep.get(&p->keys, nq));
     HIP_TRY(keep.get(&p->ids, nq));
-    HIP_TRY(keep.get(&p->starts, (size_t)nq + 1));
+    HIP_TRY(keep.get(&p->items, (size_t)nq * max_seg));
+    HIP_TRY(keep.get(&p->counts, nq));
+    if (max_seg > 1) HIP_TRY(keep.get(&p->seg_counts, (size_t)nq * max_seg * kUnitQueries));
     Scratch sc;
     uint64_t *keys_alt;
-    uint32_t *ids_alt, *flag, *rank, *d_small;
+    uint32_t *ids_alt, *flag;
     HIP_TRY(sc.get(&keys_alt, nq));
     HIP_TRY(sc.get(&ids_alt, nq));
     HIP_TRY(sc.get(&flag, nq));
+    if (nq <= kSmallPlan) {
+        HIP_TRY(keep.get(&p->items_dev, 1));
+        k_qcell_keys<<<ceil_div(nq, 256), 256, 0, s>>>(queries, nq, qg, keys_alt, ids_alt);
+        HIP_TRY(hipGetLastError());
+        const uint32_t min_seg = std::min(std::max(kSpareItems / nq, 1u), kMaxSegments / 2);
+        k_qsmall_rank<<<ceil_div(nq, 64), 256, 0, s>>>(keys_alt, nq, qg, ix, min_seg, max_seg, p->keys, p->ids,
+                                                       flag, p->counts);
+        HIP_TRY(hipGetLastError());
+        k_qsmall_items<<<1, 1024, 0, s>>>(flag, nq, p->items, p->items_dev);
+        HIP_TRY(hipGetLastError());
+        p->n_items = nq * max_seg;  // at most: the device holds their number
+        return scratch_done(s);
+    }
+    uint32_t *rank, *starts, *d_small;
     HIP_TRY(sc.get(&rank, nq));
+    HIP_TRY(sc.get(&starts, (size_t)nq + 1));
     HIP_TRY(sc.get(&d_small, 2));
+    HIP_TRY(hipMemsetAsync(p->counts, 0, sizeof(uint32_t) * nq, s));
     k_qcell_keys<<<ceil_div(nq, 256), 256, 0, s>>>(queries, nq, qg, p->keys, p->ids);
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(radix_sort_u64(p->keys, p->ids, keys_alt, ids_alt, nq, qg.key_bits, s));
@@ -625,38 +826,31 @@ hegj_status query_plan(QueryPlan *p, Scratch &keep, const QueryGeom &qg, const d
     k_qrun_flags<<<ceil_div(nq, 256), 256, 0, s>>>(p->keys, nq, qg.dead_key, flag, d_small + 1);
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(scan_u32(flag, rank, nq, d_small, s));
-    k_qrun_fill<<<ceil_div(nq, 256), 256, 0, s>>>(flag, rank, nq, p->starts);
+    k_qrun_fill<<<ceil_div(nq, 256), 256, 0, s>>>(flag, rank, nq, starts);
     HIP_TRY(hipGetLastError());
     uint32_t h[2];
     HEGJ_TRY(read_back(h, d_small, s, 2));
     const uint32_t runs = h[0];
-    p->n_live = h[1];
     // starts[runs] = end of the live queries
-    HIP_TRY(hipMemcpyAsync(p->starts + runs, &p->n_live, sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    // split the runs into units of at most kUnitQueries queries
-    p->n_units = 0;
+    HIP_TRY(hipMemcpyAsync(starts + runs, &h[1], sizeof(uint32_t), hipMemcpyHostToDevice, s));
     if (runs > 0) {
-        uint32_t *cnt, *first, *sub_starts, *d_total;
+        uint32_t *cnt, *nseg, *first, *d_total;
         HIP_TRY(sc.get(&cnt, runs));
+        HIP_TRY(sc.get(&nseg, runs));
         HIP_TRY(sc.get(&first, runs));
-        HIP_TRY(sc.get(&sub_starts, (size_t)nq + 1));
         HIP_TRY(sc.get(&d_total, 1));
-        k_sub_counts<<<ceil_div(runs, 256), 256, 0, s>>>(p->starts, runs, cnt);
+        k_item_counts<<<ceil_div(runs, 256), 256, 0, s>>>(starts, runs, p->keys, qg, ix, max_seg, nseg, cnt);
         HIP_TRY(hipGetLastError());
         HEGJ_TRY(scan_u32(cnt, first, runs, d_total, s));
-        k_sub_fill<<<ceil_div(runs, 256), 256, 0, s>>>(p->starts, runs, first, sub_starts);
+        k_item_fill<<<ceil_div(runs, 256), 256, 0, s>>>(starts, runs, nseg, first, p->items);
         HIP_TRY(hipGetLastError());
-        uint32_t units = 0;
-        HEGJ_TRY(read_back(&units, d_total, s));
-        HIP_TRY(hipMemcpyAsync(p->starts, sub_starts, sizeof(uint32_t) * units, hipMemcpyDeviceToDevice, s));
-        HIP_TRY(hipMemcpyAsync(p->starts + units, &p->n_live, sizeof(uint32_t), hipMemcpyHostToDevice, s));
-        p->n_units = units;
+        HEGJ_TRY(read_back(&p->n_items, d_total, s));
     }
-    return scratch_done(s);  // the plan outlives the copies from it
+    return scratch_done(s);
 }
 
 hegj_status query_run(const QJoinArgs &base, bool fill, int device, hipStream_t s) {
-    if (base.n_units == 0) return HEGJ_OK;
+    if (base.n_items == 0) return HEGJ_OK;
     // resident workgroups of the join on this device (thread-safe, once)
     static const uint32_t resident = [device]() {
         hipDeviceProp_t prop;
@@ -668,7 +862,7 @@ hegj_status query_run(const QJoinArgs &base, bool fill, int device, hipStream_t 
         return (uint32_t)std::max(per_cu, 1) * (uint32_t)prop.multiProcessorCount;
     }();
     const uint32_t blocks =
-        std::max<uint32_t>(1, std::min<uint32_t>(resident, ceil_div(base.n_units, kQWaves)));
+        std::max<uint32_t>(1, std::min<uint32_t>(resident, ceil_div(base.n_items, kQWaves)));
     return fill ? launch_qd<true>(base, blocks, s) : launch_qd<false>(base, blocks, s);
 }
 
@@ -696,6 +890,11 @@ hegj_status query_to_f32(const double *q, uint32_t nq, uint32_t dim, const doubl
 }
 
 hegj_status query_offsets(const uint32_t *counts, uint32_t nq, uint64_t *offsets, hipStream_t s) {
+    if (nq <= kSmallScan) {
+        k_qsmall_offsets<<<1, 1024, 0, s>>>(counts, nq, offsets);
+        HIP_TRY(hipGetLastError());
+        return HEGJ_OK;
+    }
     Scratch sc;
     uint64_t *c64;
     HIP_TRY(sc.get(&c64, nq));

@@ -186,16 +186,14 @@ hegj_status hegj_server::run(Request *r, hipStream_t s, Arena &arena, void *ctr_
     hegj_index *lv = levels[r->level];
     Scratch keep;
     double *q;
-    uint32_t *counts;
     uint64_t *offsets;
     HIP_TRY(keep.get(&q, (size_t)nq * dim));
-    HIP_TRY(keep.get(&counts, nq));
     HIP_TRY(keep.get(&offsets, (size_t)nq + 1));
     uint64_t *hitbits;
     HIP_TRY(keep.get(&hitbits, (size_t)nq * kQueryHitWords));
     HIP_TRY(hipMemcpyAsync(q, r->queries.data(), sizeof(double) * nq * dim, hipMemcpyHostToDevice, s));
     QueryPlan plan;
-    HEGJ_TRY(query_plan(&plan, keep, qg, q, nq, s));
+    HEGJ_TRY(query_plan(&plan, keep, qg, index_dev(lv), q, nq, s));
     struct Ctr {
         uint32_t head[2];
         unsigned long long hash, evals, band, rbits;
@@ -218,18 +216,19 @@ hegj_status hegj_server::run(Request *r, hipStream_t s, Arena &arena, void *ctr_
         const double R = std::max(L.radius, rq) * (1.0 + 1e-12);
         f32 = f32_thresholds(sqrt_threshold(r->eps), dim, R, &tacc, &trej);
     }
-    HIP_TRY(hipMemsetAsync(counts, 0, sizeof(uint32_t) * nq, s));
     QJoinArgs a{};
     a.qg = qg;
     a.ix = index_dev(lv);
     a.queries = q;
     a.keys = plan.keys;
     a.ids = plan.ids;
-    a.starts = plan.starts;
-    a.n_units = plan.n_units;
+    a.items = plan.items;
+    a.n_items = plan.n_items;
+    a.items_dev = plan.items_dev;
+    a.seg_counts = plan.seg_counts;
     a.queue_head = &ctr->head[0];
     a.thresh = sqrt_threshold(r->eps);
-    a.counts = counts;
+    a.counts = plan.counts;
     a.hash = &ctr->hash;
     a.evals = &ctr->evals;
     a.band = &ctr->band;
@@ -243,7 +242,7 @@ hegj_status hegj_server::run(Request *r, hipStream_t s, Arena &arena, void *ctr_
         a.trej32 = trej;
     }
     HEGJ_TRY(query_run(a, false, device, s));
-    HEGJ_TRY(query_offsets(counts, nq, offsets, s));
+    HEGJ_TRY(query_offsets(plan.counts, nq, offsets, s));
     uint64_t total = 0;
     HEGJ_TRY(read_back(&total, offsets + nq, s));
     r->t_counted = Clock::now();
