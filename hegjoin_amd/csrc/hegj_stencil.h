@@ -59,14 +59,20 @@ __device__ __forceinline__ bool cell_box(const GridGeom &g, const DevIndex &ix, 
     return ok;
 }
 
-// Rows of the box `b` into rl; returns the number of candidates, *nslots the
-// number of rows kept.  tb.gap holds the gaps of nq queries (written and
+// A lane's rows (l, l + 64, ..): the row's cells [ca, re), none where the row
+// is empty or left out, and the dim-0 window [lo, hi].
+constexpr int kLaneRows = (kMaxRows + 63) / 64;
+struct LaneRows {
+    uint32_t ca[kLaneRows], re[kLaneRows], lo[kLaneRows], hi[kLaneRows];
+};
+
+// The rows of the box `b`.  tb.gap holds the gaps of nq queries (written and
 // ordered by the caller); a cell is kept when the sum of its squared gaps is
 // at most thr for one of them (nq = 0 with thr = +inf: every cell).  c0: the
 // dim-0 coordinate, signed (a query's cell may lie one outside the grid).
-template <int QB, typename L>
-__device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevIndex &ix, L &rl,
-                                                 StencilTabs<QB> &tb, const CellBox &b, int64_t c0, uint32_t nq, float thr, uint32_t *nslots) {
+template <int QB>
+__device__ __forceinline__ void stencil_probe(const GridGeom &g, const DevIndex &ix, StencilTabs<QB> &tb,
+                                              const CellBox &b, int64_t c0, uint32_t nq, float thr, LaneRows &w) {
     const uint32_t lane = threadIdx.x & 63, k = g.k;
     // tables: lanes 0..8 take part a (dims 1, 2), lanes 16..42 part b (dims 3..5)
     const bool isb = lane >= 16;
@@ -113,8 +119,8 @@ __device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevInd
     }
     wave_lds_sync();
     const uint32_t nrows = pow3(k - 1);
-    constexpr int R = (kMaxRows + 63) / 64;
-    uint32_t wlo[R], whi[R], slot[R];
+    constexpr int R = kLaneRows;
+    uint32_t slot[R];
     uint64_t rkey[R];
     bool want[R];
 #pragma unroll
@@ -134,13 +140,11 @@ __device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevInd
         if (!(mleft <= thr) && c0 > l) l = c0;
         if (!(mright <= thr) && c0 < h) h = c0;
         want[i] = want[i] && mmid <= thr && l <= h;
-        wlo[i] = (uint32_t)l;
-        whi[i] = (uint32_t)h;
+        w.lo[i] = (uint32_t)l;
+        w.hi[i] = (uint32_t)h;
         slot[i] = hash_slot(rkey[i]) & ix.hmask;
     }
     // hash probes: first slots together, collisions one by one
-    uint32_t ca[R], re[R];
-    uint32_t longest = 0;
     {
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
         const u32x4 *const tab = reinterpret_cast<const u32x4 *>(ix.hrows);
@@ -159,18 +163,28 @@ __device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevInd
                 e[i] = tab[slot[i]];
                 hit = e[i].x == k0 && e[i].y == k1;
             }
-            want[i] = want[i] && hit;
-            ca[i] = want[i] ? e[i].z : 0u;
-            re[i] = want[i] ? e[i].w : 0u;
-            longest = max(longest, re[i] - ca[i]);
+            w.ca[i] = want[i] && hit ? e[i].z : 0u;
+            w.re[i] = want[i] && hit ? e[i].w : 0u;
         }
+    }
+}
+
+// Candidate positions [pstart, pstart + plen) of a lane's rows.
+__device__ __forceinline__ void stencil_ranges(const DevIndex &ix, const LaneRows &w, uint32_t (&pstart)[kLaneRows],
+                                               uint32_t (&plen)[kLaneRows]) {
+    constexpr int R = kLaneRows;
+    uint32_t ca[R], longest = 0;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        ca[i] = w.ca[i];
+        longest = max(longest, w.re[i] - ca[i]);
     }
     // first cell at or after the window's start, all rows in step, by the
     // cells' dim-0 coordinates (ascending within a row)
     const uint32_t *const x0 = ix.cell_xyz;
     uint32_t end[R];
 #pragma unroll
-    for (int i = 0; i < R; i++) end[i] = re[i];
+    for (int i = 0; i < R; i++) end[i] = w.re[i];
     while (__builtin_amdgcn_ballot_w64(longest > 3)) {
         uint32_t v[R];
 #pragma unroll
@@ -180,7 +194,7 @@ __device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevInd
         for (int i = 0; i < R; i++) {
             if (end[i] > ca[i]) {
                 const uint32_t mid = (ca[i] + end[i]) >> 1;
-                if (v[i] < wlo[i])
+                if (v[i] < w.lo[i])
                     ca[i] = mid + 1;
                 else
                     end[i] = mid;
@@ -190,19 +204,19 @@ __device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevInd
     }
     // at most 3 cells are left before the lower bound and 3 from it on are in
     // the window: six coordinates decide both ends
-    uint32_t pstart[R], plen[R], ck[R][6], cb[R];
+    uint32_t ck[R][6], cb[R];
 #pragma unroll
     for (int i = 0; i < R; i++)
 #pragma unroll
-        for (int j = 0; j < 6; j++) ck[i][j] = ca[i] + j < re[i] ? x0[ca[i] + j] : ~0u;
+        for (int j = 0; j < 6; j++) ck[i][j] = ca[i] + j < w.re[i] ? x0[ca[i] + j] : ~0u;
 #pragma unroll
     for (int i = 0; i < R; i++) {
         uint32_t na = 0, nb = 0;
 #pragma unroll
         for (int j = 0; j < 6; j++) {
-            const bool in_row = ca[i] + j < re[i];
-            na += in_row && ck[i][j] < wlo[i] ? 1u : 0u;
-            nb += in_row && ck[i][j] <= whi[i] ? 1u : 0u;
+            const bool in_row = ca[i] + j < w.re[i];
+            na += in_row && ck[i][j] < w.lo[i] ? 1u : 0u;
+            nb += in_row && ck[i][j] <= w.hi[i] ? 1u : 0u;
         }
         cb[i] = ca[i] + nb;
         ca[i] += na;
@@ -213,10 +227,23 @@ __device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevInd
         pstart[i] = any ? ix.cell_start[ca[i]] : 0u;
         plen[i] = any ? ix.cell_start[cb[i]] - pstart[i] : 0u;
     }
+}
+
+// Rows of the box `b` into rl; returns the number of candidates, *nslots the
+// number of rows kept.  The other arguments as for stencil_probe.
+template <int QB, typename L>
+__device__ __forceinline__ uint32_t stencil_rows(const GridGeom &g, const DevIndex &ix, L &rl,
+                                                 StencilTabs<QB> &tb, const CellBox &b, int64_t c0, uint32_t nq,
+                                                 float thr, uint32_t *nslots) {
+    LaneRows w;
+    stencil_probe<QB>(g, ix, tb, b, c0, nq, thr, w);
+    uint32_t pstart[kLaneRows], plen[kLaneRows];
+    stencil_ranges(ix, w, pstart, plen);
     // compact the non-empty rows, in row order, into the LDS list
+    const uint32_t lane = threadIdx.x & 63, nrows = pow3(g.k - 1);
     uint32_t slots = 0, total = 0;
 #pragma unroll
-    for (int i = 0; i < R; i++) {
+    for (int i = 0; i < kLaneRows; i++) {
         if (64u * i >= nrows) break;
         const uint64_t nz = __ballot(plen[i] > 0);
         uint32_t x = plen[i];
