@@ -132,8 +132,11 @@ def rooflines(n, dim, cells, pairs, evals, kernel_ms, refine):
       FP64 flops  = 3 D per distance evaluation E the kernel performs
                     (subtract + fma per dim; E is the reference's candidate
                     count less the candidates cell-box pruning leaves out)
-      MFMA flops  = 2 D per candidate pair, against the bf16 peak divided by
-                    the 3 products of a split-BF16 dot (hi.hi + hi.lo + lo.hi)
+      MFMA flops  = 2 D per candidate pair evaluated (the FP16 tiles evaluate
+                    an unordered pair once), against the bf16 peak divided by
+                    the 3 products of a split-BF16 dot (hi.hi + hi.lo + lo.hi);
+                    the FP16 tiles spend one product per dimension, so their
+                    own roof is three times as high
     Returns (binding, other): the binding roof is the one whose roof time is
     longer (the roof the kernel would hit first)."""
     t = kernel_ms * 1e-3
@@ -145,8 +148,9 @@ def rooflines(n, dim, cells, pairs, evals, kernel_ms, refine):
     if refine == "mfma":
         flops = 2.0 * dim * evals
         peak = PEAK_BF16_TFLOPS / 3.0
-        note = ("2 D flops per candidate pair; peak = bf16 dense MFMA / 3 (split-BF16 "
-                "hi.hi + hi.lo + lo.hi); kernel k_gb_join")
+        note = ("2 D flops per candidate pair evaluated; peak = bf16 dense MFMA / 3 (split-BF16 "
+                "hi.hi + hi.lo + lo.hi); kernel k_g16_join spends one fp16 product per dimension, "
+                "its own roof is 3 times this peak")
         bound = "mfma"
     elif refine == "f32":
         flops = 3.0 * dim * evals
@@ -381,7 +385,7 @@ def main():
         "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": ms_step,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": {"mfma": "bf16 hi/lo (f32 acc) + f64 band recheck",
+        "dtype": {"mfma": "f16 (f32 acc) + f64 band recheck",
                   "f32": "f32 filter + f64 band recheck"}.get(refine_used, "f64"), "data": "synthetic (reference exponential generator, seed 0)",
         "config": {"workload": cfg["name"], "n": n, "dim": dim, "indexed_dims": k,
                    "eps": eps, "pairs": pairs, "total_candidates": total_cand,

@@ -418,7 +418,7 @@ class GridIndex:
         dimensionality (tuning.tsv, written by hegjoin_amd.autotune).
         unit_order: "morton", "spatial" (linear cell id) or "workload"
         (descending candidates, the reference's order); refine: "auto",
-        "fp64" or "mfma" (split-BF16 MFMA + guard band + FP64 band
+        "fp64" or "mfma" (MFMA Gram tiles + guard band + FP64 band
         recheck) or "f32" (FP32 distance filter + exact FP64 recheck of its
         band); xcd_parts: unit ranges, one per XCD (0 = auto);
         use_graph: keep the FP64 plan in the index and replay a captured

@@ -7,7 +7,7 @@ For one workload (the reference's exponential generator, seed 0) it sweeps
 the runtime choices of the join -- queries per work unit (the points that
 share one streamed candidate tile), unit order, per-XCD unit ranges, units
 per queue grab, and at 16 dimensions and above the refine (FP64 chain or the
-split-BF16 MFMA guard band) -- times each configuration, and checks that all
+MFMA guard band) -- times each configuration, and checks that all
 of them produce the same pair count and pair hash.  A configuration whose
 result differs is an error, not a candidate.  A second stage sweeps, around
 the first stage's best grid-join configuration, the workgroup size (1, 2 or

@@ -199,12 +199,15 @@ typedef enum {
     HEGJ_REFINE_AUTO = 0,     /* MFMA guard band when dim >= 16, FP32 filter where it is
                                  built (dim 2 and 6) and its band is narrow, else FP64 */
     HEGJ_REFINE_FP64 = 1,     /* exact FP64 chain for every candidate */
-    HEGJ_REFINE_MFMA = 2,     /* split-BF16 MFMA tiles + guard band + FP64 band recheck */
+    HEGJ_REFINE_MFMA = 2,     /* MFMA Gram tiles (FP16, or split BF16 where the
+                                 data's spread is too large) + guard band + FP64
+                                 band recheck */
     HEGJ_REFINE_F32 = 3       /* FP32 distance filter + exact FP64 recheck of its band */
 } hegj_refine;
 
 typedef struct {
-    uint64_t result_capacity; /* pairs per device result batch; 0 = estimate.  MFMA
+    uint64_t result_capacity; /* pairs per device result batch; 0 = estimate, or
+                                 all candidates where they fit (2^27).  MFMA
                                  refine: the size of its first pair list (the join's
                                  pairs are held in one list, 8 bytes each; a list
                                  that overflows is rebuilt once at 1.25x the count) */
@@ -212,7 +215,8 @@ typedef struct {
     uint32_t queries_per_unit;/* FP64 kernel: 4, 8 or 16; 0 = tuned default */
     uint32_t refine;          /* hegj_refine */
     uint32_t xcd_parts;       /* unit ranges, one per XCD: 0 = auto (8), 1 = one queue */
-    uint32_t units_per_grab;  /* units a wave takes per queue atomic; 0 = auto */
+    uint32_t units_per_grab;  /* units a wave takes at a time; 0 = runs of units of
+                                 equal estimated work */
     uint32_t part_by_block;   /* 0: range by hardware XCD id, 1: by workgroup index */
     uint32_t use_graph;       /* FP64 refine: keep the plan in the index and run the
                                  batch as a replay of a captured hipGraph */
@@ -249,7 +253,7 @@ hegj_status hegj_selfjoin(hegj_index *idx, const hegj_join_opts *opts, hegj_resu
  * epsilon^2.  (No reference counterpart; exposed for callers and tests.) */
 hegj_status hegj_f32_thresholds(double epsilon, uint32_t dim, double radius, float *tacc,
                                 float *trej);
-/* The operands of the MFMA refine (no reference counterpart; for callers and
+/* The split-BF16 operands of the MFMA refine (no reference counterpart; for callers and
  * the band's tests): for n points (row-major n x dim) centred at centre[dim],
  * the split-BF16 rows A'[n * kp] and B'[n * kp] (BF16 bit patterns) and the
  * guard w[n], by the same code the device runs.  coef_scale multiplies the
