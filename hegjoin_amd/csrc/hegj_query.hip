@@ -389,9 +389,9 @@ __device__ __forceinline__ const QJoinArgs &reload(QArgsPtr p) {
 // F32: candidates from the level's centred FP32 copy, queries from the
 // request's (centred the same way); acc32 <= tacc32 accepts, acc32 > trej32
 // rejects, the band between is decided by the exact FP64 chain.
-// Held to 3 waves per SIMD (168 registers, a few spilled): at 2 waves the
-// candidate loads of too few waves are in flight (6-D, 10M points, 93k
-// queries: 290 -> 270 ms per request).
+// Held to 3 waves per SIMD (130 registers): at 2 waves the candidate loads of
+// too few waves are in flight (6-D, 10M points, 93k queries: 290 -> 270 ms per
+// request); 4 waves measured the same.
 template <int D, bool FILL, bool F32 = false, int QB = kQB>
 __global__ __launch_bounds__(64 * kQWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_qjoin(QJoinArgs) {
     static_assert(!F32 || D > 0, "FP32 filter needs a fixed dimensionality");
