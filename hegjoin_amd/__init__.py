@@ -144,6 +144,8 @@ _lib.hegj_dataset_free.argtypes = [_vp]
 _lib.hegj_stream_copy_bandwidth.argtypes = [C.c_uint64, C.c_int, C.POINTER(C.c_double)]
 _lib.hegj_release_cached_memory.argtypes = [C.c_int]
 _lib.hegj_release_cached_memory.restype = None
+_lib.hegj_fail_device_allocations.argtypes = [C.c_uint32, C.c_uint32]
+_lib.hegj_fail_device_allocations.restype = None
 _lib.hegj_index_opts_default.argtypes = [C.POINTER(_IndexOpts), C.c_uint32]
 _lib.hegj_index_build.argtypes = [_vp, C.c_uint32, C.c_double, C.POINTER(_IndexOpts), C.POINTER(_vp)]
 _lib.hegj_index_build_device.argtypes = _lib.hegj_index_build.argtypes

@@ -79,7 +79,7 @@ hipError_t Scratch::alloc(void **p, size_t bytes) {
         }
         return e;
     }
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = driver_malloc(p, bytes);
     if (e == hipSuccess) ptrs.push_back(*p);
     return e;
 }
@@ -164,6 +164,22 @@ void cache_release(int dev) {
 
 void cache_release_device(int dev) { cache_release(dev); }
 
+namespace {
+thread_local uint32_t g_fail_skip = 0, g_fail_count = 0;
+}
+hipError_t driver_malloc(void **p, size_t bytes) {
+    if (g_fail_count) {
+        if (g_fail_skip == 0) {
+            g_fail_count--;
+            return hipErrorOutOfMemory;
+        }
+        g_fail_skip--;
+    }
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 hipError_t dev_malloc(void **p, size_t bytes) {
     if (g_arena) return arena_alloc(p, bytes);
     int dev = 0;
@@ -182,11 +198,10 @@ hipError_t dev_malloc(void **p, size_t bytes) {
             return hipSuccess;
         }
     }
-    e = hipMalloc(p, rs);
+    e = driver_malloc(p, rs);
     if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
         cache_release(dev);
-        e = hipMalloc(p, rs);
+        e = driver_malloc(p, rs);
     }
     if (e == hipSuccess) {
         std::lock_guard<std::mutex> lk(g_cache_mu);
@@ -525,12 +540,19 @@ hegj_status new_index(const hegj_index_opts *o, hegj_index **out, F fill) {
 hegj_status ensure_workload(hegj_index *h) {
     if (h->have_workload) return HEGJ_OK;
     const uint32_t C = h->ix.C;
-    HIP_TRY(dev_malloc_n(&h->d_work, (size_t)C + 1));
-    HIP_TRY(dev_malloc_n(&h->d_order, (size_t)C + 1));
+    DevHold hold(h->stream);
+    uint32_t *work, *order;
+    uint64_t candidates = 0;
+    HIP_TRY(hold.get(&work, (size_t)C + 1));
+    HIP_TRY(hold.get(&order, (size_t)C + 1));
     EventTimer t(h->stream);
-    HEGJ_TRY(launch_workload(h->g, h->ix, h->d_work, h->stream));
-    HEGJ_TRY(workload_order(h->ix, h->d_work, h->d_order, &h->total_candidates, h->stream));
+    HEGJ_TRY(launch_workload(h->g, h->ix, work, h->stream));
+    HEGJ_TRY(workload_order(h->ix, work, order, &candidates, h->stream));
     h->workload_ms = t.stop();
+    hold.keep();
+    h->d_work = work;
+    h->d_order = order;
+    h->total_candidates = candidates;
     h->have_workload = true;
     return HEGJ_OK;
 }
@@ -557,8 +579,15 @@ struct Counters {
 
 hegj_status ensure_morton(hegj_index *h) {
     if (h->d_morton) return HEGJ_OK;
-    HIP_TRY(dev_malloc_n(&h->d_morton, (size_t)h->ix.C + 1));
-    return morton_order(h->g, h->ix, h->d_morton, &h->morton_ok, h->stream);
+    DevHold hold(h->stream);
+    uint32_t *order;
+    bool ok = false;
+    HIP_TRY(hold.get(&order, (size_t)h->ix.C + 1));
+    HEGJ_TRY(morton_order(h->g, h->ix, order, &ok, h->stream));
+    hold.keep();
+    h->morton_ok = ok;
+    h->d_morton = order;
+    return HEGJ_OK;
 }
 
 // Bound on |acc32 - acc| for a pair whose exact squared distance is S: acc32
@@ -1310,7 +1339,7 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
         G->grab = opts.units_per_grab ? opts.units_per_grab : grab_for(G->P, G->P.U);
         JoinArgs q{};
         G->blocks = set_queue(q, G->P, G->grab);
-        HIP_TRY(hipMalloc(&G->d_args, sizeof(JoinArgs)));
+        HIP_TRY(driver_malloc(reinterpret_cast<void **>(&G->d_args), sizeof(JoinArgs)));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&G->h_args), sizeof(JoinArgs), hipHostMallocDefault));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&G->h_ctr), sizeof(Counters), hipHostMallocDefault));
         std::memset(G->h_args, 0, sizeof(JoinArgs));
@@ -1478,6 +1507,11 @@ int hegj_device_count(void) {
     int c = 0;
     if (hipGetDeviceCount(&c) != hipSuccess) return 0;
     return c;
+}
+
+void hegj_fail_device_allocations(uint32_t skip, uint32_t count) {
+    hegj::g_fail_skip = skip;
+    hegj::g_fail_count = count;
 }
 
 void hegj_release_cached_memory(int device) {

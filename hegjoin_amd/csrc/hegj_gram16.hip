@@ -584,18 +584,10 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     const size_t rows = (size_t)n + 1;
     uint16_t *A = nullptr, *B = nullptr;
     float *w = nullptr;
-    struct Guard {
-        uint16_t *&A, *&B;
-        float *&w;
-        ~Guard() {
-            if (A || B || w) (void)hipStreamSynchronize(s);  // a failed launch's stream
-            for (void *p : {(void *)A, (void *)B, (void *)w}) dev_free(p);
-        }
-        hipStream_t s;
-    } guard{A, B, w, s};
-    HIP_TRY(dev_malloc_n(&A, rows * kb * 32));
-    HIP_TRY(dev_malloc_n(&B, rows * kb * 32));
-    HIP_TRY(dev_malloc_n(&w, rows));
+    DevHold hold(s);
+    HIP_TRY(hold.get(&A, rows * kb * 32));
+    HIP_TRY(hold.get(&B, rows * kb * 32));
+    HIP_TRY(hold.get(&w, rows));
     const uint32_t blocks = ceil_div(rows, 256);
     const double gamma = g16_gamma(kb);
     switch (kb) {
@@ -611,8 +603,7 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     ops->A = A;
     ops->B = B;
     ops->w = w;
-    A = B = nullptr;
-    w = nullptr;
+    hold.keep();
     ops->kp = kb * 32;
     ops->f16 = true;
     const double rej = tau * tau * (1.0 + 4.0 * u64);

@@ -143,6 +143,31 @@ hipError_t dev_malloc_n(T **p, size_t count) {
 }
 void dev_free(void *p);
 void cache_release_device(int dev);  // hipFree the cached buffers of one device
+// hipMalloc, with the failures that hegj_fail_device_allocations asks for; an
+// error is returned, never left behind as the runtime's last one (the next
+// launch check would report it).
+hipError_t driver_malloc(void **p, size_t bytes);
+
+// Device arrays that outlive the function that makes them, once all of its
+// steps have succeeded: until keep() they are given back when it is left.
+struct DevHold {
+    hipStream_t stream;  // may still be working on them then
+    std::vector<void *> ptrs;
+    explicit DevHold(hipStream_t s) : stream(s) {}
+    DevHold(const DevHold &) = delete;
+    DevHold &operator=(const DevHold &) = delete;
+    template <typename T>
+    hipError_t get(T **p, size_t count) {
+        hipError_t e = dev_malloc_n(p, count);
+        if (e == hipSuccess) ptrs.push_back(*p);
+        return e;
+    }
+    void keep() { ptrs.clear(); }
+    ~DevHold() {
+        if (!ptrs.empty()) (void)hipStreamSynchronize(stream);
+        for (void *p : ptrs) dev_free(p);
+    }
+};
 
 // Device -> host.  read_back: small structures through pinned memory; the
 // stream is synchronised.  copy_to_host: results into the caller's pageable

@@ -553,14 +553,22 @@ hegj_status gb_prepare(const GridGeom &g, const DevIndex &ix, GbOperands *ops, h
     if (ops->A) return HEGJ_OK;
     const uint32_t kb = gb_kblocks(dim), kp = kb * 32;
     if (kb == 0) return fail(HEGJ_ERR_UNSUPPORTED, "no MFMA refine for this dimensionality");
-    HIP_TRY(dev_malloc_n(&ops->A, (size_t)n * kp));
-    HIP_TRY(dev_malloc_n(&ops->B, (size_t)n * kp));
-    HIP_TRY(dev_malloc_n(&ops->w, n));
-    ops->kp = kp;
+    // the caller takes a non-null A for all of them: handed out together
+    DevHold hold(s);
+    uint16_t *A, *B;
+    float *w;
+    HIP_TRY(hold.get(&A, (size_t)n * kp));
+    HIP_TRY(hold.get(&B, (size_t)n * kp));
+    HIP_TRY(hold.get(&w, n));
     k_gb_prepare<<<ceil_div(n, 256), 256, 0, s>>>(ix.soa, n, dim, kp, mean, gb_coefficient(dim, kp),
-                                                 ops->A, ops->B, ops->w);
+                                                 A, B, w);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
+    hold.keep();
+    ops->A = A;
+    ops->B = B;
+    ops->w = w;
+    ops->kp = kp;
     return HEGJ_OK;
 }
 

@@ -525,7 +525,6 @@ hegj_status morton_order(const GridGeom &g, const DevIndex &ix, uint32_t *order,
         *ok = false;
         return HEGJ_OK;
     }
-    *ok = true;
     Scratch sc;
     uint64_t *keys, *keys_alt;
     uint32_t *vals_alt;
@@ -535,6 +534,7 @@ hegj_status morton_order(const GridGeom &g, const DevIndex &ix, uint32_t *order,
     k_morton_keys<<<ceil_div(ix.C, 256), 256, 0, s>>>(g, ix, bits, keys, order);
     HIP_TRY(hipGetLastError());
     HEGJ_TRY(radix_sort_u64(keys, order, keys_alt, vals_alt, ix.C, (int)(bits * g.k), s));
+    *ok = true;
     return HEGJ_OK;
 }
 
@@ -664,8 +664,10 @@ hegj_status make_soa32(const GridGeom &g, const DevIndex &ix, float **soa32, flo
     Scratch sc;
     double *part, *centre;
     HIP_TRY(sc.get(&part, (size_t)blocks * dim * 2));
-    HIP_TRY(dev_malloc_n(centre_dev, dim));
-    centre = *centre_dev;
+    // the caller takes a non-null soa32 for all of them: handed out together
+    DevHold hold(s);
+    float *soa = nullptr, *aos = nullptr;
+    HIP_TRY(hold.get(&centre, dim));
     k_dim_minmax<<<blocks, 256, 0, s>>>(ix.soa, n, dim, part);
     HIP_TRY(hipGetLastError());
     std::vector<double> hp((size_t)blocks * dim * 2), c(dim);
@@ -682,18 +684,22 @@ hegj_status make_soa32(const GridGeom &g, const DevIndex &ix, float **soa32, flo
         c[l] = g.f32dt ? 0.0 : lo + (hi - lo) * 0.5;
         R = std::max(R, std::max(hi - c[l], c[l] - lo));
     }
-    *radius = R * (1.0 + 1e-12);
     HIP_TRY(hipMemcpyAsync(centre, c.data(), sizeof(double) * dim, hipMemcpyHostToDevice, s));
-    HIP_TRY(dev_malloc_n(soa32, (size_t)n * dim));
+    HIP_TRY(hold.get(&soa, (size_t)n * dim));
     const uint64_t total = (uint64_t)n * dim;
-    k_soa32<<<ceil_div(total, 256), 256, 0, s>>>(ix.soa, total, n, centre, *soa32);
+    k_soa32<<<ceil_div(total, 256), 256, 0, s>>>(ix.soa, total, n, centre, soa);
     HIP_TRY(hipGetLastError());
     if (aos32 && dim <= kAosMaxDim) {
-        HIP_TRY(dev_malloc_n(aos32, ((size_t)n + kAos32Pad) * dim));
-        k_aos32<<<ceil_div((uint64_t)n + kAos32Pad, 256), 256, 0, s>>>(*soa32, n, dim, *aos32);
+        HIP_TRY(hold.get(&aos, ((size_t)n + kAos32Pad) * dim));
+        k_aos32<<<ceil_div((uint64_t)n + kAos32Pad, 256), 256, 0, s>>>(soa, n, dim, aos);
         HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipStreamSynchronize(s));
+    hold.keep();
+    *radius = R * (1.0 + 1e-12);
+    *centre_dev = centre;
+    *soa32 = soa;
+    if (aos32) *aos32 = aos;
     return HEGJ_OK;
 }
 

@@ -88,6 +88,11 @@ hegj_status hegj_stream_copy_bandwidth(uint64_t bytes, int device, double *gbps)
  * the unused buffers on `device` (-1: every device, and the pinned memory).
  * No reference counterpart. */
 void hegj_release_cached_memory(int device);
+/* For tests of what a call leaves behind when memory runs out: of the calling
+ * thread's next device allocations that no kept buffer serves, `skip` succeed
+ * and the `count` after them fail as if the device were full (0, 0: none).  No
+ * reference counterpart. */
+void hegj_fail_device_allocations(uint32_t skip, uint32_t count);
 
 /* ------------------------------------------------------------------------ */
 /* Datasets.                                                                */

@@ -1,0 +1,61 @@
+"""What is left behind when device memory runs out: a call that fails with
+"out of memory" leaves its index usable, wherever in the call it failed, and
+the same call afterwards gives the whole result.  No reference counterpart."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+OUT_OF_MEMORY = 4  # HEGJ_ERR_OUT_OF_MEMORY
+
+
+@pytest.fixture(scope="module")
+def H():
+    import hegjoin_amd as H
+    if H.device_count() == 0:
+        pytest.fail("no HIP device visible for a GPU test")
+    yield H
+    H.library().hegj_fail_device_allocations(0, 0)
+
+
+def data(oracle, kind):
+    """Points, eps, options: each lazily built part of an index."""
+    rng = np.random.default_rng(11)
+    if kind == "f32 copy, Morton order":
+        return oracle.generate_expo(4000, 6, seed=31), 0.03, dict(refine="f32", unit_order="morton")
+    if kind == "FP16 operands":
+        return oracle.generate_expo(1500, 18, seed=32), 0.12, dict(refine="mfma", unit_order="morton")
+    pts = rng.random((900, 24)) * 0.1
+    pts[7, 20:] = 1e7  # one point too far for FP16: split-BF16 operands
+    return pts, 0.15, dict(refine="mfma", unit_order="workload")
+
+
+@pytest.mark.parametrize("kind", ["f32 copy, Morton order", "FP16 operands", "BF16 operands"])
+def test_a_failed_first_join_can_be_repeated(H, oracle, kind):
+    """Every allocation of the first join on an index fails once, each on an
+    index of its own (no kept buffers, so each request reaches the driver)."""
+    pts, eps, kw = data(oracle, kind)
+    eoff, enb = oracle.join(pts, 6, eps)
+    lib = H.library()
+    failures = 0
+    for skip in range(200):
+        with H.GridIndex(pts, eps, indexed_dims=6) as ix:
+            H.release_cached_memory()
+            print("case", kind, "allocation", skip, flush=True)
+            lib.hegj_fail_device_allocations(skip, 1 << 30)
+            try:
+                ix.selfjoin(**kw).close()
+                done = True
+            except H.HegjError as e:
+                assert e.status == OUT_OF_MEMORY, str(e)
+                done = False
+            finally:
+                lib.hegj_fail_device_allocations(0, 0)
+            t = ix.selfjoin(**kw)
+            off, nb = t.csr(sort_rows=True)
+            t.close()
+            assert np.array_equal(off, eoff) and np.array_equal(nb, enb)
+        if done:
+            break
+        failures += 1
+    assert done and failures >= 8
