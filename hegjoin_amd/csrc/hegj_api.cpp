@@ -79,7 +79,7 @@ hipError_t Scratch::alloc(void **p, size_t bytes) {
         }
         return e;
     }
-    hipError_t e = driver_malloc(p, bytes);
+    hipError_t e = driver_malloc_or_release(p, bytes);
     if (e == hipSuccess) ptrs.push_back(*p);
     return e;
 }
@@ -180,6 +180,16 @@ hipError_t driver_malloc(void **p, size_t bytes) {
     return e;
 }
 
+hipError_t driver_malloc_or_release(void **p, size_t bytes) {
+    hipError_t e = driver_malloc(p, bytes);
+    int dev = 0;
+    if (e == hipErrorOutOfMemory && hipGetDevice(&dev) == hipSuccess) {
+        cache_release(dev);
+        e = driver_malloc(p, bytes);
+    }
+    return e;
+}
+
 hipError_t dev_malloc(void **p, size_t bytes) {
     if (g_arena) return arena_alloc(p, bytes);
     int dev = 0;
@@ -198,11 +208,7 @@ hipError_t dev_malloc(void **p, size_t bytes) {
             return hipSuccess;
         }
     }
-    e = driver_malloc(p, rs);
-    if (e == hipErrorOutOfMemory) {
-        cache_release(dev);
-        e = driver_malloc(p, rs);
-    }
+    e = driver_malloc_or_release(p, rs);
     if (e == hipSuccess) {
         std::lock_guard<std::mutex> lk(g_cache_mu);
         g_cache_live[*p] = {dev, rs};
@@ -1339,7 +1345,7 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
         G->grab = opts.units_per_grab ? opts.units_per_grab : grab_for(G->P, G->P.U);
         JoinArgs q{};
         G->blocks = set_queue(q, G->P, G->grab);
-        HIP_TRY(driver_malloc(reinterpret_cast<void **>(&G->d_args), sizeof(JoinArgs)));
+        HIP_TRY(driver_malloc_or_release(reinterpret_cast<void **>(&G->d_args), sizeof(JoinArgs)));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&G->h_args), sizeof(JoinArgs), hipHostMallocDefault));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&G->h_ctr), sizeof(Counters), hipHostMallocDefault));
         std::memset(G->h_args, 0, sizeof(JoinArgs));

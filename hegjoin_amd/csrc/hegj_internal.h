@@ -147,6 +147,9 @@ void cache_release_device(int dev);  // hipFree the cached buffers of one device
 // error is returned, never left behind as the runtime's last one (the next
 // launch check would report it).
 hipError_t driver_malloc(void **p, size_t bytes);
+// For what goes back with hipFree: where the device is full, the cache's free
+// buffers go back to it first.
+hipError_t driver_malloc_or_release(void **p, size_t bytes);
 
 // Device arrays that outlive the function that makes them, once all of its
 // steps have succeeded: until keep() they are given back when it is left.

@@ -277,9 +277,9 @@ void hegj_server::worker(uint32_t slot) {
         init_err = "slot: cannot create a stream";
     // one request at a time: its queries and every temporary of the pipeline
     arena.cap = (size_t)opts.max_queries * (opts.dim * 8 + 128 + kQueryHitWords * 8) + (32u << 20);
-    if (init_err.empty() && hipMalloc(reinterpret_cast<void **>(&arena.base), arena.cap) != hipSuccess)
+    if (init_err.empty() && driver_malloc_or_release(reinterpret_cast<void **>(&arena.base), arena.cap) != hipSuccess)
         init_err = "slot: cannot allocate its device arena";
-    if (init_err.empty() && hipMalloc(&ctr, 256) != hipSuccess) init_err = "slot: cannot allocate counters";
+    if (init_err.empty() && driver_malloc_or_release(&ctr, 256) != hipSuccess) init_err = "slot: cannot allocate counters";
     set_thread_arena(init_err.empty() ? &arena : nullptr);
     while (true) {
         Request *r = nullptr;
@@ -377,7 +377,8 @@ hegj_status hegj_serve_open(const double *database, uint32_t n, const hegj_serve
     };
     double *dev = nullptr;
     const size_t bytes = sizeof(double) * (size_t)n * o->dim;
-    if (hipMalloc(&dev, bytes) != hipSuccess) return fail(HEGJ_ERR_OUT_OF_MEMORY, "database upload");
+    if (driver_malloc_or_release(reinterpret_cast<void **>(&dev), bytes) != hipSuccess)
+        return fail(HEGJ_ERR_OUT_OF_MEMORY, "database upload");
     if (hipMemcpy(dev, database, bytes, hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipFree(dev);
         return fail(HEGJ_ERR_HIP, "database upload");
@@ -413,7 +414,7 @@ hegj_status hegj_serve_open(const double *database, uint32_t n, const hegj_serve
         S->qgeo.push_back(qg);
     }
     (void)hipFree(dev);
-    if (hipMalloc(reinterpret_cast<void **>(&S->pool_base), o->result_bytes) != hipSuccess)
+    if (driver_malloc_or_release(reinterpret_cast<void **>(&S->pool_base), o->result_bytes) != hipSuccess)
         return bail(fail(HEGJ_ERR_OUT_OF_MEMORY, "result-buffer pool"));
     S->pool.init(o->result_bytes);
     if (hipStreamCreateWithFlags(&S->copy_stream, hipStreamNonBlocking) != hipSuccess)

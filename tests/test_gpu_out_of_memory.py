@@ -59,3 +59,25 @@ def test_a_failed_first_join_can_be_repeated(H, oracle, kind):
             break
         failures += 1
     assert done and failures >= 8
+
+
+def test_kept_buffers_make_room(H, oracle):
+    """A device full with the library's own kept buffers: every allocation of
+    a server that opens, and of an index, is served after they went back."""
+    base = oracle.generate_expo(5000, 6, seed=33)
+    q = oracle.generate_expo(50, 6, seed=34)
+    eoff, enb = oracle.range_join(base, q, 0.05)
+    lib = H.library()
+    for skip in range(30):
+        with H.GridIndex(base, 0.03) as ix:
+            ix.selfjoin().close()
+        print("case allocation", skip, flush=True)
+        lib.hegj_fail_device_allocations(skip, 1)
+        try:
+            S = H.Server(base, [0.051], slots=1, result_bytes=1 << 20, max_queries=64)
+        finally:
+            lib.hegj_fail_device_allocations(0, 0)
+        with S:
+            off, nb = S.result(S.submit(q, 0.05))
+        rows = np.concatenate([np.sort(nb[off[i]:off[i + 1]]) for i in range(50)])
+        assert np.array_equal(off, eoff) and np.array_equal(rows, enb)
