@@ -195,7 +195,7 @@ hipError_t dev_malloc(void **p, size_t bytes) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    const size_t rs = cache_round(bytes);
+    size_t rs = cache_round(bytes);
     {
         // the smallest cached buffer that holds it, if not over a quarter larger
         std::lock_guard<std::mutex> lk(g_cache_mu);
@@ -209,6 +209,10 @@ hipError_t dev_malloc(void **p, size_t bytes) {
         }
     }
     e = driver_malloc_or_release(p, rs);
+    if (e == hipErrorOutOfMemory && rs > bytes) {  // the rounding may be what does not fit
+        rs = bytes;
+        e = driver_malloc(p, rs);
+    }
     if (e == hipSuccess) {
         std::lock_guard<std::mutex> lk(g_cache_mu);
         g_cache_live[*p] = {dev, rs};

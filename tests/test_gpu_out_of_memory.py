@@ -81,3 +81,18 @@ def test_kept_buffers_make_room(H, oracle):
             off, nb = S.result(S.submit(q, 0.05))
         rows = np.concatenate([np.sort(nb[off[i]:off[i + 1]]) for i in range(50)])
         assert np.array_equal(off, eoff) and np.array_equal(rows, enb)
+
+
+def test_the_rounding_of_kept_sizes_is_no_reason_to_fail(H, oracle):
+    """Sizes are rounded up so that later calls find each other's buffers.
+    Where the rounded size does not fit the device, the exact one is taken:
+    100003 points of 6 coordinates are 4800144 bytes, rounded up to 5242880."""
+    pts = oracle.generate_expo(100003, 6, seed=35)
+    H.release_cached_memory()
+    H.library().hegj_fail_device_allocations(0, 2)  # the rounded size, before and after giving buffers back
+    try:
+        ix = H.GridIndex(pts, 0.01)
+    finally:
+        H.library().hegj_fail_device_allocations(0, 0)
+    assert ix.info["n"] == len(pts)
+    ix.close()
