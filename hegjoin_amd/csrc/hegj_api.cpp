@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "hegj_internal.h"
+#include "hegj_threads.h"
 
 namespace hegj {
 
@@ -349,15 +350,16 @@ hegj_status copy_to_host(void *dst, const void *src, size_t bytes, int device, h
     chunk = std::max<size_t>((size_t)1 << 20, std::min(chunk, kPinnedChunk));
     const size_t n = (bytes + chunk - 1) / chunk;
     std::atomic<int> bad{0};
-    // Thread t moves chunks t, t + threads, ..: while it copies one out, the
-    // other threads' transfers keep the link busy.
+    std::atomic<size_t> next{0};
+    // Each thread takes the next chunk: while it copies one out, the other
+    // threads' transfers keep the link busy.
     auto work = [&](size_t t) {
         Pinned pin(true);
         hipEvent_t ev = nullptr;
         hipError_t e = t ? hipSetDevice(device) : hipSuccess;
         if (e == hipSuccess) e = pin.get();
         if (e == hipSuccess && !(ev = event_get(device))) e = hipErrorUnknown;
-        for (size_t c = t; e == hipSuccess && c < n; c += threads) {
+        for (size_t c; e == hipSuccess && (c = next++) < n;) {
             const size_t at = c * chunk, len = std::min(chunk, bytes - at);
             e = hipMemcpyAsync(pin.p, static_cast<const char *>(src) + at, len, hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipEventRecord(ev, s);
@@ -371,10 +373,7 @@ hegj_status copy_to_host(void *dst, const void *src, size_t bytes, int device, h
         }
         event_put(device, ev);
     };
-    std::vector<std::thread> pool;
-    for (size_t t = 1; t < std::min(threads, n); t++) pool.emplace_back(work, t);
-    work(0);
-    for (auto &t : pool) t.join();
+    run_on_threads(std::min(threads, n) - 1, work);
     if (bad.load()) {  // no pinned memory or a failed transfer: the plain way
         HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
