@@ -173,9 +173,10 @@ struct DevHold {
 };
 
 // Device -> host.  read_back: small structures through pinned memory; the
-// stream is synchronised.  copy_to_host: results into the caller's pageable
-// memory, in chunks through pinned buffers with several threads copying out
-// (a plain hipMemcpy to pageable memory ran at 18 GB/s, the link does 57).
+// stream is synchronised.  copy_to_host: results into the caller's memory; if
+// that is pageable, in chunks through pinned buffers with several threads
+// copying out (a plain hipMemcpy to pageable memory ran at 18 GB/s, the link
+// does 57), else straight into it.
 hegj_status read_back_bytes(void *dst, const void *src, size_t bytes, hipStream_t s);
 template <typename T>
 hegj_status read_back(T *dst, const T *src, hipStream_t s, size_t count = 1) {
