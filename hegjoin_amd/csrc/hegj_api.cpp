@@ -64,6 +64,8 @@ CallScope::~CallScope() {
 
 bool scratch_outlives() { return g_scope != nullptr || g_arena != nullptr; }
 
+void free_with_call(void *p) { g_scope->ptrs.push_back(p); }
+
 hegj_status scratch_done(hipStream_t s) {
     if (!scratch_outlives()) HIP_TRY(hipStreamSynchronize(s));
     return HEGJ_OK;
@@ -791,6 +793,23 @@ void set_chunk(JoinPlan &P, double est) {
 }
 constexpr uint64_t kBoundCandidates = 1ull << 27;
 
+// A result keeps its batch until it is freed, so one sized by the candidates
+// (60k 6-D points at 64 neighbours: half a GiB for 16 MB of rows) is changed for
+// one of the size that its rows took, where that saves 16 MiB and half of it:
+// a copy of the rows at the device's copy rate (16 MB: 8 us).  The old one
+// is given back when the call ends; without memory for the copy it stays.
+hegj_status fit_batch(hegj_result *r, uint64_t capacity, uint64_t used, hipStream_t s) {
+    used = std::min(used, capacity);  // (the last chunk reserved may reach past the end)
+    if (capacity < 2 * used + (4u << 20)) return HEGJ_OK;
+    uint32_t *fit = nullptr;
+    const uint64_t n16 = (used + 3) / 4;
+    if (dev_malloc_n(&fit, std::max<uint64_t>(n16 * 4, 4)) != hipSuccess) return HEGJ_OK;
+    free_with_call(r->batches[0]);
+    const uint32_t *const rows = r->batches[0];
+    r->batches[0] = fit;
+    return copy_16(fit, rows, n16, s);
+}
+
 // At most 60% of the free device memory for one batch.
 hegj_status cap_to_free(uint64_t *capacity) {
     size_t free_b = 0, total_b = 0;
@@ -1066,6 +1085,7 @@ struct BatchRunner {
         r->info.band_rechecks = c.sum(kStatBand);
         r->info.refine_used = P.f32 ? HEGJ_REFINE_F32 : HEGJ_REFINE_FP64;
         if (P.bounded) r->info.estimated_pairs = r->info.total_neighbors;
+        if (P.bounded && r->batches.size() == 1) HEGJ_TRY(fit_batch(r, capacity, used, s));
         r->info.n_batches = (uint32_t)r->batches.size();
         r->info.join_ms = join_ms;
         r->info.join_launches = launches;
@@ -1417,7 +1437,10 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
     r->info.evals_executed = c.sum(kStatEvals);
     r->info.band_rechecks = c.sum(kStatBand);
     r->info.refine_used = G.P.f32 ? HEGJ_REFINE_F32 : HEGJ_REFINE_FP64;
-    if (G.P.bounded) r->info.estimated_pairs = r->info.total_neighbors;
+    if (G.P.bounded) {
+        r->info.estimated_pairs = r->info.total_neighbors;
+        HEGJ_TRY(fit_batch(r, G.P.capacity, c.cursor, s));
+    }
     r->info.n_batches = 1;
     r->info.join_launches = 1;
     r->info.join_kernel_avg_ms = r->info.join_ms;

@@ -112,6 +112,8 @@ struct CallScope {
 // Whether a Scratch's memory outlives the function that owns it (an open call
 // scope or an installed arena).
 bool scratch_outlives();
+// Gives a dev_malloc buffer back at the end of the open call, which there must be.
+void free_with_call(void *p);
 // Before a Scratch goes out of scope with kernels still using it.
 hegj_status scratch_done(hipStream_t s);
 
@@ -430,6 +432,8 @@ hegj_status gather_rows(const std::vector<uint32_t *> &batches, const std::vecto
                         uint32_t n, uint32_t *out, bool sorted, hipStream_t s);
 
 hegj_status stream_copy(uint64_t bytes, int reps, double *ms_per_copy);
+// n16 pieces of 16 bytes, on one device (a kernel: less host time than hipMemcpyAsync).
+hegj_status copy_16(void *dst, const void *src, uint64_t n16, hipStream_t s);
 // row_off[qid[i]] = base + off[i], row_cnt[qid[i]] = cnt[i] (rows answered
 // on the host, added to a device result).
 hegj_status scatter_rows(const uint32_t *qid, const uint64_t *off, const uint32_t *cnt, uint32_t m,

@@ -433,6 +433,14 @@ __global__ __launch_bounds__(256) void k_stream_copy(const uint4 *__restrict__ s
 }
 }  // namespace
 
+hegj_status copy_16(void *dst, const void *src, uint64_t n16, hipStream_t s) {
+    if (n16 == 0) return HEGJ_OK;
+    k_stream_copy<<<std::min<uint32_t>(ceil_div(n16, 256), 8192), 256, 0, s>>>(static_cast<const uint4 *>(src),
+                                                                             static_cast<uint4 *>(dst), n16);
+    HIP_TRY(hipGetLastError());
+    return HEGJ_OK;
+}
+
 hegj_status stream_copy(uint64_t bytes, int reps, double *ms_per_copy) {
     uint64_t n16 = bytes / 16;
     Scratch sc;
