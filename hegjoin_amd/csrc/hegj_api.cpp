@@ -1409,7 +1409,12 @@ hegj_status selfjoin_graph(hegj_index *h, const hegj_join_opts &opts, uint32_t q
     r->info.estimated_pairs = G.P.estimated_pairs;
     HEGJ_TRY(alloc_rows(r, n, s));
     uint32_t *buf = nullptr;
-    HIP_TRY(dev_malloc_n(&buf, G.P.capacity));
+    const hipError_t e = dev_malloc_n(&buf, G.P.capacity);
+    if (e == hipErrorOutOfMemory && !opts.result_capacity) {
+        *fits = false;  // the eager join cuts its batches to the free memory
+        return HEGJ_OK;
+    }
+    HIP_TRY(e);
     r->batches.push_back(buf);
     r->bases.push_back(0);
     JoinArgs a = base_args(h, opts, G.P);
@@ -1855,7 +1860,7 @@ hegj_status hegj_selfjoin(hegj_index *h, const hegj_join_opts *opts_in, hegj_res
     if (opts.use_graph && !h->g.f32dt) {
         bool fits = false;
         HEGJ_TRY(selfjoin_graph(h, opts, qb, order, r.get(), &fits));
-        if (!fits) {  // the cached capacity was too small: this call runs eagerly
+        if (!fits) {  // the cached capacity was too small, or too large for the device now: this call runs eagerly
             r.reset(new hegj_result());
             r->idx = h;
             r->info.total_candidates = h->total_candidates;

@@ -96,3 +96,23 @@ def test_the_rounding_of_kept_sizes_is_no_reason_to_fail(H, oracle):
         H.library().hegj_fail_device_allocations(0, 0)
     assert ix.info["n"] == len(pts)
     ix.close()
+
+
+def test_graph_without_room_for_its_batch(H, oracle):
+    """A replay whose output batch does not fit the device runs eagerly, with
+    batches cut to the free memory, and the next one replays again."""
+    pts = oracle.generate_expo(20000, 6, seed=36)
+    eoff, enb = oracle.join(pts, 6, 0.02)
+    with H.GridIndex(pts, 0.02, indexed_dims=6) as ix:
+        for fail in (0, 3, 0):  # of a batch: the rounded size twice, the exact one
+            if fail:
+                H.release_cached_memory()
+                H.library().hegj_fail_device_allocations(1, fail)  # after the row table
+            try:
+                t = ix.selfjoin(use_graph=True)
+            finally:
+                H.library().hegj_fail_device_allocations(0, 0)
+            assert t.info["graph_replay"] == (0 if fail else 1)
+            off, nb = t.csr(sort_rows=True)
+            t.close()
+            assert np.array_equal(off, eoff) and np.array_equal(nb, enb)
