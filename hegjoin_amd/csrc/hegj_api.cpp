@@ -819,6 +819,26 @@ hegj_status cap_to_free(uint64_t *capacity) {
     return HEGJ_OK;
 }
 
+// The queue of the plan's units: ranges per XCD, split by estimated work, of
+// single units or, without units_per_grab, of runs.  (The hybrid modes, whose
+// list covers all cells, launch pieces of it: grabs, sized for each.)
+// hegj_selfjoin_noalloc, kernel: 2-D 1M points at 300 neighbours 3.11 ms with a
+// unit per grab, 1.98 with the best fixed number (8), 1.95 with runs; 6-D
+// 60k 0.95 (best 1 unit), 0.78; 6-D 1.5M 16.6, 14.1 (2), 11.6.
+hegj_status make_queue(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, JoinPlan &P, bool all_cells = false) {
+    hipStream_t s = h->stream;
+    const uint32_t U = P.U;
+    P.parts = opts.xcd_parts ? std::min<uint32_t>(opts.xcd_parts, kMaxParts) : kMaxParts;
+    if (U < P.parts * 256) P.parts = 1;
+    if (opts.units_per_grab || all_cells || U == 0)
+        return split_units(h->ix, P.units, U, qb, h->d_work, P.parts, P.part_end, s);
+    P.n_runs = (uint32_t)std::min<uint64_t>(U, (uint64_t)P.max_blocks * P.waves * kRunsPerWave);
+    HIP_TRY(dev_malloc_n(&P.runs, (size_t)P.n_runs + 1));
+    HEGJ_TRY(unit_runs(h->ix, P.units, U, qb, h->g.dim, h->d_work, P.n_runs, P.runs, s));
+    for (uint32_t p = 0; p < P.parts; p++) P.part_end[p] = (uint32_t)((uint64_t)P.n_runs * (p + 1) / P.parts);
+    return HEGJ_OK;
+}
+
 // all_cells: units also for the cells the cell-0 wrap silences (the hybrid
 // queue covers every query).
 hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, const uint32_t *order,
@@ -851,17 +871,7 @@ hegj_status make_plan(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, co
     // per-wave hit-mask scratch for units whose masks exceed LDS
     set_waves(P, opts);
     HIP_TRY(dev_malloc_n(&P.gmask, (size_t)P.max_blocks * P.waves * P.gmask_slots));
-    // unit ranges per XCD, split by estimated work
-    P.parts = opts.xcd_parts ? std::min<uint32_t>(opts.xcd_parts, kMaxParts) : kMaxParts;
-    if (U < P.parts * 256) P.parts = 1;
-    if (opts.units_per_grab || all_cells || U == 0) {
-        HEGJ_TRY(split_units(h->ix, P.units, U, qb, h->d_work, P.parts, P.part_end, s));
-    } else {
-        P.n_runs = (uint32_t)std::min<uint64_t>(U, (uint64_t)P.max_blocks * P.waves * kRunsPerWave);
-        HIP_TRY(dev_malloc_n(&P.runs, (size_t)P.n_runs + 1));
-        HEGJ_TRY(unit_runs(h->ix, P.units, U, qb, h->g.dim, h->d_work, P.n_runs, P.runs, s));
-        for (uint32_t p = 0; p < P.parts; p++) P.part_end[p] = (uint32_t)((uint64_t)P.n_runs * (p + 1) / P.parts);
-    }
+    HEGJ_TRY(make_queue(h, opts, qb, P, all_cells));
     // batch estimate: count-only pass over a strided sample of ~8192 units
     // (a few per cent of the join's work at most)
     P.capacity = opts.result_capacity;
@@ -1981,16 +1991,13 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
                             P.f32 ? JoinKind::f32 : h->g.f32dt ? JoinKind::flt : JoinKind::fp64));
     set_waves(P, opts);
     P.gmask_slots = 0;  // units whose masks exceed LDS re-evaluate in the write pass
-    P.parts = opts.xcd_parts ? std::min<uint32_t>(opts.xcd_parts, kMaxParts) : kMaxParts;
-    if (U < P.parts * 256) P.parts = 1;
-    HEGJ_TRY(too_small(split_units(h->ix, P.units, U, qb, h->d_work, P.parts, P.part_end, s)));
+    HEGJ_TRY(too_small(make_queue(h, opts, qb, P)));
     JoinArgs a = base_args(h, opts, P);
     a.row_off = row_off;
     a.row_cnt = row_cnt;
     a.units = P.units;
     a.n_units = U;
-    a.units_per_grab = opts.units_per_grab ? opts.units_per_grab : grab_for(P, U);
-    set_parts(a, P.parts, P.part_end);
+    const uint32_t blocks = set_queue(a, P, opts.units_per_grab ? opts.units_per_grab : 1u);
     a.out = neighbors;
     a.out_base = 0;
     a.capacity = capacity;
@@ -2000,7 +2007,7 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
     if (U > 0) {
         HIP_TRY(hipStreamSynchronize(s));
         const auto tj = std::chrono::steady_clock::now();
-        HEGJ_TRY(launch_join(a, qb, blocks_for(P, U, a.units_per_grab), s));
+        HEGJ_TRY(launch_join(a, qb, blocks, s));
         HIP_TRY(hipStreamSynchronize(s));
         join_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - tj).count();
         HEGJ_TRY(launch_pair_hash(a, capacity, s));
@@ -2028,7 +2035,7 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
         e.cursor = &P.d_ctr2->cursor;
         e.stats = P.d_ctr2->stats[0];
         HEGJ_TRY(zero_words(P.d_ctr2, sizeof(Counters), s));
-        HEGJ_TRY(launch_join(e, qb, blocks_for(P, U, e.units_per_grab), s));
+        HEGJ_TRY(launch_join(e, qb, blocks, s));
         Counters c2;
         HIP_TRY(hipMemcpyAsync(&c2, P.d_ctr2, sizeof(c2), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
