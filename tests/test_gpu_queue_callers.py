@@ -1,0 +1,47 @@
+"""The unit queues of the entry points beside hegj_selfjoin, at the sizes where
+they change: runs of units in hegj_selfjoin_noalloc (fewer units than waves,
+one run each, and more), one or two units per grab in the hybrid pieces."""
+import numpy as np
+import pytest
+
+from hiprt import Buf, runtime
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def H():
+    import hegjoin_amd as H
+    if H.device_count() == 0:
+        pytest.fail("no HIP device visible for a GPU test")
+    return H
+
+
+@pytest.mark.parametrize("n, dim, eps", [(1, 2, 0.01), (9, 6, 0.05), (30000, 2, 0.0002), (400000, 2, 0.00005)])
+def test_noalloc_runs(H, oracle, n, dim, eps):
+    rt = runtime()
+    pts = oracle.generate_expo(n, dim, seed=51)
+    total, want = oracle.join_stats(pts, dim, eps)
+    print("case noalloc", n, dim, total, flush=True)
+    nb, off, cnt = bufs = [Buf(rt, t, m) for m, t in ((total + 1, np.uint32), (n, np.uint64), (n, np.uint32))]
+    with H.GridIndex(pts, eps) as ix:
+        ix.selfjoin().close()  # its lazily built arrays are inputs
+        for _ in range(2):
+            info = ix.selfjoin_noalloc(nb.p, total + 1, off.p, cnt.p)
+            assert (info["total_neighbors"], info["pair_hash"]) == (total, want)
+            assert int(cnt.get().sum()) == total
+    for b in bufs:
+        b.free()
+
+
+@pytest.mark.parametrize("piece", [100, 8191, 8192, 16383, 16384, 60000])
+def test_hybrid_pieces(H, oracle, piece):
+    pts = oracle.generate_expo(50000, 6, seed=52)
+    total, want = oracle.join_stats(pts, 6, 0.012)
+    with H.GridIndex(pts, 0.012) as ix:
+        print("case piece", piece, flush=True)
+        t = ix.selfjoin_hybrid("static", gpu_fraction=0.99, gpu_chunk=piece, cpu_threads=2)
+        info = t.info
+        t.close()
+    assert info["n_units"] > 16384
+    assert (info["total_neighbors"], info["pair_hash"]) == (total, want)
