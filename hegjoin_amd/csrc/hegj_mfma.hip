@@ -623,16 +623,27 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
     Ctr c{};
     for (int attempt = 0; attempt < 4; attempt++) {
         uint64_t *pairs = nullptr, *band = nullptr;
-        Scratch it;
-        HIP_TRY(it.get(&pairs, pair_cap));
+        Scratch it, first;  // first: what only the join and its decisions need
         uint64_t *raw = nullptr;
         float *raw_s = nullptr;
-        if (ops.f16) {
+        while (true) {
             raw_cap = std::min<uint64_t>((raw_cap + kGbBlk - 1) / kGbBlk, 0xFFFFFFu) * kGbBlk;
-            HIP_TRY(it.get(&raw, raw_cap));
-            HIP_TRY(it.get(&raw_s, raw_cap));
-        } else {
-            HIP_TRY(it.get(&band, band_cap));
+            hipError_t e = it.get(&pairs, pair_cap);
+            if (ops.f16) {
+                if (e == hipSuccess) e = first.get(&raw, raw_cap);
+                if (e == hipSuccess) e = first.get(&raw_s, raw_cap);
+            } else {
+                if (e == hipSuccess) e = first.get(&band, band_cap);
+            }
+            if (e == hipSuccess) break;
+            // the first sizes are a guess: smaller lists, which count what they
+            // could not hold, where the device has no room for them
+            if (e != hipErrorOutOfMemory || attempt || pair_cap_first || pair_cap <= (1u << 20)) HIP_TRY(e);
+            HEGJ_TRY(it.drop(s));
+            HEGJ_TRY(first.drop(s));
+            pair_cap /= 2;
+            raw_cap /= 2;
+            band_cap /= 2;
         }
         HIP_TRY(hipMemsetAsync(d, 0, sizeof(Ctr), s));
         GbArgs a{};
@@ -686,12 +697,14 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
             raw_cap = need;
             pair_cap = std::max(pair_cap, need * (mirror ? 2 : 1));
             HEGJ_TRY(it.drop(s));
+            HEGJ_TRY(first.drop(s));
             continue;
         }
         if (c.overflow) {
             pair_cap = std::max(pair_cap * 2, (uint64_t)((c.n_accept + (ops.f16 ? 0 : c.n_band)) * 1.25) + (1u << 22));
             band_cap = std::max(band_cap * 2, (uint64_t)(c.n_band * 1.25) + (1u << 22));
             HEGJ_TRY(it.drop(s));
+            HEGJ_TRY(first.drop(s));
             continue;
         }
         // exact FP64 recheck of the band
@@ -705,6 +718,7 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
             if (c.overflow) {
                 pair_cap = std::max(pair_cap * 2, (uint64_t)(c.n_accept * 1.25) + (1u << 22));
                 HEGJ_TRY(it.drop(s));
+                HEGJ_TRY(first.drop(s));
                 continue;
             }
         }
@@ -714,6 +728,7 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
         if (ntot > 0xFFFFFFFFull) return fail(HEGJ_ERR_UNSUPPORTED, "more than 2^32 pair slots");
         int qbits = 0;
         while (qbits < 32 && ((uint64_t)n >> qbits) != 0) qbits++;
+        HEGJ_TRY(first.drop(s));
         uint64_t *keys_alt;
         HIP_TRY(it.get(&keys_alt, ntot + 1));
         HEGJ_TRY(radix_sort_pairs(pairs, keys_alt, (uint32_t)ntot, qbits, s));

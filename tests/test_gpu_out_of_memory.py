@@ -116,3 +116,35 @@ def test_graph_without_room_for_its_batch(H, oracle):
             off, nb = t.csr(sort_rows=True)
             t.close()
             assert np.array_equal(off, eoff) and np.array_equal(nb, enb)
+
+
+@pytest.mark.parametrize("kind", ["FP16 operands", "BF16 operands"])
+def test_mfma_lists_shrink_to_the_memory(H, oracle, kind):
+    """The first size of the pair and survivor lists is a guess: where one of
+    them does not fit the device, the join runs with smaller ones."""
+    pts, eps, kw = data(oracle, kind)
+    eoff, enb = oracle.join(pts, 6, eps)
+    lib = H.library()
+    with H.GridIndex(pts, eps, indexed_dims=6) as ix:
+        ix.selfjoin(**kw).close()  # everything lazily built
+
+        def attempt(skip, count):
+            H.release_cached_memory()
+            print("case", kind, "allocation", skip, count, flush=True)
+            lib.hegj_fail_device_allocations(skip, count)
+            try:
+                t = ix.selfjoin(**kw)
+            except H.HegjError as e:
+                assert e.status == OUT_OF_MEMORY
+                return False
+            finally:
+                lib.hegj_fail_device_allocations(0, 0)
+            off, nb = t.csr(sort_rows=True)
+            t.close()
+            assert np.array_equal(off, eoff) and np.array_equal(nb, enb)
+            return True
+
+        total = next(k for k in range(200) if attempt(k, 1 << 30))
+        # one request in vain: at its rounded size, again, and at the exact one
+        served = sum(attempt(k, 3) for k in range(total))
+        assert served >= (3 if kind == "FP16 operands" else 2)
