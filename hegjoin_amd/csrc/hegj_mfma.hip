@@ -611,6 +611,8 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
     uint64_t band_cap = std::max<uint64_t>((uint64_t)n * 8, 1u << 22);
     // FP16: one survivor stands for up to two pairs
     uint64_t raw_cap = pair_cap_first ? pair_cap : std::max<uint64_t>((uint64_t)n * 32, 1u << 22);
+    const uint64_t raw_max = 0xFFFFFFull * kGbBlk;  // 32-bit slots
+    auto raw_round = [&](uint64_t v) { return std::min<uint64_t>((v + kGbBlk - 1) / kGbBlk * kGbBlk, raw_max); };
     struct Ctr {
         uint32_t queue_heads[kMaxParts], overflow, pad;
         unsigned long long pair_cursor, band_cursor, n_accept, n_band, evals, raw_cursor, raw_lost;
@@ -627,7 +629,7 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
         uint64_t *raw = nullptr;
         float *raw_s = nullptr;
         while (true) {
-            raw_cap = std::min<uint64_t>((raw_cap + kGbBlk - 1) / kGbBlk, 0xFFFFFFu) * kGbBlk;
+            raw_cap = raw_round(raw_cap);
             hipError_t e = it.get(&pairs, pair_cap);
             if (ops.f16) {
                 if (e == hipSuccess) e = first.get(&raw, raw_cap);
@@ -692,10 +694,10 @@ hegj_status gb_join(const GridGeom &g, const DevIndex &ix, const void *units, ui
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         if (c.raw_lost) {
-            const uint64_t need = (uint64_t)((raw_cap + c.raw_lost) * 1.125) + (1u << 22);
-            if (need > 0xFFFFFF00ull) return fail(HEGJ_ERR_UNSUPPORTED, "more than 2^32 pair slots");
-            raw_cap = need;
-            pair_cap = std::max(pair_cap, need * (mirror ? 2 : 1));
+            const uint64_t need = raw_cap + c.raw_lost;
+            if (need > raw_max || raw_cap == raw_max) return fail(HEGJ_ERR_UNSUPPORTED, "more than 2^32 pair slots");
+            raw_cap = raw_round((uint64_t)(need * 1.125) + (1u << 22));
+            pair_cap = std::max(pair_cap, raw_cap * (mirror ? 2 : 1));
             HEGJ_TRY(it.drop(s));
             HEGJ_TRY(first.drop(s));
             continue;
