@@ -177,6 +177,8 @@ _lib.hegj_superego_rows.argtypes = [_vp, C.c_uint32, C.c_uint32, C.c_double, C.c
                                     C.POINTER(C.c_uint64)]
 _lib.hegj_gb_operands.argtypes = [_vp, C.c_uint32, C.c_uint32, _vp, C.c_double, _vp, _vp, _vp,
                                   C.POINTER(C.c_uint32), C.POINTER(C.c_double)]
+_lib.hegj_g16_operands.argtypes = [_vp, C.c_uint32, C.c_uint32, _vp, C.c_double, C.c_double, _vp, _vp, _vp,
+                                   C.POINTER(C.c_uint32), C.POINTER(C.c_float), C.POINTER(C.c_double)]
 _lib.hegj_free.argtypes = [_vp]
 _lib.hegj_free.restype = None
 _lib.hegj_static_partition_model.argtypes = [C.c_uint32, C.c_uint32, C.c_double]
@@ -308,6 +310,21 @@ def gb_operands(points, centre, coef_scale=1.0):
     _check(_lib.hegj_gb_operands(pts.ctypes.data, n, dim, c.ctypes.data, coef_scale, A.ctypes.data,
                                  B.ctypes.data, w.ctypes.data, C.byref(kp), C.byref(coef)))
     return A, B, w, kp.value, coef.value
+
+
+def g16_operands(points, centre, epsilon, guard_scale=1.0):
+    """The MFMA refine's FP16 operands of `points` centred at `centre`, and its
+    thresholds (hegj_g16_operands): (A, B, w, kp, trej, tacc)."""
+    pts = np.ascontiguousarray(points, np.float64)
+    centre = np.ascontiguousarray(centre, np.float64)
+    n, dim = pts.shape
+    kp, trej, tacc = C.c_uint32(), C.c_float(), C.c_double()
+    _check(_lib.hegj_g16_operands(None, n, dim, None, epsilon, guard_scale, None, None, None, C.byref(kp), None, None))
+    A, B = np.zeros((n, kp.value), np.uint16), np.zeros((n, kp.value), np.uint16)
+    w = np.zeros(n, np.float32)
+    _check(_lib.hegj_g16_operands(pts.ctypes.data, n, dim, centre.ctypes.data, epsilon, guard_scale, A.ctypes.data,
+                                  B.ctypes.data, w.ctypes.data, C.byref(kp), C.byref(trej), C.byref(tacc)))
+    return A, B, w, kp.value, trej.value, tacc.value
 
 
 def static_partition_model(n, dim, epsilon):

@@ -89,20 +89,20 @@ __global__ __launch_bounds__(256) void k_g16_maxnorm(const double *__restrict__ 
     }
 }
 
-__device__ __forceinline__ uint16_t h_bits(_Float16 h) {
+__host__ __device__ __forceinline__ uint16_t h_bits(_Float16 h) {
     uint16_t b;
     __builtin_memcpy(&b, &h, 2);
     return b;
 }
 
 // fp16 of v (FP64), elements below the normal range to zero.
-__device__ __forceinline__ _Float16 to_h16(double v) {
+__host__ __device__ __forceinline__ _Float16 to_h16(double v) {
     const _Float16 h = (_Float16)(float)v;
-    return fabs((double)(float)h) < 6.103515625e-05 ? (_Float16)0.0f : h;
+    return __builtin_fabs((double)(float)h) < 6.103515625e-05 ? (_Float16)0.0f : h;
 }
 
 // fp16 not above v (|v| in the normal range or moved down into it).
-__device__ __forceinline__ _Float16 h16_down(double v) {
+__host__ __device__ __forceinline__ _Float16 h16_down(double v) {
     if (v >= 0.0 && v < 6.103515625e-05) return (_Float16)0.0f;
     if (v < 0.0 && v > -6.103515625e-05) return (_Float16)-6.103515625e-05f;
     _Float16 h = (_Float16)(float)v;
@@ -110,14 +110,85 @@ __device__ __forceinline__ _Float16 h16_down(double v) {
         uint16_t b = h_bits(h);
         b = h > (_Float16)0.0f ? b - 1 : b + 1;  // one step toward -inf
         __builtin_memcpy(&h, &b, 2);
-        if (fabs((double)(float)h) < 6.103515625e-05) h = (_Float16)0.0f;  // stepped out of the normals
+        if (__builtin_fabs((double)(float)h) < 6.103515625e-05) h = (_Float16)0.0f;  // stepped out of the normals
     }
     return h;
 }
 
-// One thread per point (cell order): rows A' and B' and the accept guard w;
-// row n of each is the padding row (an absent query or candidate: s' >=
-// 65504 against anything, above any tau^2).  sum_err += E.
+// One point's rows A' and B' (kp values, a multiple of 32) and its accept
+// guard w, from its coordinates x (stride `stride` between dims); returns its
+// rounding error E.  real = false, or a coordinate that is not finite: the
+// padding row (s' >= 65504 against anything, above any tau^2), E = 0.
+// Built for the host too, where the guards are tested: guard_scale (1 in the
+// join) shrinks them.
+__host__ __device__ __forceinline__ double g16_point(const double *x, uint64_t stride, uint32_t dim, int kp,
+                                                     const double *mean, double sigma, double tau, double gamma,
+                                                     double guard_scale, bool real, uint16_t *A, uint16_t *B,
+                                                     float *w) {
+    const bool point = real;
+    f16x8 az, bz;
+    double N = 0.0, e2 = 0.0, y2 = 0.0, err = 0.0;
+    f16x8 *arow = reinterpret_cast<f16x8 *>(A);
+    f16x8 *brow = reinterpret_cast<f16x8 *>(B);
+    for (int k0 = 0; k0 < kp; k0 += 8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t l = (uint32_t)(k0 + i);
+            _Float16 z = (_Float16)0.0f;
+            if (l < dim && point) {
+                const double xl = x[(uint64_t)l * stride], y = (xl - mean[l]) * sigma;
+                real &= __builtin_isfinite(xl);
+                z = real ? to_h16(y) : (_Float16)0.0f;
+                const double zd = (double)(float)z, e = y - zd;
+                N = __builtin_fma(zd, zd, N);
+                e2 = __builtin_fma(e, e, e2);
+                y2 = __builtin_fma(y, y, y2);
+            }
+            bz[i] = z;
+            az[i] = z * (_Float16)-2.0f;  // exact
+        }
+        if (k0 < kp - 8) {
+            arow[k0 / 8] = az;
+            brow[k0 / 8] = bz;
+        }
+    }
+    // the last group of 8 ends with the norm slots (dim <= kp - 4); a
+    // point with a coordinate that is not finite becomes a padding row
+    _Float16 nhi = (_Float16)kPadNorm, nlo = (_Float16)kPadNorm;
+    if (point && !real) {
+        *w = 0.0f;
+        az = bz = (f16x8)(_Float16)0.0f;
+        for (int j = 0; j < kp / 8 - 1; j++) arow[j] = brow[j] = az;
+    }
+    if (real) {
+        const double u64 = 1.1102230246251565e-16;
+        const double rel = 4.0 * (dim + 4) * u64;
+        // measured error, its own rounding, and that of x - mean
+        err = (__builtin_sqrt(e2) * (1.0 + rel) + 4.0 * u64 * __builtin_sqrt(y2)) * guard_scale;
+        const double s0 = (2.0 * tau * err + 2.0 * err * err) * (1.0 + 1e-12);
+        const double acc = 2.0 * gamma * guard_scale * (2.1 * N + 1.1 * s0);
+        const double v = N * (1.0 - rel) - s0 - acc;
+        nhi = to_h16(v);
+        nlo = h16_down(v - (double)(float)nhi);
+        const double nt = (double)(float)nhi + (double)(float)nlo;
+        const double wd = (N * (1.0 + rel) - nt) + 2.0 * tau * err * (1.0 + 1e-12) + acc;
+        float wf = (float)wd;
+        if ((double)wf < wd) wf = f32_next_up(wf);
+        *w = wf;
+    }
+    az[4] = nhi;
+    az[5] = nlo;
+    az[6] = az[7] = (_Float16)1.0f;
+    bz[4] = bz[5] = (_Float16)1.0f;
+    bz[6] = nhi;
+    bz[7] = nlo;
+    arow[kp / 8 - 1] = az;
+    brow[kp / 8 - 1] = bz;
+    return err;
+}
+
+// One thread per point (cell order); row n of A and B is the padding row.
+// sum_err += E.
 template <int KB>
 __global__ __launch_bounds__(256) void k_g16_prepare(const double *__restrict__ soa, uint32_t n,
                                                      uint32_t dim, const double *__restrict__ mean,
@@ -127,67 +198,9 @@ __global__ __launch_bounds__(256) void k_g16_prepare(const double *__restrict__ 
     constexpr int KP = KB * 32;
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     double err = 0.0;
-    if (p <= n) {
-        bool real = p < n;  // false: the padding row
-        f16x8 az, bz;
-        double N = 0.0, e2 = 0.0, y2 = 0.0;
-        f16x8 *arow = reinterpret_cast<f16x8 *>(A + (uint64_t)p * KP);
-        f16x8 *brow = reinterpret_cast<f16x8 *>(B + (uint64_t)p * KP);
-        for (int k0 = 0; k0 < KP; k0 += 8) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const uint32_t l = (uint32_t)(k0 + i);
-                _Float16 z = (_Float16)0.0f;
-                if (l < dim && p < n) {
-                    const double x = soa[(uint64_t)l * n + p], y = (x - mean[l]) * sigma;
-                    real &= __builtin_isfinite(x);
-                    z = real ? to_h16(y) : (_Float16)0.0f;
-                    const double zd = (double)(float)z, e = y - zd;
-                    N = __builtin_fma(zd, zd, N);
-                    e2 = __builtin_fma(e, e, e2);
-                    y2 = __builtin_fma(y, y, y2);
-                }
-                bz[i] = z;
-                az[i] = z * (_Float16)-2.0f;  // exact
-            }
-            if (k0 < KP - 8) {
-                arow[k0 / 8] = az;
-                brow[k0 / 8] = bz;
-            }
-        }
-        // the last group of 8 ends with the norm slots (dim <= KP - 4); a
-        // point with a coordinate that is not finite becomes a padding row
-        _Float16 nhi = (_Float16)kPadNorm, nlo = (_Float16)kPadNorm;
-        if (p < n && !real) {
-            w[p] = 0.0f;
-            az = bz = (f16x8)(_Float16)0.0f;
-            for (int j = 0; j < KP / 8 - 1; j++) arow[j] = brow[j] = az;
-        }
-        if (real) {
-            const double u64 = 1.1102230246251565e-16;
-            const double rel = 4.0 * (dim + 4) * u64;
-            // measured error, its own rounding, and that of x - mean
-            err = sqrt(e2) * (1.0 + rel) + 4.0 * u64 * sqrt(y2);
-            const double s0 = (2.0 * tau * err + 2.0 * err * err) * (1.0 + 1e-12);
-            const double acc = 2.0 * gamma * (2.1 * N + 1.1 * s0);
-            const double v = N * (1.0 - rel) - s0 - acc;
-            nhi = to_h16(v);
-            nlo = h16_down(v - (double)(float)nhi);
-            const double nt = (double)(float)nhi + (double)(float)nlo;
-            const double wd = (N * (1.0 + rel) - nt) + 2.0 * tau * err * (1.0 + 1e-12) + acc;
-            float wf = (float)wd;
-            if ((double)wf < wd) wf = f32_next_up(wf);
-            w[p] = wf;
-        }
-        az[4] = nhi;
-        az[5] = nlo;
-        az[6] = az[7] = (_Float16)1.0f;
-        bz[4] = bz[5] = (_Float16)1.0f;
-        bz[6] = nhi;
-        bz[7] = nlo;
-        arow[KP / 8 - 1] = az;
-        brow[KP / 8 - 1] = bz;
-    }
+    if (p <= n)
+        err = g16_point(soa + (p < n ? p : 0), n, dim, KP, mean, sigma, tau, gamma, 1.0, p < n,
+                        A + (uint64_t)p * KP, B + (uint64_t)p * KP, w + p);
     for (int o = 32; o > 0; o >>= 1) err += __shfl_xor(err, o, 64);
     __shared__ double sh[4];
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = err;
@@ -551,6 +564,31 @@ static double g16_gamma(uint32_t kb) {
     return nadd * up / (1.0 - nadd * up);
 }
 
+// Scale and thresholds of the operands, from the largest squared norm of the
+// centred points.
+struct G16Scale {
+    double sigma, tau;
+    float trej;
+    double tacc;
+};
+static G16Scale g16_scale(double max2, double thresh, double eps, uint32_t dim) {
+    // sigma: norms and eps below 112, so every s' of a real pair stays far
+    // below the padding's and all norms fit FP16
+    const double top = std::max(std::sqrt(max2) * 1.0001, eps);
+    const int e = std::min(1000, (int)std::floor(std::log2(112.0 / top)));
+    G16Scale r;
+    r.sigma = std::ldexp(1.0, e);
+    const double u64 = std::ldexp(1.0, -53), slop = 4.0 * (dim + 8) * u64;
+    const double tau2 = thresh * r.sigma * r.sigma;
+    r.tau = std::sqrt(tau2) * (1.0 + slop);
+    const double rej = r.tau * r.tau * (1.0 + 4.0 * u64);
+    float rf = (float)rej;
+    if ((double)rf < rej) rf = f32_next_up(rf);
+    r.trej = rf;
+    r.tacc = tau2 * (1.0 - slop);
+    return r;
+}
+
 // Operands for one index and its threshold; ops->A stays null when FP16
 // cannot serve the data (a norm overflows FP64, or the mean rounding
 // error exceeds 1/16 of eps: a far outlier then sets the scale, the band would
@@ -574,13 +612,8 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     double max2;
     std::memcpy(&max2, &bits, sizeof(max2));
     if (!std::isfinite(max2)) return HEGJ_OK;
-    // sigma: norms and eps below 112, so every s' of a real pair stays far
-    // below the padding's and all norms fit FP16
-    const double top = std::max(std::sqrt(max2) * 1.0001, g.eps);
-    const int e = std::min(1000, (int)std::floor(std::log2(112.0 / top)));
-    const double sigma = std::ldexp(1.0, e);
-    const double u64 = std::ldexp(1.0, -53), slop = 4.0 * (dim + 8) * u64;
-    const double tau2 = g.thresh * sigma * sigma, tau = std::sqrt(tau2) * (1.0 + slop);
+    const G16Scale sc16 = g16_scale(max2, g.thresh, g.eps, dim);
+    const double sigma = sc16.sigma, tau = sc16.tau;
     const size_t rows = (size_t)n + 1;
     uint16_t *A = nullptr, *B = nullptr;
     float *w = nullptr;
@@ -606,11 +639,8 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     hold.keep();
     ops->kp = kb * 32;
     ops->f16 = true;
-    const double rej = tau * tau * (1.0 + 4.0 * u64);
-    float rf = (float)rej;
-    if ((double)rf < rej) rf = f32_next_up(rf);
-    ops->trej = rf;
-    ops->tacc = tau2 * (1.0 - slop);
+    ops->trej = sc16.trej;
+    ops->tacc = sc16.tacc;
     return HEGJ_OK;
 }
 
@@ -671,3 +701,37 @@ hegj_status g16_launch(const GbArgs &a, uint32_t blocks, hipStream_t s) {
 }
 
 }  // namespace hegj
+
+extern "C" hegj_status hegj_g16_operands(const double *pts, uint32_t n, uint32_t dim, const double *centre, double epsilon,
+                                         double guard_scale, uint16_t *A, uint16_t *B, float *w, uint32_t *kp,
+                                         float *trej, double *tacc) {
+    using namespace hegj;
+    const uint32_t kb = g16_kblocks(dim);
+    if (dim == 0 || kb == 0) return fail(HEGJ_ERR_UNSUPPORTED, "no FP16 MFMA refine for this dimensionality");
+    if (kp) *kp = kb * 32;
+    if (!A && !B && !w) return HEGJ_OK;
+    if (!pts || !centre || !A || !B || !w || !trej || !tacc || !(epsilon > 0.0))
+        return fail(HEGJ_ERR_INVALID_ARG, "NULL argument or bad epsilon");
+    double max2 = 0.0;
+    for (uint32_t p = 0; p < n; p++) {
+        double s = 0.0;
+        bool fin = true;
+        for (uint32_t l = 0; l < dim; l++) {
+            const double x = pts[(uint64_t)p * dim + l], y = x - centre[l];
+            fin &= std::isfinite(x);
+            s = std::fma(y, y, s);
+        }
+        if (fin) max2 = std::max(max2, s);
+    }
+    const G16Scale r = g16_scale(max2, sqrt_threshold(epsilon), epsilon, dim);
+    std::vector<f16x8> a(kb * 4), b(kb * 4);  // (the caller's rows may not be aligned)
+    for (uint32_t p = 0; p < n; p++) {
+        g16_point(pts + (uint64_t)p * dim, 1, dim, (int)kb * 32, centre, r.sigma, r.tau, g16_gamma(kb), guard_scale, true,
+                  reinterpret_cast<uint16_t *>(a.data()), reinterpret_cast<uint16_t *>(b.data()), w + p);
+        std::memcpy(A + (uint64_t)p * kb * 32, a.data(), kb * 64);
+        std::memcpy(B + (uint64_t)p * kb * 32, b.data(), kb * 64);
+    }
+    *trej = r.trej;
+    *tacc = r.tacc;
+    return HEGJ_OK;
+}

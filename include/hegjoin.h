@@ -259,6 +259,16 @@ hegj_status hegj_selfjoin(hegj_index *idx, const hegj_join_opts *opts, hegj_resu
  * epsilon^2.  (No reference counterpart; exposed for callers and tests.) */
 hegj_status hegj_f32_thresholds(double epsilon, uint32_t dim, double radius, float *tacc,
                                 float *trej);
+/* The FP16 operands of the MFMA refine (no reference counterpart; for callers
+ * and the guards' tests): rows A'[n * kp] and B'[n * kp] (FP16 bit patterns)
+ * and the guards w[n] of n points centred at centre[dim], at one scale, by the
+ * code that the device runs.  With s' = A'_q . B'_c in FP32, s' > *trej rejects
+ * a pair and s' + w_q + w_c <= *tacc accepts it; the others are rechecked in
+ * FP64.  guard_scale multiplies the guards (1 in the join).  kp alone with A, B
+ * and w NULL. */
+hegj_status hegj_g16_operands(const double *points, uint32_t n, uint32_t dim, const double *centre, double epsilon,
+                              double guard_scale, uint16_t *A, uint16_t *B, float *w, uint32_t *kp,
+                              float *trej, double *tacc);
 /* The split-BF16 operands of the MFMA refine (no reference counterpart; for callers and
  * the band's tests): for n points (row-major n x dim) centred at centre[dim],
  * the split-BF16 rows A'[n * kp] and B'[n * kp] (BF16 bit patterns) and the
