@@ -578,7 +578,10 @@ static G16Scale g16_scale(double max2, double thresh, double eps, uint32_t dim) 
     const int e = std::min(1000, (int)std::floor(std::log2(112.0 / top)));
     G16Scale r;
     r.sigma = std::ldexp(1.0, e);
-    const double u64 = std::ldexp(1.0, -53), slop = 4.0 * (dim + 8) * u64;
+    // the FP64 chain against the exact sum, relative to T: its roundings, and
+    // where squares underflow half of the smallest FP64 number for each of them
+    const double u64 = std::ldexp(1.0, -53);
+    const double slop = 4.0 * (dim + 8) * u64 + (dim + 8) * std::ldexp(1.0, -1074) / thresh;
     const double tau2 = thresh * r.sigma * r.sigma;
     r.tau = std::sqrt(tau2) * (1.0 + slop);
     const double rej = r.tau * r.tau * (1.0 + 4.0 * u64);

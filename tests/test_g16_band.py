@@ -102,3 +102,23 @@ def test_decisions_are_sound_at_every_scale(oracle, eps):
     for mode in ("rne", "ru", "rd"):
         reject, accept = decide(H, q, c, eps, 1.0, mode, "seq", None)
         assert not (reject & truth).any() and not (accept & ~truth).any()
+
+
+@pytest.mark.parametrize("eps", [2.0 ** -500, 2.0 ** -515, 2.0 ** -525, 2.0 ** -530, 2.0 ** -534, 2.0 ** -536])
+def test_decisions_where_squares_underflow(oracle, eps):
+    """Thresholds down to a few units of the smallest FP64 number, where the
+    FP64 chain itself rounds by parts of T.  Points that FP16 holds exactly
+    (E = 0), so no other guard hides it."""
+    import hegjoin_amd as H
+    rng = np.random.default_rng(9)
+    dim, m, u = 18, 3000, 2.0 ** -10
+    q = rng.integers(-1000, 1000, (m, dim)) * u
+    d = rng.standard_normal((m, dim))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    c = np.rint((q + d * (1 + rng.uniform(-0.02, 0.02, (m, 1)))) / u) * u
+    q, c = q * eps, c * eps
+    truth = oracle.chain(q, c) <= oracle.threshold(eps)
+    assert truth.any() and (~truth).any()
+    for mode in ("rne", "ru", "rd"):
+        reject, accept = decide(H, q, c, eps, 1.0, mode, "seq", None)
+        assert not (reject & truth).any() and not (accept & ~truth).any()
