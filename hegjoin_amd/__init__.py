@@ -75,7 +75,7 @@ class _ResultInfo(C.Structure):
                 ("estimate_ms", C.c_double), ("join_ms", C.c_double), ("workload_ms", C.c_double),
                 ("total_ms", C.c_double), ("join_kernel_avg_ms", C.c_double),
                 ("join_launches", C.c_uint32), ("refine_used", C.c_uint32),
-                ("graph_replay", C.c_uint32), ("reserved", C.c_uint32),
+                ("graph_replay", C.c_uint32), ("mfma_operands", C.c_uint32),
                 ("estimated_pairs", C.c_uint64)]
 
 
@@ -125,6 +125,8 @@ def _struct_dict(s):
             continue
         if name == "refine_used":
             v = {1: "fp64", 2: "mfma", 3: "f32"}.get(v, "none")
+        if name == "mfma_operands":
+            v = {1: "f16", 2: "bf16"}.get(v, "none")
         if isinstance(v, C.Array):
             v = list(v)
         out[name] = v

@@ -1546,6 +1546,7 @@ hegj_status selfjoin_mfma(hegj_index *h, const uint32_t *order, uint64_t result_
     r->info.join_launches = 1;
     r->info.join_kernel_avg_ms = o.kernel_ms;
     r->info.refine_used = HEGJ_REFINE_MFMA;
+    r->info.mfma_operands = h->gb.f16 ? 1u : 2u;
     return HEGJ_OK;
 }
 

@@ -301,7 +301,7 @@ typedef struct {
     uint32_t join_launches;
     uint32_t refine_used;      /* hegj_refine that ran: FP64 or MFMA */
     uint32_t graph_replay;     /* 1: the join ran as a replay of the captured graph */
-    uint32_t reserved;
+    uint32_t mfma_operands;    /* HEGJ_REFINE_MFMA: 1 = FP16 tiles, 2 = split BF16; else 0 */
     uint64_t estimated_pairs;  /* the batch estimator's pair estimate ("[GPU | RESULT] ~
                                   Total estimated workload", GPU.cu:635); the MFMA
                                   refine and joins of up to 2^27 candidates size
