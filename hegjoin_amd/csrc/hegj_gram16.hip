@@ -116,18 +116,22 @@ __host__ __device__ __forceinline__ _Float16 h16_down(double v) {
 }
 
 // One point's rows A' and B' (kp values, a multiple of 32) and its accept
-// guard w, from its coordinates x (stride `stride` between dims); returns its
-// rounding error E.  real = false, or a coordinate that is not finite: the
-// padding row (s' >= 65504 against anything, above any tau^2), E = 0.
+// guard w, from its coordinates x (stride `stride` between dims); its rounding
+// error E and squared norm N are returned.  real = false, or a coordinate that is not finite: the
+// padding row (s' >= 65504 against anything, above any tau^2), E = N = 0.
 // Built for the host too, where the guards are tested: guard_scale (1 in the
 // join) shrinks them.
-__host__ __device__ __forceinline__ double g16_point(const double *x, uint64_t stride, uint32_t dim, int kp,
+struct G16Point {
+    double err, norm;
+};
+__host__ __device__ __forceinline__ G16Point g16_point(const double *x, uint64_t stride, uint32_t dim, int kp,
                                                      const double *mean, double sigma, double tau, double gamma,
                                                      double guard_scale, bool real, uint16_t *A, uint16_t *B,
                                                      float *w) {
     const bool point = real;
     f16x8 az, bz;
-    double N = 0.0, e2 = 0.0, y2 = 0.0, err = 0.0;
+    double N = 0.0, e2 = 0.0, y2 = 0.0;
+    G16Point r{0.0, 0.0};
     f16x8 *arow = reinterpret_cast<f16x8 *>(A);
     f16x8 *brow = reinterpret_cast<f16x8 *>(B);
     for (int k0 = 0; k0 < kp; k0 += 8) {
@@ -164,7 +168,7 @@ __host__ __device__ __forceinline__ double g16_point(const double *x, uint64_t s
         const double u64 = 1.1102230246251565e-16;
         const double rel = 4.0 * (dim + 4) * u64;
         // measured error, its own rounding, and that of x - mean
-        err = (__builtin_sqrt(e2) * (1.0 + rel) + 4.0 * u64 * __builtin_sqrt(y2)) * guard_scale;
+        const double err = (__builtin_sqrt(e2) * (1.0 + rel) + 4.0 * u64 * __builtin_sqrt(y2)) * guard_scale;
         const double s0 = (2.0 * tau * err + 2.0 * err * err) * (1.0 + 1e-12);
         const double acc = 2.0 * gamma * guard_scale * (2.1 * N + 1.1 * s0);
         const double v = N * (1.0 - rel) - s0 - acc;
@@ -175,6 +179,7 @@ __host__ __device__ __forceinline__ double g16_point(const double *x, uint64_t s
         float wf = (float)wd;
         if ((double)wf < wd) wf = f32_next_up(wf);
         *w = wf;
+        r = G16Point{err, N};
     }
     az[4] = nhi;
     az[5] = nlo;
@@ -184,28 +189,46 @@ __host__ __device__ __forceinline__ double g16_point(const double *x, uint64_t s
     bz[7] = nlo;
     arow[kp / 8 - 1] = az;
     brow[kp / 8 - 1] = bz;
-    return err;
+    return r;
 }
 
+// Sums over the points, each on a line of its own: E, and the shares of tau^2
+// that the guards of a pair of such points take, here and in the split-BF16
+// join (at most 1: then every near pair is in the band).
+enum G16Sum { kSumErr, kSumShare, kSumShareBf, kSums };
+constexpr int kLineDoubles = kLineWords / 2;
+
 // One thread per point (cell order); row n of A and B is the padding row.
-// sum_err += E.
+// bf: the split-BF16 join's guard of two points per unit of N.
 template <int KB>
 __global__ __launch_bounds__(256) void k_g16_prepare(const double *__restrict__ soa, uint32_t n,
                                                      uint32_t dim, const double *__restrict__ mean,
-                                                     double sigma, double tau, double gamma,
+                                                     double sigma, double tau, double gamma, double bf,
                                                      uint16_t *__restrict__ A, uint16_t *__restrict__ B,
-                                                     float *__restrict__ w, double *sum_err) {
+                                                     float *__restrict__ w, double *sums) {
     constexpr int KP = KB * 32;
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
-    double err = 0.0;
-    if (p <= n)
-        err = g16_point(soa + (p < n ? p : 0), n, dim, KP, mean, sigma, tau, gamma, 1.0, p < n,
-                        A + (uint64_t)p * KP, B + (uint64_t)p * KP, w + p);
-    for (int o = 32; o > 0; o >>= 1) err += __shfl_xor(err, o, 64);
-    __shared__ double sh[4];
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = err;
+    double v[kSums] = {};
+    if (p <= n) {
+        const G16Point r = g16_point(soa + (p < n ? p : 0), n, dim, KP, mean, sigma, tau, gamma, 1.0, p < n,
+                                     A + (uint64_t)p * KP, B + (uint64_t)p * KP, w + p);
+        if (p < n) {
+            v[kSumErr] = r.err;
+            v[kSumShare] = fmin(1.0, 2.0 * (double)w[p] / (tau * tau));
+            v[kSumShareBf] = fmin(1.0, bf * r.norm / (tau * tau));
+        }
+    }
+    __shared__ double sh[kSums][4];
+#pragma unroll
+    for (int k = 0; k < kSums; k++) {
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+        if ((threadIdx.x & 63) == 0) sh[k][threadIdx.x >> 6] = v[k];
+    }
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(sum_err, sh[0] + sh[1] + sh[2] + sh[3]);
+    if (threadIdx.x < kSums) {
+        const double *s = sh[threadIdx.x];
+        atomicAdd(sums + threadIdx.x * kLineDoubles, s[0] + s[1] + s[2] + s[3]);
+    }
 }
 
 // ---- work units ------------------------------------------------------------
@@ -593,21 +616,32 @@ static G16Scale g16_scale(double max2, double thresh, double eps, uint32_t dim) 
 }
 
 // Operands for one index and its threshold; ops->A stays null when FP16
-// cannot serve the data (a norm overflows FP64, or the mean rounding
-// error exceeds 1/16 of eps: a far outlier then sets the scale, the band would
-// hold a large share of the near pairs and the split BF16, whose exponent
-// range is FP32's, is the better filter).
+// cannot serve the data: a norm overflows FP64, or the band would hold a large
+// share of the near pairs and the split BF16, whose exponent range is FP32's,
+// is the better filter.  A far outlier does that: it sets the scale, and what is
+// below 2^-14 of it (coordinates, and the norms' low parts) is lost.
+// `share`, the part of tau^2 that a pair's guards take, decides; total join
+// time FP16 / split BF16 with two opposite outliers, by share:
+//     18-D 250k  .029 3.7 / 19.2 ms   .106 4.1 / 19.0   .41 576 / 19
+//     18-D 1M    .037 25.6 / 160      .134 61 / 160     .50 5309 / 160
+//     32-D 200k  .029 145 / 318       .107 416 / 317    .42 2673 / 320
+//     64-D 100k  .040 2.2 / 11.9      .154 35 / 11.7    .52 1555 / 11.9
+//     90-D 100k  .027 1.6 / 10.3      .103 2.4 / 10.5   .40 852 / 10.4
+//     124-D 60k  .020 0.8 / 4.5       .073 0.9 / 4.5    .28 16.6 / 4.5
+// Clusters far from their mean widen the split BF16's guards no less, and FP16
+// stays ahead (18-D 200k, 50 centres 100 eps out: shares .64 and 1, 1.6 / 793
+// ms), until its mean error exceeds 1/16 of eps.
 hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mean, GbOperands *ops,
                         hipStream_t s) {
     const uint32_t n = g.n, dim = g.dim, kb = g16_kblocks(dim);
     if (kb == 0) return HEGJ_OK;
     Scratch sc;
     unsigned long long *d_bits;
-    double *d_err;
+    double *d_sums;
     HIP_TRY(sc.get(&d_bits, 1));
-    HIP_TRY(sc.get(&d_err, 1));
+    HIP_TRY(sc.get(&d_sums, kSums * kLineDoubles));
     HIP_TRY(hipMemsetAsync(d_bits, 0, sizeof(*d_bits), s));
-    HIP_TRY(hipMemsetAsync(d_err, 0, sizeof(*d_err), s));
+    HIP_TRY(hipMemsetAsync(d_sums, 0, sizeof(double) * kSums * kLineDoubles, s));
     k_g16_maxnorm<<<std::min<uint32_t>(ceil_div(n, 256), 2048), 256, 0, s>>>(ix.soa, n, dim, mean, d_bits);
     HIP_TRY(hipGetLastError());
     unsigned long long bits = 0;
@@ -626,16 +660,21 @@ hegj_status g16_prepare(const GridGeom &g, const DevIndex &ix, const double *mea
     HIP_TRY(hold.get(&w, rows));
     const uint32_t blocks = ceil_div(rows, 256);
     const double gamma = g16_gamma(kb);
+    // twice 4 delta (hegj_mfma.hip); without such a kernel its share is 1
+    const uint32_t kbf = gb_kblocks(dim);
+    const double bf = kbf ? 8.0 * gb_coefficient(dim, kbf * 32) : INFINITY;
     switch (kb) {
-        case 1: k_g16_prepare<1><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, A, B, w, d_err); break;
-        case 2: k_g16_prepare<2><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, A, B, w, d_err); break;
-        case 3: k_g16_prepare<3><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, A, B, w, d_err); break;
-        default: k_g16_prepare<4><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, A, B, w, d_err); break;
+        case 1: k_g16_prepare<1><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, bf, A, B, w, d_sums); break;
+        case 2: k_g16_prepare<2><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, bf, A, B, w, d_sums); break;
+        case 3: k_g16_prepare<3><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, bf, A, B, w, d_sums); break;
+        default: k_g16_prepare<4><<<blocks, 256, 0, s>>>(ix.soa, n, dim, mean, sigma, tau, gamma, bf, A, B, w, d_sums); break;
     }
     HIP_TRY(hipGetLastError());
-    double err = 0;
-    HEGJ_TRY(read_back(&err, d_err, s));
-    if (!(err / n <= tau / 16.0)) return HEGJ_OK;
+    double sums[kSums * kLineDoubles];
+    HEGJ_TRY(read_back(sums, d_sums, s, kSums * kLineDoubles));
+    const double err = sums[kSumErr * kLineDoubles] / n, share = sums[kSumShare * kLineDoubles] / n,
+                 share_bf = sums[kSumShareBf * kLineDoubles] / n;
+    if (!(err <= tau / 16.0) || !(share <= 1.0 / 16 || share <= share_bf)) return HEGJ_OK;
     ops->A = A;
     ops->B = B;
     ops->w = w;

@@ -94,3 +94,26 @@ def test_split_bf16_band_list_overflow(H, oracle):
     pts[3, -4:] = 1e10
     info = join(H, oracle, pts, 0.02, "bf16")
     assert info["band_rechecks"] > 1 << 22
+
+
+@pytest.mark.parametrize("dim", [16, 18, 32, 64, 90, 124])
+@pytest.mark.parametrize("far, operands", [(100, "f16"), (800, "f16"), (6400, "bf16"), (100000, "bf16")])
+def test_outliers_choose_the_operands(H, oracle, dim, far, operands):
+    """Outliers `far` eps out set the FP16 scale.  At 6400 the norms' low parts
+    are below FP16's normal range by more than eps^2 can bear: FP16 tiles would
+    send most near pairs to the FP64 recheck."""
+    pts, eps = cloud(np.random.default_rng(dim), 900, dim, 0)
+    pts[7, -2:], pts[8, -2:] = far * eps, -far * eps
+    info = join(H, oracle, pts, eps, operands)
+    assert info["band_rechecks"] < info["total_neighbors"] / 2
+
+
+def test_clusters_keep_fp16(H, oracle):
+    """Centres 60 eps from the mean: wide guards in both, FP16 the faster."""
+    rng = np.random.default_rng(2)
+    pts, eps = cloud(rng, 1500, 18, 0)
+    centre = rng.standard_normal((12, 18))
+    centre[:, :6] = 0
+    centre *= 60 * eps / np.linalg.norm(centre, axis=1, keepdims=True)
+    pts += centre[rng.integers(0, 12, len(pts))]
+    join(H, oracle, pts, eps, "f16")
