@@ -122,7 +122,7 @@ def cpu_baseline(pts, eps, dim, seconds_budget=20.0):
             "sample": f"Super-EGO restatement, {len(qids)} queries"}
 
 
-def rooflines(n, dim, cells, pairs, evals, kernel_ms, refine):
+def rooflines(n, dim, cells, pairs, evals, kernel_ms, refine, operands="bf16"):
     """The dominant join kernel against its two roofs, per launch.
 
     Algorithmic work (per unit, times the units one launch processes):
@@ -133,10 +133,10 @@ def rooflines(n, dim, cells, pairs, evals, kernel_ms, refine):
                     (subtract + fma per dim; E is the reference's candidate
                     count less the candidates cell-box pruning leaves out)
       MFMA flops  = 2 D per candidate pair evaluated (the FP16 tiles evaluate
-                    an unordered pair once), against the bf16 peak divided by
-                    the 3 products of a split-BF16 dot (hi.hi + hi.lo + lo.hi);
-                    the FP16 tiles spend one product per dimension, so their
-                    own roof is three times as high
+                    an unordered pair once), against the dense 16-bit peak:
+                    whole for operands "f16", one product per dimension, a
+                    third of it for "bf16", whose split dots take three
+                    (hi.hi + hi.lo + lo.hi)
     Returns (binding, other): the binding roof is the one whose roof time is
     longer (the roof the kernel would hit first)."""
     t = kernel_ms * 1e-3
@@ -147,10 +147,14 @@ def rooflines(n, dim, cells, pairs, evals, kernel_ms, refine):
            "note": "8nD + 4n + 24C + 8P bytes per launch"}
     if refine == "mfma":
         flops = 2.0 * dim * evals
-        peak = PEAK_BF16_TFLOPS / 3.0
-        note = ("2 D flops per candidate pair evaluated; peak = bf16 dense MFMA / 3 (split-BF16 "
-                "hi.hi + hi.lo + lo.hi); kernel k_g16_join spends one fp16 product per dimension, "
-                "its own roof is 3 times this peak")
+        if operands == "bf16":
+            peak = PEAK_BF16_TFLOPS / 3.0
+            note = ("2 D flops per candidate pair evaluated; peak = bf16 dense MFMA / 3 (split-BF16 "
+                    "hi.hi + hi.lo + lo.hi); kernel k_gb_join")
+        else:
+            peak = PEAK_BF16_TFLOPS  # fp16 and bf16 alike
+            note = ("2 D flops per candidate pair evaluated, an unordered pair once; peak = fp16 dense "
+                    "MFMA, one product per dimension; kernel k_g16_join (K = D + 4 in blocks of 32)")
         bound = "mfma"
     elif refine == "f32":
         flops = 3.0 * dim * evals
@@ -375,7 +379,7 @@ def main():
     # pruning leaves out candidates the reference evaluates)
     evals_launch = sum(i["evals_executed"] for i in infos) / launches
     roof, roof_alt = rooflines(n, dim, iinfo["nNonEmptyCells"], pairs, evals_launch,
-                               kernel_ms, refine_used)
+                               kernel_ms, refine_used, infos[-1]["mfma_operands"])
     roof_alt["attainable_copy_gbs"] = copy_gbs
     attach_traffic(roof, a.config, refine_used, kernel_ms)
     out = {
@@ -385,8 +389,10 @@ def main():
         "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": ms_step,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": {"mfma": "f16 (f32 acc) + f64 band recheck",
-                  "f32": "f32 filter + f64 band recheck"}.get(refine_used, "f64"), "data": "synthetic (reference exponential generator, seed 0)",
+        "dtype": {"mfma": ("bf16 hi/lo" if infos[-1]["mfma_operands"] == "bf16" else "f16") +
+                          " (f32 acc) + f64 band recheck",
+                  "f32": "f32 filter + f64 band recheck"}.get(refine_used, "f64"),
+        "data": "synthetic (reference exponential generator, seed 0)",
         "config": {"workload": cfg["name"], "n": n, "dim": dim, "indexed_dims": k,
                    "eps": eps, "pairs": pairs, "total_candidates": total_cand,
                    "cells": iinfo["nNonEmptyCells"], "cell0_silenced": iinfo["n_cell0_queries"],
