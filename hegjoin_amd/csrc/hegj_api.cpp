@@ -1372,6 +1372,7 @@ hegj_status capture_graph(hegj_index *h, GraphPlan &G) {
     JoinArgs proto{};
     proto.g = h->g;  // with f32: selects the kernel instantiation
     proto.f32 = G.P.f32 ? 1u : 0u;
+    proto.block_waves = G.P.waves;  // the blocks and the mask scratch are sized for it
     hipGraph_t graph = nullptr;
     HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     hegj_status st = HEGJ_OK;
