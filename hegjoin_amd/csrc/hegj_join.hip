@@ -235,70 +235,86 @@ __device__ __forceinline__ void dist_regs_lds(const double *x, const double *qs,
     }
 }
 
+constexpr int kRegDims = 32;  // dims kept in registers (with prefetch)
+constexpr int kQGroup = 4;    // coordinates of a query read from LDS at a time
+
 // Generic dimension count (runtime or large D): candidate coordinates are
-// streamed in tiles of 16 dims, acc keeps the dimension order.  The unit's
-// query coordinates come from LDS (qs[qi * dim + l]).
+// streamed in tiles of DT dims, acc keeps the dimension order.  The unit's
+// query coordinates come from LDS (qs[qi * stride + l]), padded with zeros to
+// whole groups of 4 like the candidate's: a pad adds fma(0, 0, acc) = acc.
+// So there is a branch per group and not per coordinate, and none per query:
+// the unit's queries are rounded up to QB, QB / 2 or QB / 4.  With a branch per
+// coordinate each LDS read was waited for by itself and the kernel's time moved
+// by a fifth with the compiler's layout of the blocks (the same instructions,
+// 22% more wave cycles).  Kernel at 40k uniform points: 8-D 2.25 -> 1.42 ms,
+// 12-D 9.6 -> 4.1, 15-D 11.3 -> 4.8 (7.2 in the better of the layouts).
+// Bound by the FP64 rate (8 queries of 15-D: 240 instructions a chunk) and, at
+// three waves a SIMD, by the latency of the 16 loads at a chunk's start.
 // FLT: DTYPE=float (params.h:24).  The coordinates are floats held in
 // doubles; the chain is the reference's FP32 one, d = fl32(c - q),
 // acc = fmaf(d, d, acc), returned widened to double (exact).
-template <int D, int QB, bool FLT = false>
-__device__ __forceinline__ void dist_stream(const JoinArgs &a, uint32_t pos, bool valid,
-                                            const double *qs, uint32_t nq, double *acc) {
+template <int D, int QL, int DT, bool FLT>
+__device__ __forceinline__ void dist_stream_ql(const JoinArgs &a, uint32_t pos, const double *qs, uint32_t stride,
+                                               double *acc) {
+    typedef typename std::conditional<FLT, float, double>::type FT;
+    typedef double d2 __attribute__((ext_vector_type(2)));
     const uint32_t dim = D > 0 ? (uint32_t)D : a.g.dim;
     const uint64_t n = a.g.n;
-    const double *__restrict__ soa = a.ix.soa;
-    constexpr int DT = 16;
-    if constexpr (FLT) {
-        float accf[QB];
+    const double *__restrict__ src = a.ix.soa + pos;
+    FT sum[QL];
 #pragma unroll
-        for (int qi = 0; qi < QB; qi++) accf[qi] = 0.0f;
-        for (uint32_t d0 = 0; d0 < dim; d0 += DT) {
-            float x[DT];
+    for (int qi = 0; qi < QL; qi++) sum[qi] = (FT)0;
+#pragma unroll 1
+    for (uint32_t d0 = 0; d0 < dim; d0 += DT) {
+        FT x[DT];  // coordinates of the candidate in flight
 #pragma unroll
-            for (int i = 0; i < DT; i++) {
-                uint32_t l = d0 + i;
-                x[i] = (valid && l < dim) ? (float)soa[(uint64_t)l * n + pos] : 0.0f;
-            }
+        for (int g = 0; g < DT; g += kQGroup) {
+            if (g && d0 + g >= dim) break;
 #pragma unroll
-            for (int qi = 0; qi < QB; qi++) {
-                if ((uint32_t)qi < nq) {
-#pragma unroll
-                    for (int i = 0; i < DT; i++) {
-                        uint32_t l = d0 + i;
-                        if (l < dim) {
-                            const float dd = x[i] - (float)qs[qi * dim + l];
-                            accf[qi] = __builtin_fmaf(dd, dd, accf[qi]);
-                        }
-                    }
-                }
+            for (int i = g; i < g + kQGroup; i++) {
+                const uint32_t l = d0 + i;
+                const FT v = (FT)src[(uint64_t)min(l, dim - 1) * n];
+                x[i] = l < dim ? v : (FT)0;
             }
         }
 #pragma unroll
-        for (int qi = 0; qi < QB; qi++) acc[qi] = (double)accf[qi];
-        return;
+        for (int g = 0; g < DT; g += kQGroup) {
+            if (g && d0 + g >= dim) break;
+#pragma unroll
+            for (int qi = 0; qi < QL; qi++) {
+                const d2 *q2 = reinterpret_cast<const d2 *>(qs + qi * stride + d0 + g);
+                const d2 q0 = q2[0], q1 = q2[1];
+                const FT q[kQGroup] = {(FT)q0.x, (FT)q0.y, (FT)q1.x, (FT)q1.y};
+#pragma unroll
+                for (int i = 0; i < kQGroup; i++) {
+                    const FT d = x[g + i] - q[i];
+                    if constexpr (FLT)
+                        sum[qi] = __builtin_fmaf(d, d, sum[qi]);
+                    else
+                        sum[qi] = __builtin_fma(d, d, sum[qi]);
+                }
+            }
+        }
     }
 #pragma unroll
-    for (int qi = 0; qi < QB; qi++) acc[qi] = 0.0;
-    for (uint32_t d0 = 0; d0 < dim; d0 += DT) {
-        double x[DT];
+    for (int qi = 0; qi < QL; qi++) acc[qi] = (double)sum[qi];
+}
+
+template <int D, int QB, bool FLT = false>
+__device__ __forceinline__ void dist_stream(const JoinArgs &a, uint32_t pos, const double *qs, uint32_t stride,
+                                            uint32_t nq, double *acc) {
 #pragma unroll
-        for (int i = 0; i < DT; i++) {
-            uint32_t l = d0 + i;
-            x[i] = (valid && l < dim) ? soa[(uint64_t)l * n + pos] : 0.0;
-        }
-#pragma unroll
-        for (int qi = 0; qi < QB; qi++) {
-            if ((uint32_t)qi < nq) {
-#pragma unroll
-                for (int i = 0; i < DT; i++) {
-                    uint32_t l = d0 + i;
-                    if (l < dim) {
-                        double dd = x[i] - qs[qi * dim + l];
-                        acc[qi] = __builtin_fma(dd, dd, acc[qi]);
-                    }
-                }
-            }
-        }
+    for (int qi = 0; qi < QB; qi++) acc[qi] = 0.0;  // (unused where nq leaves queries out)
+    constexpr int DT = QB <= 4 ? 8 : 16;  // (16 spill in the 128 registers of the QB 4 instances)
+    if constexpr (QB >= 4) {
+        if (nq <= (uint32_t)QB / 4)
+            dist_stream_ql<D, QB / 4, DT, FLT>(a, pos, qs, stride, acc);
+        else if (nq <= (uint32_t)QB / 2)
+            dist_stream_ql<D, QB / 2, DT, FLT>(a, pos, qs, stride, acc);
+        else
+            dist_stream_ql<D, QB, DT, FLT>(a, pos, qs, stride, acc);
+    } else {
+        dist_stream_ql<D, QB, DT, FLT>(a, pos, qs, stride, acc);
     }
 }
 
@@ -311,9 +327,16 @@ constexpr bool q_in_sgprs() {
     return D > 0 && D <= 32 && QB * D <= 24;
 }
 
+// Doubles from one query's coordinates to the next in LDS: those of the
+// streaming instances are padded with zeros to whole groups.
+template <int D>
+__host__ __device__ constexpr uint32_t q_stride(uint32_t dim) {
+    return D > 0 && D <= kRegDims ? dim : (dim + kQGroup - 1) / kQGroup * kQGroup;
+}
+
 template <int D, int QB>
 constexpr uint32_t q_lds_bytes(uint32_t dim) {
-    return q_in_sgprs<D, QB>() ? 0u : (uint32_t)(kWavesPerBlockQ * QB * (D > 0 ? D : dim) * sizeof(double));
+    return q_in_sgprs<D, QB>() ? 0u : (uint32_t)(kWavesPerBlockQ * QB * q_stride<D>(D > 0 ? D : dim) * sizeof(double));
 }
 
 // Hit masks of one unit: mask[ch * nq + qi], one 64-bit ballot per
@@ -325,7 +348,6 @@ struct HitStore {
     uint64_t w[kMaskSlots];
 };
 
-constexpr int kRegDims = 32;  // dims kept in registers (with prefetch)
 
 // The kernel arguments, to be read again from here on.  They are ~100 scalar
 // registers' worth; kept live through a unit's loops they were spilled to
@@ -483,7 +505,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
     static_assert(!FLT || D == 0, "DTYPE=float: generic instance only");
     __shared__ RowList rls[kWavesPerBlock];
     __shared__ HitStore hs_all[kWavesPerBlock];
-    extern __shared__ double q_dyn[];  // QB * dim query coordinates per wave
+    extern __shared__ __attribute__((aligned(16))) double q_dyn[];  // the query coordinates of each wave
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     RowList &rl = rls[wid];
     uint64_t *const hs_lds = hs_all[wid].w;
@@ -494,7 +516,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
     constexpr int DR = kRegs ? D : 1;
     uint64_t my_evals = 0, my_pairs = 0;
     constexpr bool kQS = q_in_sgprs<D, QB>();
-    const uint32_t dimq = D > 0 ? (uint32_t)D : a0.g.dim;
+    const uint32_t dimq = q_stride<D>(D > 0 ? (uint32_t)D : a0.g.dim);
     double *const qs = q_dyn + (size_t)wid * QB * dimq;
     double qreg[kQS ? QB : 1][kQS ? DR : 1];
     __shared__ unsigned long long sh_stats[3];
@@ -545,7 +567,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
             } else {
                 for (uint32_t i = lane; i < QB * dimq; i += 64) {
                     const uint32_t qi = i / dimq, l = i - qi * dimq;
-                    qs[i] = qi < nq ? a.ix.soa[(uint64_t)l * a.g.n + qpos0 + qi] : 0.0;
+                    qs[i] = qi < nq && l < (D > 0 ? (uint32_t)D : a.g.dim) ? a.ix.soa[(uint64_t)l * a.g.n + qpos0 + qi] : 0.0;
                 }
             }
             wave_lds_sync();
@@ -634,7 +656,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
                                 const uint32_t pos = valid ? cur.pos(rl, t) : 0u;
                                 uint32_t qoff = (uint32_t)wid * QB * dimq;
                                 __asm__ volatile("" : "+v"(qoff));
-                                dist_stream<D, QB, FLT>(a, pos, valid, q_dyn + qoff, nq, acc);
+                                dist_stream<D, QB, FLT>(a, pos, q_dyn + qoff, dimq, nq, acc);
                             }
 #pragma unroll
                             for (int qi = 0; qi < QL; qi++)
@@ -774,7 +796,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, (join_min_waves<D, QB>())) voi
                                 acc1 = __builtin_fma(dd, dd, acc1);
                             }
                         } else {
-                            dist_stream<D, 1, FLT>(a, pos, valid, qs + qi * dimq, 1, &acc1);
+                            dist_stream<D, 1, FLT>(a, pos, qs + qi * dimq, dimq, 1, &acc1);
                         }
                         const uint64_t m = __ballot(valid && acc1 <= T);
                         if (m == 0) continue;
