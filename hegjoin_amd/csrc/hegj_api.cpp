@@ -828,6 +828,17 @@ hegj_status cap_to_free(uint64_t *capacity) {
     return HEGJ_OK;
 }
 
+// Fewer than four units per wave of at least 7 coordinates a distance: long
+// and much alike, so a run of two makes its wave the last one, and there is no
+// other gain to set against that.  Kernel with runs and with single units:
+// 7-D 40k (2.7 units a wave) 1.88 and 1.70 ms, 9-D 60k (2.8) 4.62 and 3.94, 10-D
+// 40k (1.8) 3.01 and 2.38, 15-D 40k (1.7) 4.64 and 3.38; from four on they are
+// level (12-D 100k, 4.1: 76.0 and 76.3).  Shorter ones gain by runs however few
+// they are: 2-D 20k (0.7) 0.102 and 0.123, 6-D 20k (2.4) 0.203 and 0.250.
+bool few_long_units(const hegj_index *h, const JoinPlan &P) {
+    return h->g.dim >= 7 && P.U < 4ull * P.max_blocks * P.waves;
+}
+
 // The queue of the plan's units: ranges per XCD, split by estimated work, of
 // single units or, without units_per_grab, of runs.  (The hybrid modes, whose
 // list covers all cells, launch pieces of it: grabs, sized for each.)
@@ -839,7 +850,7 @@ hegj_status make_queue(hegj_index *h, const hegj_join_opts &opts, uint32_t qb, J
     const uint32_t U = P.U;
     P.parts = opts.xcd_parts ? std::min<uint32_t>(opts.xcd_parts, kMaxParts) : kMaxParts;
     if (U < P.parts * 256) P.parts = 1;
-    if (opts.units_per_grab || all_cells || U == 0)
+    if (opts.units_per_grab || all_cells || U == 0 || few_long_units(h, P))
         return split_units(h->ix, P.units, U, qb, h->d_work, P.parts, P.part_end, s);
     P.n_runs = (uint32_t)std::min<uint64_t>(U, (uint64_t)P.max_blocks * P.waves * kRunsPerWave);
     HIP_TRY(dev_malloc_n(&P.runs, (size_t)P.n_runs + 1));

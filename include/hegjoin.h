@@ -221,8 +221,9 @@ typedef struct {
     uint32_t refine;          /* hegj_refine */
     uint32_t xcd_parts;       /* unit ranges, one per XCD: 0 = auto (8), 1 = one queue */
     uint32_t units_per_grab;  /* units a wave takes at a time; 0 = runs of units of
-                                 equal estimated work (hybrid modes: by the number
-                                 of units of each launch) */
+                                 equal estimated work, or one where few units of 7
+                                 or more dims each keep a wave long (hybrid modes:
+                                 by the number of units of each launch) */
     uint32_t part_by_block;   /* 0: range by hardware XCD id, 1: by workgroup index */
     uint32_t use_graph;       /* FP64 refine: keep the plan in the index and run the
                                  batch as a replay of a captured hipGraph */
