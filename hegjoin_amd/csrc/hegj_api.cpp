@@ -1990,7 +1990,7 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
     P.tacc32 = tacc;
     P.trej32 = trej;
     auto too_small = [&](hegj_status st) {
-        if (st != HEGJ_OK && arena.used + (1u << 20) >= arena.cap)
+        if (st == HEGJ_ERR_OUT_OF_MEMORY)  // (nothing else is allocated here)
             return fail(HEGJ_ERR_CAPACITY, "hegj_selfjoin_noalloc: this index needs more than the " +
                                                std::to_string(kNoAllocScratchBytes >> 20) +
                                                " MiB of fixed scratch (n = " + std::to_string(n) +

@@ -317,8 +317,8 @@ hegj_status hegj_result_get_info(const hegj_result *res, hegj_result_info *info)
  * neighbors[capacity] (rows back to back), row_off[n] (offset of each point's
  * row in neighbors) and row_cnt[n] (its length), by original point id -- and
  * every temporary comes from a fixed 64 MiB device array per GPU (about
- * 12 bytes per work unit plus 8 per non-empty cell: enough for the 5M-point
- * 6-D workload).  An index that needs more fails with HEGJ_ERR_CAPACITY; so
+ * 20 bytes per work unit plus 8 per non-empty cell: enough for the 5M-point
+ * 6-D workload; with units_per_grab given 28 per unit).  An index that needs more fails with HEGJ_ERR_CAPACITY; so
  * does a result larger than `capacity`, with info->total_neighbors set to
  * the count needed.  The index's lazily built arrays are inputs: run
  * hegj_selfjoin once with the same options first (HEGJ_ERR_INVALID_ARG

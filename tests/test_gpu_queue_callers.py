@@ -45,3 +45,19 @@ def test_hybrid_pieces(H, oracle, piece):
         t.close()
     assert info["n_units"] > 16384
     assert (info["total_neighbors"], info["pair_hash"]) == (total, want)
+
+
+def test_noalloc_beyond_its_scratch(H):
+    """3M cells of a point each: units and their weights need more than the
+    fixed scratch, which is a matter of capacity."""
+    rt = runtime()
+    n = 3_000_000
+    pts = np.random.default_rng(5).permutation(n).astype(np.float64)[:, None] / n
+    nb, off, cnt = bufs = [Buf(rt, t, n) for t in (np.uint32, np.uint64, np.uint32)]
+    with H.GridIndex(pts, 0.4 / n) as ix:
+        ix.selfjoin().close()
+        with pytest.raises(H.HegjError) as e:
+            ix.selfjoin_noalloc(nb.p, n, off.p, cnt.p)
+        assert e.value.status == 6 and "scratch" in str(e.value)
+    for b in bufs:
+        b.free()
