@@ -805,12 +805,14 @@ constexpr uint64_t kBoundCandidates = 1ull << 27;
 
 // A result keeps its batch until it is freed, so one sized by the candidates
 // (60k 6-D points at 64 neighbours: half a GiB for 16 MB of rows) is changed for
-// one of the size that its rows took, where that saves 16 MiB and half of it:
-// a copy of the rows at the device's copy rate (16 MB: 8 us).  The old one
-// is given back when the call ends; without memory for the copy it stays.
+// one of the size that its rows took, where that is under a quarter of it and
+// 16 MiB are saved: a copy of the rows at the device's copy rate (16 MB: 8 us).
+// (2-D rows are a third of the candidates: copying 65 MB of them took 27 of 292
+// us, so these stay.)  The old one is given back when the call ends; without
+// memory for the copy it stays.
 hegj_status fit_batch(hegj_result *r, uint64_t capacity, uint64_t used, hipStream_t s) {
     used = std::min(used, capacity);  // (the last chunk reserved may reach past the end)
-    if (capacity < 2 * used + (4u << 20)) return HEGJ_OK;
+    if (capacity < 4 * used + (4u << 20)) return HEGJ_OK;
     uint32_t *fit = nullptr;
     const uint64_t n16 = (used + 3) / 4;
     if (dev_malloc_n(&fit, std::max<uint64_t>(n16 * 4, 4)) != hipSuccess) return HEGJ_OK;
