@@ -792,7 +792,9 @@ JoinArgs base_args(const hegj_index *h, const hegj_join_opts &opts, const JoinPl
 // Waves reserve output in chunks of 16 average units (less when the waves'
 // last chunks would exceed an eighth of the result of about `est` pairs).  Up
 // to a quarter of a chunk stays unused when the next one is taken, and each
-// wave's last one: room for both is added to the capacity.
+// wave's last one: room for the latter and for 15% of the pairs is added to the
+// capacity (units far smaller than a chunk leave a few per cent; where more is
+// left, the last units are deferred).
 void set_chunk(JoinPlan &P, double est) {
     const double avg = est / P.U, waves = (double)P.max_blocks * P.waves;
     const double chunk = std::min(16.0 * avg + 64.0, (est / 8 + (1 << 20)) / waves);

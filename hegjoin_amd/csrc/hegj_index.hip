@@ -46,8 +46,6 @@ __global__ __launch_bounds__(kT) void k_minmax(const double *__restrict__ pts, u
     }
 }
 
-// S2 + S3 (kernel.cu:54-60): FP64 subtract, IEEE FP64 divide, truncation to
-// unsigned, linear id with dim 0 fastest.  Also the identity permutation.
 // Indexed coordinates of each non-empty cell, one plane per dim.
 __global__ __launch_bounds__(kT) void k_cell_xyz(const uint64_t *__restrict__ cell_key, uint32_t C, GridGeom g,
                                                  uint32_t *__restrict__ xyz) {
@@ -58,6 +56,8 @@ __global__ __launch_bounds__(kT) void k_cell_xyz(const uint64_t *__restrict__ ce
     for (uint32_t j = 0; j < g.k; j++) xyz[(uint64_t)j * C + i] = c[j];
 }
 
+// S2 + S3 (kernel.cu:54-60): FP64 subtract, IEEE FP64 divide, truncation to
+// unsigned, linear id with dim 0 fastest.  Also the identity permutation.
 __global__ __launch_bounds__(kT) void k_cell_ids(const double *__restrict__ pts, GridGeom g,
                                                  uint64_t *__restrict__ keys,
                                                  uint64_t *__restrict__ point_key,

@@ -248,8 +248,9 @@ constexpr int kQGroup = 4;    // coordinates of a query read from LDS at a time
 // by a fifth with the compiler's layout of the blocks (the same instructions,
 // 22% more wave cycles).  Kernel at 40k uniform points: 8-D 2.25 -> 1.42 ms,
 // 12-D 9.6 -> 4.1, 15-D 11.3 -> 4.8 (7.2 in the better of the layouts).
-// Bound by the FP64 rate (8 queries of 15-D: 240 instructions a chunk) and, at
-// three waves a SIMD, by the latency of the 16 loads at a chunk's start.
+// What bounds it: the FP64 rate (8 queries of 15-D: 256 of some 390 vector
+// instructions a chunk, 1.3 ms) and, at three waves a SIMD, the latency of the
+// 16 loads at a chunk's start.
 // FLT: DTYPE=float (params.h:24).  The coordinates are floats held in
 // doubles; the chain is the reference's FP32 one, d = fl32(c - q),
 // acc = fmaf(d, d, acc), returned widened to double (exact).
