@@ -1862,6 +1862,7 @@ hegj_status hegj_selfjoin(hegj_index *h, const hegj_join_opts *opts_in, hegj_res
         return fail(HEGJ_ERR_INVALID_ARG, "queries_per_unit must be 4, 8 or 16");
     if (!valid_waves_batches(opts))
         return fail(HEGJ_ERR_INVALID_ARG, "block_waves must be 0, 1, 2 or 4 and batches at most 32");
+    opts.units_per_grab = std::min(opts.units_per_grab, h->g.n);  // (at most n units; larger ones overflow)
     hipStream_t s = h->stream;
     const uint32_t n = h->g.n;
 
@@ -1950,6 +1951,7 @@ hegj_status hegj_selfjoin_noalloc(hegj_index *h, const hegj_join_opts *opts_in, 
     if (qb != 4 && qb != 8 && qb != 16) return fail(HEGJ_ERR_INVALID_ARG, "queries_per_unit must be 4, 8 or 16");
     if (!valid_waves_batches(opts))
         return fail(HEGJ_ERR_INVALID_ARG, "block_waves must be 0, 1, 2 or 4 and batches at most 32");
+    opts.units_per_grab = std::min(opts.units_per_grab, h->g.n);  // (at most n units; larger ones overflow)
     // the index's lazily built arrays are inputs here: they must exist
     const char *prep = "the index must have run hegj_selfjoin once with these options first";
     if (!h->have_workload) return fail(HEGJ_ERR_INVALID_ARG, std::string(prep) + " (workload order)");
@@ -2109,6 +2111,7 @@ hegj_status hegj_selfjoin_hybrid(hegj_index *h, const hegj_join_opts *opts_in,
     if (qb != 4 && qb != 8 && qb != 16) return fail(HEGJ_ERR_INVALID_ARG, "queries_per_unit must be 4, 8 or 16");
     if (!valid_waves_batches(opts))
         return fail(HEGJ_ERR_INVALID_ARG, "block_waves must be 0, 1, 2 or 4 and batches at most 32");
+    opts.units_per_grab = std::min(opts.units_per_grab, h->g.n);  // (at most n units; larger ones overflow)
     CallScope scope(h->stream);
     std::unique_ptr<hegj_result> r(new hegj_result());
     r->idx = h;

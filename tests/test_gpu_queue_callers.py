@@ -61,3 +61,25 @@ def test_noalloc_beyond_its_scratch(H):
         assert e.value.status == 6 and "scratch" in str(e.value)
     for b in bufs:
         b.free()
+
+
+@pytest.mark.parametrize("grab", [20000, 20001, 1 << 30, (1 << 32) - 1])
+def test_grabs_larger_than_the_join(H, oracle, grab):
+    """More units per grab than there are, up to the largest 32-bit number, in
+    every entry point: one grab, all of the result."""
+    rt = runtime()
+    pts = oracle.generate_expo(20000, 6, seed=53)
+    total, want = oracle.join_stats(pts, 6, 0.012)
+    nb, off, cnt = bufs = [Buf(rt, t, m) for m, t in ((total, np.uint32), (20000, np.uint64), (20000, np.uint32))]
+    with H.GridIndex(pts, 0.012) as ix:
+        print("case grab", grab, flush=True)
+        for t in (ix.selfjoin(units_per_grab=grab), ix.selfjoin(units_per_grab=grab, use_graph=True),
+                  ix.selfjoin(units_per_grab=grab, result_capacity=total // 3),
+                  ix.selfjoin_hybrid("static", gpu_fraction=0.99, cpu_threads=2, units_per_grab=grab)):
+            info = t.info
+            t.close()
+            assert (info["total_neighbors"], info["pair_hash"]) == (total, want)
+        info = ix.selfjoin_noalloc(nb.p, total, off.p, cnt.p, units_per_grab=grab)
+        assert (info["total_neighbors"], info["pair_hash"]) == (total, want)
+    for b in bufs:
+        b.free()
